@@ -35,6 +35,7 @@
 // prefill causal mask).
 #include "common.hpp"
 
+#include <float.h>
 #include <math.h>
 
 #include <atomic>
@@ -554,227 +555,308 @@ __global__ __launch_bounds__(64 * kWaves) void attn_f16_d128(
 
 // ----------------------------------------------------------------------------
 // Prefill (q_len > 1), fp16 pools, head_dim 128, G <= 8.  The query vectors of one
-// sequence and KV head (vector v = t * G + g over its q_len new tokens) form 16-vector
-// tiles, one per wavefront, kPfWaves per workgroup.  A workgroup walks the 32-token
-// K/V blocks its last token sees, kPfGroup blocks at a time: every K and V load of a
-// group is issued at once, while the previous group is being multiplied, and lands in
-// LDS (V transposed) in the other of two buffers.  Each block is read once per 128 query
-// vectors instead of once per query row.  Both products run on MFMA 16x16x32 f16:
-//   * S^T = K Q^T: A = 16 token rows of K (lane t + 16g holds K[t][32s + 8g ..]), B =
-//     Q^T (lane q + 16g holds Q[q][32s + 8g ..]); lane q + 16g ends with S[q][4g + r]
-//     of each 16-token tile;
-//   * O^T = V^T P^T: the B operand is P as the lanes already hold it -- lane q + 16g
-//     takes P[q][4g .. 4g+3] of tile 0 and P[q][16 + 4g .. +3] of tile 1 as its 8 k
-//     values -- and V^T's A operand takes the same token order (lane d + 16g: V^T[d] at
-//     tokens 4g .. and 16 + 4g ..), so no lane exchange is needed; lane q + 16g ends with
-//     O[q][16 dt + 4g + r], all of one query, so the softmax rescale and the final 1/l
-//     are per lane (O = P V, the other way round, spread four queries over each lane and
-//     needed four shuffles of the rescale factors per block).
-// Causal mask per query vector (keys at positions <= its token's), applied only to the
-// blocks a wavefront's first query does not see whole; softmax as in the decode kernel
-// (base 2, p rounded to fp16, l summing the rounded p), with the hardware exp2 (the
-// library exp2f's extra range steps only change results below 2^-126, which round to
-// zero in fp16 p and are negligible in the rescale), and the rescale of O skipped when
-// no lane's running max moved.  A wavefront skips the blocks past its last token.  The
-// tiles of a sequence are dispatched last first, so the longest contexts start first.
-// At two blocks per LDS buffer a workgroup holds 70 KiB and 112 VGPRs, so two fit on a
-// CU.  Against one workgroup per CU at four blocks per buffer (140 KiB), the library
-// exp2f, O = P V and V^T written 4 tokens x 16 column chunks per wavefront (4 banks), a
-// 2048-token prompt (32/8 heads) took 135 against 224 us, 4 x 512 tokens 44 against 66.
-// PAIRED: once the one-tile grid fills both workgroup slots of every CU, all of it is
-// resident at once and the longest tiles set the kernel's time (at 2048 tokens tile 63
-// walks 64 blocks, the mean is 32.5).  A workgroup then runs tile tiles - 1 - x and tile
-// x one after the other (tiles + 1 tiles' worth of blocks each, 120 VGPRs): 2048 tokens
-// 121 us, 4096 tokens 308 against 401, 8 x 512 tokens 60 against 80, the same bits.
-// Smaller grids keep one tile per workgroup.  NG: blocks per LDS buffer.  A grid of at
-// most one workgroup per CU takes 4 (143 KiB; 166 VGPRs paired, 129 not), twice the loads
-// in flight: 2048 tokens 110 us, 2 x 1024 61 against 67, 2 x 512 28.1 against 29.2; a
-// larger one would then run in two rounds (4096 tokens 374 against 289), so it keeps 2.
-constexpr int kPfWaves = 8;
-constexpr int kPfGroup = 2;    // blocks per LDS buffer (two buffers: 70 KiB)
-constexpr int kPfKRow = 136;   // K row stride in LDS (halves): 256 B + 16, a tile's rows on distinct banks
-constexpr int kPfVRow = 36;    // V^T row stride (halves): 64 B + 8; V is loaded 32 tokens x 2 column chunks per
-                               // wavefront, so each transposed 2-byte write covers 32 banks
+// sequence and KV head (vector v = t * G + g over its q_len new tokens) form 32-vector
+// tiles, one per wavefront.  A workgroup of VW * CW wavefronts holds VW tiles; its CW
+// groups take turns of NB 32-token blocks of the context, so a stage of NB * CW blocks
+// feeds all of them, and merge (max, sum, O) through LDS at the end.
+//   * Staging: K and V rows go from their pages to LDS by DMA (16 bytes a lane, no
+//     registers), one stage ahead, one barrier per stage.  Each stage has an array of
+//     its own, so the compiler does not make the reads of one wait for the DMA into
+//     another.  16-byte chunk c of a K row r sits in slot c ^ (r % 16), of a V row in slot
+//     c ^ (4 (r % 4) + r / 4 % 4): the reads below then cover all banks evenly.
+//   * S^T = K Q^T on MFMA 32x32x16 f16: lane q + 32h ends with S[q][8j + 4h + e].
+//   * O^T = V^T P^T: the B operand is P as the lanes hold it (8 tokens 8j + 4h ..), and
+//     V^T's A operand takes the same token order by gfx950's transposing LDS read
+//     (ds_read_b64_tr_b16: 16 lanes read 4 token rows of 16 dims and each gets 4 tokens of
+//     one dim), so neither product exchanges lanes and the softmax rescale is per lane.
+// Causal mask per query vector, applied only to blocks a wavefront's first query does not
+// see whole; softmax in base 2 with p rounded to fp16 for P V and l summing the rounded p;
+// the rescale is skipped when no running max moved; a wavefront skips the blocks past its
+// last token.  The longest tiles are dispatched first, so a causal grid of several rounds
+// balances itself.
+//
+// What bounds it: 32 vectors x 32 tokens cost a wavefront 512 matrix cycles, ~450 VALU
+// cycles of softmax and 16 KiB of LDS reads (128 of the CU's LDS cycles), so at 8
+// wavefronts per CU the three pipes are near balance and the time is what they do not
+// overlap.  The earlier kernel (16 vectors per wavefront: twice the LDS bytes per product;
+// V transposed by 2-byte LDS writes) was bound by LDS.  Measured (us, before -> now): 2 x
+// 509 tokens after 3500 (28/4 heads) 178 -> 84, 2048 after 6000 (32/8) 625 -> 271 (870
+// TFLOP/s), a 2048-token prompt 102 -> 57, 8 x 512 tokens 54 -> 41, 10 tokens after 5000
+// (28/4) 209 -> 19.  NB = 2 (one max, one rescale and one barrier per 64 tokens of a
+// wavefront) against 1: 2048 after 6000 280 -> 251.
+constexpr int kPfVec = 32;  // query vectors per wavefront (one 32-wide MFMA tile)
 
-template <bool PAIRED, int NG>
-__global__ __launch_bounds__(64 * kPfWaves) void attn_prefill_f16_d128(
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+// Transposing LDS read: see the kernel's header.
+__device__ __forceinline__ f16x4 lds_read_tr(const uint8_t* p) {
+  typedef __fp16 h4 __attribute__((ext_vector_type(4)));
+  const h4 v = __builtin_amdgcn_ds_read_tr16_b64_v4f16((__attribute__((address_space(3))) h4*)(p));
+  return __builtin_bit_cast(f16x4, v);
+}
+// This wavefront's DMA has landed, then every wavefront's.  The wait is the builtin, not asm: the compiler counts it,
+// and then puts no wait of its own (which would cover the next stage's DMA too) before the reads of the landed stage.
+__device__ __forceinline__ void dma_wait_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0x70);  // vmcnt(0), lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
+
+template <int VW, int CW, int NB>
+__global__ __launch_bounds__(64 * VW * CW, 2) void attn_prefill_f16_d128(
     const f16* __restrict__ q, const f16* __restrict__ kp, const f16* __restrict__ vp,
-    const int32_t* __restrict__ pt, const int32_t* __restrict__ lens, f16* __restrict__ out, int q_len, int Hq,
-    int Hkv, int P, int max_pages, float scale_log2) {
+    const int32_t* __restrict__ pt, const int32_t* __restrict__ lens, f16* __restrict__ out,
+    float* __restrict__ part_o, float* __restrict__ part_ml, int q_len, int Hq, int Hkv, int P, int max_pages, int S,
+    float scale_log2) {
   constexpr int D = 128;
-  static_assert(kBlock == 32 && 64 * kPfWaves == kBlock * (D / 8), "one 16-byte K and V chunk per thread");
-  static_assert(NG == kPfGroup || NG == 2 * kPfGroup, "blocks per LDS buffer");
-  __shared__ __align__(16) f16 sk[2][NG][kBlock * kPfKRow];
-  __shared__ __align__(16) f16 sv[2][NG][D * kPfVRow];
-  const int kvh = blockIdx.y, b = blockIdx.z;
+  constexpr int W = VW * CW;
+  constexpr int kTok = kBlock * NB * CW;   // tokens per stage
+  constexpr int kHalf = kTok * D * 2;      // bytes of K (then V) in a stage
+  constexpr int kRows = kTok / W; // rows of K and of V a wavefront brings in (within one page: kRows | 16)
+  static_assert(kRows == 8 || kRows == 16, "a wavefront's rows lie in one page");
+  __shared__ __align__(16) uint8_t st0[2 * kHalf];
+  __shared__ __align__(16) uint8_t st1[2 * kHalf];
+  __shared__ float sm_ml[CW > 1 ? CW : 1][VW][2][64];
+  const int kvh = blockIdx.x % Hkv, b = blockIdx.x / Hkv;
+  const int tile = gridDim.y - 1 - blockIdx.y;  // the longest contexts first
+  const int split = blockIdx.z;
   const int G = Hq / Hkv;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
-  const int li = lane & 15, lg = lane >> 4;
+  const int vw = wave % VW, cw = wave / VW;
+  const int l32 = lane & 31, h = lane >> 5;
   const int nvec = q_len * G;
-  const int max_ctx = max_pages * P;
   const int L = lens[b];
-  const int Lc = min(L, max_ctx);  // keys the page table can address
-  const int past = L - q_len;      // context before the new tokens
+  const int Lc = min(L, max_pages * P);  // keys the page table can address
+  const int past = L - q_len;            // context before the new tokens
   const int32_t* ptrow = pt + (size_t)b * max_pages;
   // Last key position query vector v sees (negative: none, its output is zero).
   auto pos_of = [&](int v) __attribute__((always_inline)) { return min(past + v / G, Lc - 1); };
-  const int tiles = (nvec + 16 * kPfWaves - 1) / (16 * kPfWaves);
-  // Unpaired: one tile per workgroup, the last (longest) tiles first.  Paired: tile tiles - 1 - x, then tile x
-  // (once when they coincide), so every workgroup walks tiles + 1 tiles' worth of blocks under the causal mask.
-  for (int pass = 0; pass < (PAIRED ? 2 : 1); ++pass) {
-    const int tile = !PAIRED ? (int)(gridDim.x - 1 - blockIdx.x)
-                             : (pass == 0 ? tiles - 1 - (int)blockIdx.x : (int)blockIdx.x);
-    if (PAIRED && pass == 1) {
-      if (tile == tiles - 1 - (int)blockIdx.x) break;
-      __syncthreads();  // the first tile's LDS reads are done before the second's first stash
+  const int tv0 = tile * kPfVec * VW;                   // the workgroup's first vector
+  const int tv1 = min(nvec, tv0 + kPfVec * VW) - 1;     // and its last
+  const int nblk = pos_of(tv1) >= 0 ? pos_of(tv1) / kBlock + 1 : 0;  // blocks the last token sees
+  const int nst = (nblk + NB * CW - 1) / (NB * CW), per = (nst + S - 1) / S;
+  const int s0 = min(nst, split * per), s1 = min(nst, s0 + per);     // this split's stages
+  const int v0 = tv0 + kPfVec * vw;                     // this wavefront's first vector
+  const int wlast = min(nvec - 1, v0 + kPfVec - 1);
+  const int wblk = (v0 < nvec && pos_of(wlast) >= 0) ? pos_of(wlast) / kBlock + 1 : 0;  // uniform
+
+  // DMA of stage st: this wavefront's rows kRows * wave .. of the stage, 4 rows per instruction (lane / 16 = row,
+  // lane % 16 = LDS slot).  Rows past the context re-read its last token (masked; p = 0 meets finite values).
+  const int drow = kRows * wave + (lane >> 4), dslot = lane & 15;
+  int page = 0, prow = 0;  // the page of its rows of the stage to issue next, and the page's first position
+  auto fetch_page = [&](int st) __attribute__((always_inline)) {
+    const int i = min(st * kTok + kRows * wave, Lc - 1) / P;
+    page = ptrow[i];
+    prow = i * P;
+  };
+  auto issue = [&](uint8_t* buf, int st) __attribute__((always_inline)) {
+    const size_t base = ((size_t)page * Hkv + kvh) * P * D;
+    const rsrc_t rk = make_rsrc(kp + base, (uint32_t)P * 2 * D), rv = make_rsrc(vp + base, (uint32_t)P * 2 * D);
+    const int row0 = st * kTok - prow, last = Lc - 1 - prow;
+#pragma unroll
+    for (int u = 0; u < kRows / 4; ++u) {
+      const int r = drow + 4 * u;
+      const uint32_t at = (uint32_t)min(row0 + r, last) * 2 * D;
+      buf16_to_lds(rk, buf + (kRows * wave + 4 * u) * 2 * D, at + 16 * (dslot ^ (r & 15)), 0);
+      buf16_to_lds(rv, buf + kHalf + (kRows * wave + 4 * u) * 2 * D,
+                   at + 16 * (dslot ^ (((r & 3) << 2) | ((r >> 2) & 3))), 0);
     }
-    const int tv0 = tile * 16 * kPfWaves;                     // the workgroup's first vector
-    const int tv1 = min(nvec, tv0 + 16 * kPfWaves) - 1;       // and its last
-    const int nblk = pos_of(tv1) >= 0 ? pos_of(tv1) / kBlock + 1 : 0;  // blocks the last token sees
-    const int v0 = tv0 + 16 * wave;                           // this wavefront's first vector
-    const int wlast = min(nvec - 1, v0 + 15);
-    const int wblk = (v0 < nvec && pos_of(wlast) >= 0) ? pos_of(wlast) / kBlock + 1 : 0;  // uniform
+  };
 
-    // Thread t loads 16 bytes of K and of V per block: K at token t / 16, dims 8 * (t % 16); V at token t % 32,
-    // dims 8 * (t / 32).
-    const int lt = threadIdx.x >> 4, lc = threadIdx.x & 15;
-    const int vt = threadIdx.x & 31, vc = threadIdx.x >> 5;
-    f16x8 kr[NG], vr[NG];
-    auto load_group = [&](int g0, int nb) __attribute__((always_inline)) {
+  // Q^T as the B operand (zero past the last vector); a negative scale is folded into q's sign, so the running max
+  // can be taken before scaling.
+  f16x8 qb[8];
+  const int vq = v0 + l32;
+  const bool live = vq < nvec;
+  const int qpos = pos_of(live ? vq : nvec - 1);
+  const int qmin = pos_of(min(v0, nvec - 1));  // the wavefront's first query position (the least)
+  const float sc = fabsf(scale_log2);
+  {
+    const int vv = live ? vq : 0;
+    const int t = vv / G, g = vv - t * G;
+    const f16* qrow = q + (((size_t)b * q_len + t) * Hq + (size_t)kvh * G + g) * D + 8 * h;
+    const uint32_t flip = scale_log2 < 0.f ? 0x80008000u : 0u;
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 #pragma unroll
-      for (int i = 0; i < NG; ++i) {
-        if (i < nb) {
-          const int tok = min((g0 + i) * kBlock + lt, Lc - 1);  // past the context: masked, a valid page
-          const int page = ptrow[tok / P];
-          const size_t at = (((size_t)page * Hkv + kvh) * P + tok % P) * D + 8 * lc;
-          kr[i] = *reinterpret_cast<const f16x8*>(kp + at);
-          const int vtok = min((g0 + i) * kBlock + vt, Lc - 1);
-          const int vpage = ptrow[vtok / P];
-          vr[i] = *reinterpret_cast<const f16x8*>(vp + (((size_t)vpage * Hkv + kvh) * P + vtok % P) * D + 8 * vc);
-        }
-      }
-    };
-    auto stash_group = [&](int buf, int nb) __attribute__((always_inline)) {
-#pragma unroll
-      for (int i = 0; i < NG; ++i) {
-        if (i < nb) {
-          *reinterpret_cast<f16x8*>(&sk[buf][i][lt * kPfKRow + 8 * lc]) = kr[i];
-#pragma unroll
-          for (int e = 0; e < 8; ++e) sv[buf][i][(8 * vc + e) * kPfVRow + vt] = vr[i][e];
-        }
-      }
-    };
-    if (nblk > 0) load_group(0, min(NG, nblk));
-
-    // Q^T as the B operand (zero past the last vector), and each lane's query position.
-    f16x8 qb[4];
-    const int vq = v0 + li;
-    const bool live = vq < nvec;
-    const int qpos = pos_of(live ? vq : nvec - 1);
-    const int qmin = pos_of(min(v0, nvec - 1));  // the wavefront's first query position (the least)
-    {
-      const int vv = live ? vq : 0;
-      const int t = vv / G, g = vv - t * G;
-      const f16* qrow = q + (((size_t)b * q_len + t) * Hq + (size_t)kvh * G + g) * D + 8 * lg;
-#pragma unroll
-      for (int s = 0; s < 4; ++s) {
-        const f16x8 x = *reinterpret_cast<const f16x8*>(qrow + 32 * s);
-        qb[s] = live ? x : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
-      }
+    for (int s = 0; s < 8; ++s) {
+      const u32x4 x = *reinterpret_cast<const u32x4*>(qrow + 16 * s) ^ flip;
+      qb[s] = live ? __builtin_bit_cast(f16x8, x) : f16x8{0, 0, 0, 0, 0, 0, 0, 0};
     }
-    if (nblk > 0) stash_group(0, min(NG, nblk));
-    __syncthreads();
+  }
 
-    float m = -INFINITY, l = 0.f;  // query li: running max (every lane of the query), this lane's share of the sum
-    f32x4 acc[D / 16];             // O[query 4 lg + r][16 dt + li]
+  const float one = as_f32_value(1.f);
+  float m = -INFINITY, l = 0.f;  // query l32: running max (both lanes of the query), this lane's share of the sum
+  f32x16 acc[D / 32];            // O[query l32][32 dt + 8 j + 4 h + e], element 4 j + e
 #pragma unroll
-    for (int dt = 0; dt < D / 16; ++dt) acc[dt] = f32x4{0.f, 0.f, 0.f, 0.f};
-    auto block = [&](int buf, int i, int blk) __attribute__((always_inline)) {
-      f32x4 c[kTiles];
+  for (int dt = 0; dt < D / 32; ++dt)
 #pragma unroll
-      for (int j = 0; j < kTiles; ++j) {
-        c[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int r = 0; r < 16; ++r) acc[dt][r] = 0.f;
+
+  // Byte offsets of this lane's reads inside a stage.
+  const int krow = (kBlock * NB * cw + l32) * 2 * D, kx = 16 * (h ^ (l32 & 15));
+  const int ti = lane & 15, sub = (lane >> 4) & 1;
+  int vo[2];
 #pragma unroll
-        for (int s = 0; s < 4; ++s) {
-          const f16x8 a = *reinterpret_cast<const f16x8*>(&sk[buf][i][(16 * j + li) * kPfKRow + 32 * s + 8 * lg]);
-          c[j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a, qb[s], c[j], 0, 0, 0);
+  for (int a = 0; a < 2; ++a)
+    vo[a] = kHalf + (kBlock * NB * cw + 8 * a + 4 * h + (ti >> 2)) * 2 * D +
+            16 * ((2 * sub + ((ti & 3) >> 1)) ^ (2 * a + h)) + 8 * (ti & 1);
+
+  // This wavefront's NB blocks of a stage, from block `blk` on.
+  auto blocks = [&](const uint8_t* buf, int blk) __attribute__((always_inline)) {
+    f32x16 c[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      f16x8 ka[8];
+#pragma unroll
+      for (int s = 0; s < 8; ++s)
+        ka[s] = *reinterpret_cast<const f16x8*>(buf + krow + j * kBlock * 2 * D + (kx ^ (32 * s)));
+#pragma unroll
+      for (int r = 0; r < 16; ++r) c[j][r] = 0.f;
+#pragma unroll
+      for (int s = 0; s < 8; ++s) c[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(ka[s], qb[s], c[j], 0, 0, 0);
+    }
+    f16x8 va[NB][D / 32][2];
+    auto load_v = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+          const uint8_t* pv = buf + 64 * (dt ^ (ti >> 2)) + (2 * j + ks) * 16 * 2 * D;
+          const f16x4 lo = lds_read_tr(pv + vo[0]), hi = lds_read_tr(pv + vo[1]);
+          va[j][dt][ks] = f16x8{lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
         }
-      }
-      float mx = -INFINITY;
-      if (blk * kBlock + kBlock - 1 <= qmin) {  // uniform: every query of the wavefront sees the whole block
+    };
+    load_v(0);  // V^T of the first block goes to registers before the softmax, which hides the LDS latency
+    __builtin_amdgcn_sched_barrier(0);
+    if ((blk + NB) * kBlock - 1 > qmin) {  // uniform: some query of the wavefront does not see all the blocks
 #pragma unroll
-        for (int j = 0; j < kTiles; ++j)
+      for (int j = 0; j < NB; ++j)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            c[j][r] = c[j][r] * scale_log2;
-            mx = fmaxf(mx, c[j][r]);
-          }
-      } else {
+        for (int r = 0; r < 16; ++r)
+          c[j][r] = ((blk + j) * kBlock + 8 * (r >> 2) + 4 * h + (r & 3) <= qpos) ? c[j][r] : -INFINITY;
+    }
+    float mx = c[0][0];
 #pragma unroll
-        for (int j = 0; j < kTiles; ++j)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int key = blk * kBlock + 16 * j + 4 * lg + r;
-            c[j][r] = key <= qpos ? c[j][r] * scale_log2 : -INFINITY;
-            mx = fmaxf(mx, c[j][r]);
-          }
-      }
-      mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
-      mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-      // Block 0 comes first and key 0 is visible to every query with a position, so m is finite from then on and
-      // a fully masked later block leaves mn = m, alpha = 1 and p = 0.  A query with no key at all keeps m = -inf:
-      // alpha 1 and p 0 (not the NaN of -inf - -inf), l stays 0 and its output 0.
+    for (int r = 1; r < 16 * NB; ++r) mx = fmaxf(mx, c[r >> 4][r & 15]);
+    mx = fmaxf(mx, __shfl_xor(mx, 32, 64)) * sc;
+    // (m follows the running max exactly, so the largest p is exactly one: letting it lag by up to 2^8 to save most
+    // rescales took 5% off the time and added 3-5% to the error.)
+    // A query that has seen no key yet keeps m = -inf and subtracts 0 instead: its p and alpha are exp2(-inf) = 0
+    // (not the NaN of -inf - -inf).
+    if (__builtin_amdgcn_ballot_w64(mx > m) != 0) {  // uniform
       const float mn = fmaxf(m, mx);
-      const bool none = mn == -INFINITY;
-      const float alpha = none ? 1.f : __builtin_amdgcn_exp2f(m - mn);
-      f16x8 pa;
-      float ps = 0.f;
-#pragma unroll
-      for (int j = 0; j < kTiles; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const f16 p = static_cast<f16>(none ? 0.f : __builtin_amdgcn_exp2f(c[j][r] - mn));
-          pa[4 * j + r] = p;
-          ps += static_cast<float>(p);
-        }
-      l = l * alpha + ps;
+      const float alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+      l *= alpha;
       m = mn;
-      if (__builtin_amdgcn_ballot_w64(alpha != 1.f) != 0) {  // uniform
 #pragma unroll
-        for (int dt = 0; dt < D / 16; ++dt) acc[dt] *= alpha;
-      }
-#pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt) {
-        const f16* vrow = &sv[buf][i][(16 * dt + li) * kPfVRow];
-        const f16x4 lo = *reinterpret_cast<const f16x4*>(vrow + 4 * lg);
-        const f16x4 hi = *reinterpret_cast<const f16x4*>(vrow + 16 + 4 * lg);
-        const f16x8 vb = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
-        acc[dt] = __builtin_amdgcn_mfma_f32_16x16x32_f16(vb, pa, acc[dt], 0, 0, 0);
-      }
-    };
-    int buf = 0;
-    for (int g0 = 0; g0 < nblk; g0 += NG, buf ^= 1) {  // uniform
-      const int nb = min(NG, nblk - g0);
-      const int g1 = g0 + NG, nb1 = min(NG, nblk - g1);
-      if (nb1 > 0) load_group(g1, nb1);  // in flight during this group's math
-      for (int i = 0; i < nb; ++i)
-        if (g0 + i < wblk) block(buf, i, g0 + i);
-      if (nb1 > 0) stash_group(buf ^ 1, nb1);
-      __syncthreads();
+      for (int dt = 0; dt < D / 32; ++dt) acc[dt] *= alpha;
     }
-    l += __shfl_xor(l, 16, 64);
-    l += __shfl_xor(l, 32, 64);
+    const float ms = m == -INFINITY ? 0.f : m;
+#pragma unroll
+    for (int j = 0; j < NB; ++j) {
+      float ps = 0.f;
+      f16x8 pa[2];
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        pa[r >> 3][r & 7] = static_cast<f16>(__builtin_amdgcn_exp2f(fmaf(c[j][r], sc, -ms)));
+        // l sums the rounded p; the multiply by one (opaque) makes it one v_fma_mix_f32 reading the fp16 value
+        ps = fmaf(static_cast<float>(pa[r >> 3][r & 7]), one, ps);
+      }
+      l += ps;
+      if (j > 0) load_v(j);
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int dt = 0; dt < D / 32; ++dt)
+          acc[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(va[j][dt][ks], pa[ks], acc[dt], 0, 0, 0);
+    }
+  };
+  // Stage st: wait for its DMA, issue the next stage into the buffer that stage st - 1 has just left, multiply.
+  auto step = [&](const uint8_t* cur, uint8_t* other, int st) __attribute__((always_inline)) {
+    dma_wait_barrier();
+    if (st + 1 < s1) {
+      issue(other, st + 1);
+      fetch_page(min(st + 2, s1 - 1));
+    }
+    const int blk = (st * CW + cw) * NB;
+    if (blk < wblk) blocks(cur, blk);
+  };
+  if (s0 < s1) {
+    fetch_page(s0);
+    issue(st0, s0);
+    fetch_page(min(s0 + 1, s1 - 1));
+    for (int st = s0;;) {  // uniform
+      step(st0, st1, st);
+      if (++st >= s1) break;
+      step(st1, st0, st);
+      if (++st >= s1) break;
+    }
+  }
+  l += __shfl_xor(l, 32, 64);
 
-    if (live) {
-      const int t = vq / G, g = vq - t * G;
-      f16* po = out + (((size_t)b * q_len + t) * Hq + (size_t)kvh * G + g) * D + 4 * lg;
-      const float inv = l > 0.f ? 1.f / l : 0.f;
+  // Merge the CW groups in order: groups 1.. park (max, sum, O) in the stage buffers.
+  if constexpr (CW > 1) {
+    dma_wait_barrier();  // every DMA has landed, every wavefront has read its last stage
+    constexpr int kWaveO = 64 * 64 * 4;            // O of one wavefront
+    constexpr int kPer = 2 * kHalf / kWaveO;       // wavefronts per stage buffer
+    static_assert((CW - 1) * VW <= 2 * kPer, "parked outputs fit the first two buffers");
+    auto park = [&](int g, int v) __attribute__((always_inline)) -> float* {
+      const int i = (g - 1) * VW + v;
+      return reinterpret_cast<float*>((i < kPer ? st0 : st1) + (i % kPer) * kWaveO) + lane;
+    };
+    if (cw > 0) {
+      float* o = park(cw, vw);
 #pragma unroll
-      for (int dt = 0; dt < D / 16; ++dt)
-        *reinterpret_cast<f16x4*>(po + 16 * dt) = f16x4{static_cast<f16>(acc[dt][0] * inv), static_cast<f16>(acc[dt][1] * inv),
-                                                      static_cast<f16>(acc[dt][2] * inv), static_cast<f16>(acc[dt][3] * inv)};
+      for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[(16 * dt + r) * 64] = acc[dt][r];
+      sm_ml[cw][vw][0][lane] = m;
+      sm_ml[cw][vw][1][lane] = l;
     }
-  }  // pass
+    __syncthreads();
+    if (cw > 0) return;
+#pragma unroll
+    for (int g = 1; g < CW; ++g) {
+      const float* o = park(g, vw);
+      const float mg = sm_ml[g][vw][0][lane], lg = sm_ml[g][vw][1][lane];
+      const float mn = fmaxf(m, mg), ms = mn == -INFINITY ? 0.f : mn;
+      const float fa = __builtin_amdgcn_exp2f(m - ms), fb = __builtin_amdgcn_exp2f(mg - ms);
+      m = mn;
+      l = fmaf(l, fa, lg * fb);
+#pragma unroll
+      for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[dt][r] = fmaf(acc[dt][r], fa, o[(16 * dt + r) * 64] * fb);
+    }
+  }
+  if (!live) return;
+  const int t = vq / G, g = vq - t * G;
+  const size_t head = ((size_t)b * q_len + t) * Hq + (size_t)kvh * G + g;
+  if (S == 1) {
+    f16* po = out + head * D + 4 * h;
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<f16x4*>(po + 32 * dt + 8 * j) =
+            f16x4{static_cast<f16>(acc[dt][4 * j] * inv), static_cast<f16>(acc[dt][4 * j + 1] * inv),
+                  static_cast<f16>(acc[dt][4 * j + 2] * inv), static_cast<f16>(acc[dt][4 * j + 3] * inv)};
+  } else {
+    float* po = part_o + (head * S + split) * D + 4 * h;
+#pragma unroll
+    for (int dt = 0; dt < D / 32; ++dt)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        *reinterpret_cast<f32x4*>(po + 32 * dt + 8 * j) =
+            f32x4{acc[dt][4 * j], acc[dt][4 * j + 1], acc[dt][4 * j + 2], acc[dt][4 * j + 3]};
+    if (h == 0) {
+      float* ml = part_ml + (head * S + split) * 2;
+      ml[0] = m;
+      ml[1] = l;
+    }
+  }
 }
 
 // ----------------------------------------------------------------------------
@@ -952,6 +1034,34 @@ int device_cus() {
   return n;
 }
 
+// Prefill launch: wavefronts on query tiles x wavefronts sharing their context, tiles per (sequence, KV head) and
+// context splits.  Measured on MI355X, us per launch (32/8 heads unless said):
+//   * up to kPfSplitTokens of context a workgroup walks few stages and its start and merge dominate: four wavefronts,
+//     two workgroups per CU, no merge (8 x 512 tokens 39.7 against 51.2 with 8 wavefronts, 5 x 301 at 28/4 15.1
+//     against 20.4).  The choice looks at the sequence alone there, so a batch gives the bits of its sequences
+//     launched one by one.
+//   * longer contexts: 8 wavefronts in two context groups (2 x 509 tokens after 3500 at 28/4: 78.6 against 94.8 with
+//     four wavefronts in one group); four in one group again once the grid keeps every CU's two workgroups busy for more than one round
+//     (2 x 2048 tokens: 89.0 against 98.3); 64-vector tiles in four context groups where 128-vector tiles leave half
+//     of the CUs idle (4 x 400 tokens after 1000 at 8/8: 23.5 against 28.9, 100 after 3000: 24.3 against 28.5).
+//   * a grid below one workgroup per CU splits long contexts into pieces of kPfSplitTokens / 2 or more.
+struct PrefillPlan {
+  int vec_waves, ctx_waves, tiles, splits;
+};
+constexpr int kPfSplitTokens = 1024;
+PrefillPlan prefill_plan(int batch, int q_len, int Hkv, int G, int max_ctx) {
+  const int nvec = q_len * G;
+  const long seqs = (long)Hkv * batch, cus = device_cus();
+  const long groups4 = (nvec + 4 * kPfVec - 1) / (4 * kPfVec) * seqs;  // workgroups at 128 vectors each
+  const bool longctx = max_ctx > kPfSplitTokens;
+  PrefillPlan p;
+  p.vec_waves = (nvec <= 2 * kPfVec || (longctx && 2 * groups4 <= cus)) ? 2 : 4;
+  p.ctx_waves = p.vec_waves == 2 ? 4 : (longctx && groups4 < 3 * cus) ? 2 : 1;
+  p.tiles = (nvec + kPfVec * p.vec_waves - 1) / (kPfVec * p.vec_waves);
+  p.splits = longctx ? (int)max(1L, min(2L * max_ctx / kPfSplitTokens, cus / (p.tiles * seqs))) : 1;
+  return p;
+}
+
 int launch_attention(const void* q, const void* k_pool, const void* v_pool, const int32_t* page_table,
                      const int32_t* seq_lens, void* out, void* workspace, size_t workspace_bytes,
                      int batch, int q_len, int Hq, int Hkv, int D, int P, int max_pages, float scale,
@@ -985,22 +1095,20 @@ int launch_attention(const void* q, const void* k_pool, const void* v_pool, cons
   float* part_o = static_cast<float*>(workspace);
   float* part_ml = part_o + (size_t)rows * Hq * S * D;
   dim3 grid(S, Hkv, rows);
-  if (mfma && q_len > 1) {  // prefill: query tiles of 128 vectors over each sequence's blocks, no partials
-    const int tiles = (q_len * G + 16 * kPfWaves - 1) / (16 * kPfWaves);
-    // Pairs of tiles per workgroup once the unpaired grid fills every CU's two workgroup slots: the causal
-    // mask's long and short tiles then share a workgroup instead of the longest setting the kernel's time.
-    const long one_tile = (long)tiles * Hkv * batch;
-    const bool paired = tiles > 1 && one_tile >= 2L * device_cus();
-    const long workgroups = paired ? (long)((tiles + 1) / 2) * Hkv * batch : one_tile;
-    // A grid of at most one workgroup per CU stages twice the blocks per buffer (143 KiB of LDS, twice the loads
-    // in flight); a larger one keeps 70 KiB so two workgroups share a CU and the grid runs in one round.
-    const bool deep = workgroups <= device_cus();
-    const auto kernel = paired ? (deep ? attn_prefill_f16_d128<true, 2 * kPfGroup> : attn_prefill_f16_d128<true, kPfGroup>)
-                               : (deep ? attn_prefill_f16_d128<false, 2 * kPfGroup>
-                                       : attn_prefill_f16_d128<false, kPfGroup>);
-    kernel<<<dim3(paired ? (tiles + 1) / 2 : tiles, Hkv, batch), 64 * kPfWaves, 0, s>>>(
+  if (mfma && q_len > 1) {  // prefill: query tiles over each sequence's blocks
+    const PrefillPlan pl = prefill_plan(batch, q_len, Hkv, G, max_ctx);
+    const dim3 pgrid(Hkv * batch, pl.tiles, pl.splits);
+    const auto kernel = pl.ctx_waves == 4   ? attn_prefill_f16_d128<2, 4, 1>
+                        : pl.ctx_waves == 2 ? attn_prefill_f16_d128<4, 2, 2>
+                                            : attn_prefill_f16_d128<4, 1, 2>;
+    part_ml = part_o + (size_t)rows * Hq * pl.splits * D;
+    kernel<<<pgrid, 64 * pl.vec_waves * pl.ctx_waves, 0, s>>>(
         static_cast<const f16*>(q), static_cast<const f16*>(k_pool), static_cast<const f16*>(v_pool), page_table,
-        seq_lens, static_cast<f16*>(out), q_len, Hq, Hkv, P, max_pages, scale_log2);
+        seq_lens, static_cast<f16*>(out), part_o, part_ml, q_len, Hq, Hkv, P, max_pages, pl.splits,
+        scale_log2 == 0.f ? FLT_MIN : scale_log2);  // (a masked score is -inf: -inf * 0 would be NaN)
+    const int st = launch_status();
+    if (st || pl.splits == 1) return st;
+    attn_merge<f16><<<dim3(Hq, rows), 128, 0, s>>>(part_o, part_ml, static_cast<f16*>(out), Hq, D, pl.splits);
     return launch_status();
   }
   if (mfma) {

@@ -49,6 +49,19 @@ template <typename T> __device__ __forceinline__ T from_f32(float v);
 template <> __device__ __forceinline__ float from_f32<float>(float v) { return v; }
 template <> __device__ __forceinline__ f16 from_f32<f16>(float v) { return static_cast<f16>(v); }
 
+typedef __amdgpu_buffer_rsrc_t rsrc_t;
+// Raw buffer resource over [p, p + bytes) (gfx9 descriptor word 3: raw byte-addressed
+// loads, out-of-range lanes read 0).
+__device__ __forceinline__ rsrc_t make_rsrc(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
+}
+// 16 bytes per lane from the buffer straight into LDS: lane l's bytes land at lds + 16 l.
+// (A device function, not a lambda: kernel lambdas are also compiled for the host,
+// where the builtin does not exist, and the host pass then drops the kernel's stub.)
+__device__ __forceinline__ void buf16_to_lds(rsrc_t r, uint8_t* lds, uint32_t voff, uint32_t soff) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, 0);
+}
+
 // Wavefront (64-lane) reductions through DPP/swizzle-backed shuffles.
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll

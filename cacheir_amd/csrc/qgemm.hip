@@ -627,12 +627,6 @@ __global__ __launch_bounds__(256 * KG) void qgemm_xs_kernel(const f16* __restric
 }
 
 // ------------------------------------------------------------------ GEMV -----
-typedef __amdgpu_buffer_rsrc_t rsrc_t;
-// Raw buffer resource over [p, p + bytes) (gfx9 descriptor word 3: raw byte-addressed
-// loads, out-of-range lanes read 0).
-__device__ __forceinline__ rsrc_t make_rsrc(const void* p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), (short)0, (int)bytes, 0x00020000);
-}
 __device__ __forceinline__ uint4 buf16(rsrc_t r, uint32_t voff, uint32_t soff) {
   const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
   return uint4{v.x, v.y, v.z, v.w};
@@ -642,13 +636,6 @@ __device__ __forceinline__ uint2 buf8(rsrc_t r, uint32_t voff, uint32_t soff) {
   const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
   return uint2{v.x, v.y};
 }
-// 16 bytes per lane from the buffer straight into LDS: lane l's bytes land at lds + 16 l.
-// (A device function, not a lambda: kernel lambdas are also compiled for the host,
-// where the builtin does not exist, and the host pass then drops the kernel's stub.)
-__device__ __forceinline__ void buf16_to_lds(rsrc_t r, uint8_t* lds, uint32_t voff, uint32_t soff) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)lds, 16, voff, soff, 0, 0);
-}
-
 // ------------------------------------------------------------- large m ------
 // m > 32 (qgemm_xl_kernel): a workgroup of 4 wavefronts covers 8 weight tiles (128
 // output columns, 2 per wavefront) and 16*MT activation rows, so each weight tile is

@@ -201,6 +201,35 @@ def test_prefill_attention_fp16_random_shapes(device, seed):
         close16(out[b * q_len:(b + 1) * q_len], ref)
 
 
+@pytest.mark.parametrize("batch,g,hkv,q_len,past,scale", [
+    (1, 7, 2, 9, 1100, None),      # at most 64 query vectors over a long context: 64-vector tiles, context splits
+    (1, 4, 2, 33, 2500, None),     # few 128-vector tiles: 64-vector tiles, context splits with a ragged last one
+    (2, 8, 8, 140, 1000, None),    # 8 wavefronts in two context groups, unsplit
+    (6, 8, 8, 257, 800, None),     # a grid past three workgroups per CU: 4 wavefronts over a long context
+    (2, 3, 2, 50, 40, -0.1),       # a negative scale (folded into q's sign)
+    (1, 1, 1, 65, 0, 0.0),         # a zero scale: uniform weights over the visible tokens
+])
+def test_prefill_attention_geometries(device, batch, g, hkv, q_len, past, scale):
+    """Each launch geometry of the fp16 prefill kernel against the oracle, at sizes whose tiles, stages and splits end
+    ragged; fp16 storage bound as the other attention tests."""
+    from cacheir_amd import kernels
+
+    rng = np.random.default_rng(q_len + past)
+    total = np.array([past + q_len + 13 * b for b in range(batch)])
+    kp, vp, pt, lens = paged.build_pool(rng, total, hkv, 128, 16)
+    hq = g * hkv
+    q = rng.standard_normal((batch * q_len, hq, 128)).astype(np.float16)
+    out = kernels.paged_prefill_attention(to_dev(q, device), to_dev(kp, device), to_dev(vp, device), to_dev(pt, device),
+                                          to_dev(lens, device), q_len, scale=scale).float().cpu().numpy()
+    unit = 1.0 if scale is None else scale * 128 ** 0.5  # the oracle scales by 128^-0.5
+    for b in range(batch):
+        kh = paged.gather_sequence(kp, pt[b], int(total[b])).astype(np.float32)[None]
+        vh = paged.gather_sequence(vp, pt[b], int(total[b])).astype(np.float32)[None]
+        qh = q[b * q_len:(b + 1) * q_len].astype(np.float32)[None] * np.float32(unit)
+        ref = ops.attention(qh, kh, vh, hq, hkv, 128, causal=True).reshape(q_len, hq, 128)
+        close16(out[b * q_len:(b + 1) * q_len], ref)
+
+
 @pytest.mark.parametrize("q_len,batch", [(600, 14), (590, 14), (512, 16), (600, 10)])
 def test_prefill_attention_paired_tiles(device, q_len, batch):
     """A prefill grid of at least two workgroups per CU runs tile pairs (tiles - 1 - x, then x) in one workgroup:
