@@ -860,71 +860,159 @@ __global__ __launch_bounds__(64 * VW * CW, 2) void attn_prefill_f16_d128(
 }
 
 // ----------------------------------------------------------------------------
-// Generic VALU kernel (fp32 or fp16 pools, any page size, head_dim <= 256):
-// one wavefront per (128-token chunk, KV head, row); always writes partials.
-template <typename T>
-__global__ __launch_bounds__(64) void attn_chunk_generic(
+// Generic kernel (fp32 or fp16 pools, any page size, head_dim <= 256): four wavefronts
+// per (128-token chunk, KV head, row).  LPT lanes (D <= 4 LPT) hold four dims each of a
+// token's K and V rows, so a wavefront takes TPW = 64 / LPT tokens per load and kGenU
+// loads of each in flight; the score of a token is summed over its LPT lanes by DPP and
+// stays in their registers, where P V needs it, so nothing but the wavefronts' (max, sum,
+// O) goes through LDS.  kGenHeads query heads of the group share each load.  One chunk
+// (NC == 1) writes the output itself; more leave partials for attn_merge.  These launches
+// are bound by latency (page entry, then K and V): the tiny model's decode attention took
+// 23.5 us with one wavefront per chunk, a token per lane and the dims in turn.
+constexpr int kGenWaves = 4;
+constexpr int kGenU = 8;
+constexpr int kGenHeads = 4;
+
+// Four consecutive values as fp32 (VEC: one vector load; else one by one, zero past n).
+template <bool VEC>
+__device__ __forceinline__ f32x4 load_dims(const float* p, int n) {
+  if constexpr (VEC) return *reinterpret_cast<const f32x4*>(p);
+  f32x4 v;
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = e < n ? p[e] : 0.f;
+  return v;
+}
+template <bool VEC>
+__device__ __forceinline__ f32x4 load_dims(const f16* p, int n) {
+  f32x4 v;
+  if constexpr (VEC) {
+    const f16x4 t = *reinterpret_cast<const f16x4*>(p);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = static_cast<float>(t[e]);
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) v[e] = e < n ? static_cast<float>(p[e]) : 0.f;
+  }
+  return v;
+}
+
+template <typename T, int LPT, bool VEC>
+__global__ __launch_bounds__(64 * kGenWaves) void attn_chunk_generic(
     const T* __restrict__ q, const T* __restrict__ kp, const T* __restrict__ vp,
-    const int32_t* __restrict__ pt, const int32_t* __restrict__ lens,
+    const int32_t* __restrict__ pt, const int32_t* __restrict__ lens, T* __restrict__ out,
     float* __restrict__ part_o, float* __restrict__ part_ml,
     int q_len, int Hq, int Hkv, int D, int P, int max_pages, int NC, float scale_log2) {
-  __shared__ float qs[256];
-  __shared__ float ps[kChunk];
+  constexpr int TPW = 64 / LPT;
+  __shared__ float sm_m[kGenWaves][kGenHeads], sm_l[kGenWaves][kGenHeads];
+  __shared__ __align__(16) float sm_o[kGenWaves][kGenHeads][4 * LPT];
   const int chunk = blockIdx.x, kvh = blockIdx.y, row = blockIdx.z;
   const int L = visible_len(lens, row, q_len, max_pages * P);
   const int t0 = chunk * kChunk;
   const int G = Hq / Hkv;
-  const int lane = threadIdx.x;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int d0 = 4 * (lane & (LPT - 1)), grp = lane / LPT;
+  const int nd = max(0, min(4, D - d0));  // this lane's dims (none: it repeats dim 0 and drops out by zeros)
   const int n = max(0, min(L, t0 + kChunk) - t0);
-  const int b = row / q_len;
-  const int32_t* ptrow = pt + (size_t)b * max_pages;
-  for (int h = 0; h < G; ++h) {
-    const int head = kvh * G + h;
-    float* ml = part_ml + (((size_t)row * Hq + head) * NC + chunk) * 2;
-    if (n == 0) {  // empty chunk: neutral partial
-      for (int d = lane; d < D; d += 64) part_o[(((size_t)row * Hq + head) * NC + chunk) * D + d] = 0.f;
+  const int32_t* ptrow = pt + (size_t)(row / q_len) * max_pages;
+  const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+  for (int h0 = 0; h0 < G; h0 += kGenHeads) {  // uniform
+    const int nh = min(kGenHeads, G - h0);
+    const size_t head0 = (size_t)row * Hq + (size_t)kvh * G + h0;
+    f32x4 qv[kGenHeads], o[kGenHeads];
+    float m[kGenHeads], l[kGenHeads];
+#pragma unroll
+    for (int h = 0; h < kGenHeads; ++h) {
+      const f32x4 t = load_dims<VEC>(q + (head0 + min(h, nh - 1)) * D + (nd ? d0 : 0), nd);
+      qv[h] = nd ? t : zero;
+      o[h] = zero;
+      m[h] = -INFINITY;
+      l[h] = 0.f;
+    }
+    for (int j0 = wave * TPW; j0 < n; j0 += kGenU * kGenWaves * TPW) {  // uniform; tokens j0 + i * kGenWaves * TPW + grp
+      f32x4 kv[kGenU], vv[kGenU];
+      bool in[kGenU];
+#pragma unroll
+      for (int i = 0; i < kGenU; ++i) {
+        const int j = j0 + i * kGenWaves * TPW + grp;
+        in[i] = j < n;
+        const int t = t0 + (in[i] ? j : 0);  // tokens past the chunk re-read its first one (p = 0)
+        const size_t at = (((size_t)ptrow[t / P] * Hkv + kvh) * P + t % P) * D + (nd ? d0 : 0);
+        const f32x4 a = load_dims<VEC>(kp + at, nd), c = load_dims<VEC>(vp + at, nd);
+        kv[i] = nd ? a : zero;
+        vv[i] = in[i] ? c : zero;
+      }
+#pragma unroll
+      for (int h = 0; h < kGenHeads; ++h) {
+        if (h >= nh) break;
+        float s[kGenU], mx = m[h];
+#pragma unroll
+        for (int i = 0; i < kGenU; ++i) {
+          float dot = 0.f;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) dot = fmaf(qv[h][e], kv[i][e], dot);
+          dot = row16_sum(dot);
+          if constexpr (LPT >= 32) dot += __shfl_xor(dot, 16, 64);
+          if constexpr (LPT >= 64) dot += __shfl_xor(dot, 32, 64);
+          s[i] = in[i] ? dot * scale_log2 : -INFINITY;
+          mx = fmaxf(mx, s[i]);
+        }
+        if constexpr (LPT <= 16) mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
+        if constexpr (LPT <= 32) mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
+        const float a = exp2f(m[h] - mx);  // finite mx: token j0 of the wavefront exists
+        l[h] *= a;
+        o[h] *= a;
+        m[h] = mx;
+#pragma unroll
+        for (int i = 0; i < kGenU; ++i) {
+          const float p = exp2f(s[i] - mx);
+          l[h] += p;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[h][e] = fmaf(p, vv[i][e], o[h][e]);
+        }
+      }
+    }
+    // Sum the TPW token groups of the wavefront, then merge the wavefronts in order.
+#pragma unroll
+    for (int h = 0; h < kGenHeads; ++h) {
+#pragma unroll
+      for (int off = LPT; off < 64; off <<= 1) {
+        l[h] += __shfl_xor(l[h], off, 64);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[h][e] += __shfl_xor(o[h][e], off, 64);
+      }
+      if (grp == 0) *reinterpret_cast<f32x4*>(&sm_o[wave][h][d0]) = o[h];
       if (lane == 0) {
-        ml[0] = -INFINITY;
-        ml[1] = 0.f;
+        sm_m[wave][h] = m[h];
+        sm_l[wave][h] = l[h];
       }
-      continue;
     }
     __syncthreads();
-    for (int d = lane; d < D; d += 64) qs[d] = to_f32(q[((size_t)row * Hq + head) * D + d]);
-    __syncthreads();
-    float mx = -INFINITY;
-    for (int j = lane; j < n; j += 64) {
-      const int t = t0 + j;
-      const int page = ptrow[t / P];
-      const T* krow = kp + (((size_t)page * Hkv + kvh) * P + (t % P)) * D;
-      float dot = 0.f;
-      for (int d = 0; d < D; ++d) dot = fmaf(qs[d], to_f32(krow[d]), dot);
-      const float s = dot * scale_log2;
-      ps[j] = s;
-      mx = fmaxf(mx, s);
-    }
-    mx = wave_max(mx);
-    float sum = 0.f;
-    for (int j = lane; j < n; j += 64) {
-      const float p = exp2f(ps[j] - mx);
-      ps[j] = p;
-      sum += p;
-    }
-    sum = wave_sum(sum);
-    __syncthreads();
-    for (int d = lane; d < D; d += 64) {
-      float o = 0.f;
-      for (int j = 0; j < n; ++j) {
-        const int t = t0 + j;
-        const int page = ptrow[t / P];
-        o = fmaf(ps[j], to_f32(vp[(((size_t)page * Hkv + kvh) * P + (t % P)) * D + d]), o);
+    for (int idx = threadIdx.x; idx < nh * D; idx += 64 * kGenWaves) {
+      const int h = idx / D, d = idx - h * D;
+      float M = -INFINITY;
+#pragma unroll
+      for (int w = 0; w < kGenWaves; ++w) M = fmaxf(M, sm_m[w][h]);
+      float den = 0.f, acc = 0.f;
+      if (M != -INFINITY) {
+#pragma unroll
+        for (int w = 0; w < kGenWaves; ++w) {
+          const float f = exp2f(sm_m[w][h] - M);
+          den = fmaf(sm_l[w][h], f, den);
+          acc = fmaf(sm_o[w][h][d], f, acc);
+        }
       }
-      part_o[(((size_t)row * Hq + head) * NC + chunk) * D + d] = o;
+      if (NC == 1) {
+        out[(head0 + h) * D + d] = from_f32<T>(as_f32_value(acc * (den > 0.f ? 1.f / den : 0.f)));
+      } else {
+        part_o[((head0 + h) * NC + chunk) * D + d] = acc;
+        if (d == 0) {
+          float* ml = part_ml + ((head0 + h) * NC + chunk) * 2;
+          ml[0] = M;
+          ml[1] = den;
+        }
+      }
     }
-    if (lane == 0) {
-      ml[0] = mx;
-      ml[1] = sum;
-    }
+    __syncthreads();  // the next heads write the same arrays
   }
 }
 
@@ -1137,17 +1225,23 @@ int launch_attention(const void* q, const void* k_pool, const void* v_pool, cons
     const int st = launch_status();
     if (st || S == 1 || !merge) return st;
   } else {
-    if (kv_dtype == CIR_F16) {
-      attn_chunk_generic<f16><<<grid, 64, 0, s>>>(static_cast<const f16*>(q), static_cast<const f16*>(k_pool),
-                                                  static_cast<const f16*>(v_pool), page_table, seq_lens, part_o,
-                                                  part_ml, q_len, Hq, Hkv, D, P, max_pages, S, scale_log2);
-    } else {
-      attn_chunk_generic<float><<<grid, 64, 0, s>>>(static_cast<const float*>(q), static_cast<const float*>(k_pool),
-                                                    static_cast<const float*>(v_pool), page_table, seq_lens, part_o,
-                                                    part_ml, q_len, Hq, Hkv, D, P, max_pages, S, scale_log2);
-    }
+    // Vector loads of four dims need rows on whole, aligned groups of four.
+    const bool vec = D % 4 == 0 && (reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k_pool) |
+                                    reinterpret_cast<uintptr_t>(v_pool)) % 16 == 0;
+    auto go = [&]<typename T, int LPT, bool VEC>() {
+      attn_chunk_generic<T, LPT, VEC><<<grid, 64 * kGenWaves, 0, s>>>(
+          static_cast<const T*>(q), static_cast<const T*>(k_pool), static_cast<const T*>(v_pool), page_table, seq_lens,
+          static_cast<T*>(out), part_o, part_ml, q_len, Hq, Hkv, D, P, max_pages, S, scale_log2);
+    };
+    auto by_dim = [&]<typename T, bool VEC>() {
+      if (D <= 64) go.template operator()<T, 16, VEC>();
+      else if (D <= 128) go.template operator()<T, 32, VEC>();
+      else go.template operator()<T, 64, VEC>();
+    };
+    if (kv_dtype == CIR_F16) vec ? by_dim.template operator()<f16, true>() : by_dim.template operator()<f16, false>();
+    else vec ? by_dim.template operator()<float, true>() : by_dim.template operator()<float, false>();
     const int st = launch_status();
-    if (st) return st;
+    if (st || S == 1) return st;
   }
   dim3 mgrid(Hq, rows);
   if (kv_dtype == CIR_F16) {
