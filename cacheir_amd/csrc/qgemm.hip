@@ -345,7 +345,87 @@ __device__ __forceinline__ void row_sums(const f16x8 (&x)[MT][4], f32x4 (&sx)[MT
     for (int a = 0; a < MT; ++a) sx[a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(x[a][j], ones, sx[a], 0, 0, 0);
 }
 
-// Dense fp32: one wavefront per output row n, lanes over k; all m rows.
+// Dense fp32 (the reference's unquantized artifacts): y = x W^T on the fp32 MFMA 16x16x4, whose products and sums are
+// fp32.  A workgroup of four wavefronts owns 16 output columns and 16 * MT rows and shares out k: wavefront w takes
+// the 64-column pieces w, w + 4, ... of the split, loads a piece's operands (16 bytes a lane, 256 contiguous bytes a
+// row) before the first product, and the four sums meet in LDS.  Lane 16g + r holds columns
+// 4g .. 4g + 3 of 16-column step u for row r of either operand, so MFMA e of a step covers columns 4g + e: a fixed
+// permutation of k, the same for both.  Every step (and at MT = 1 every MFMA of it) of a piece has an accumulator of its
+// own, added pairwise at the end, so a sum's chain stays as short as the lanes-then-tree order of the plain kernel below
+// (one accumulator: 1.3-1.6 times its error).  Launches of these sizes are bound by latency (one load round trip per piece);
+// the tiny model's 48-row products (k 256, n 256 - 1376) took 53-72 us one wavefront per column with the rows in turn.
+template <int MT>
+__global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restrict__ x, int ldx,
+                                                            const float* __restrict__ w, float* __restrict__ part,
+                                                            int M, int N, int K, int kc) {
+  constexpr int U = 4;                // 16-column steps per piece
+  constexpr int E = MT == 1 ? 4 : 1;  // accumulators per step
+  __shared__ f32x4 red[3][MT][64];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int li = lane & 15, lg = lane >> 4;
+  const int n = blockIdx.x * 16 + li, m0 = blockIdx.z * 16 * MT;
+  const int split = blockIdx.y;
+  const int k0 = split * kc, k1 = min(K, k0 + kc);  // both multiples of 4 (the host's check)
+  const float* wr = w + (size_t)min(n, N - 1) * K;  // rows past the end repeat the last one (not stored)
+  const float* xr[MT];
+#pragma unroll
+  for (int a = 0; a < MT; ++a) xr[a] = x + (size_t)min(m0 + 16 * a + li, M - 1) * ldx;
+  f32x4 part_acc[U * E][MT];
+#pragma unroll
+  for (int i = 0; i < U * E; ++i)
+#pragma unroll
+    for (int a = 0; a < MT; ++a) part_acc[i][a] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int kb = k0 + 16 * U * wave; kb < k1; kb += 64 * U) {
+    f32x4 wv[U], xv[U][MT];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = kb + 16 * u + 4 * lg;
+      const bool in = k < k1;  // columns past the split are zero in both operands
+      const int kk = in ? k : k0;
+      wv[u] = *reinterpret_cast<const f32x4*>(wr + kk);
+#pragma unroll
+      for (int a = 0; a < MT; ++a) xv[u][a] = *reinterpret_cast<const f32x4*>(xr[a] + kk);
+      if (!in) {
+        wv[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int a = 0; a < MT; ++a) xv[u][a] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int a = 0; a < MT; ++a)
+          part_acc[u * E + e % E][a] =
+              __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u][a][e], wv[u][e], part_acc[u * E + e % E][a], 0, 0, 0);
+  }
+#pragma unroll
+  for (int half = U * E / 2; half > 0; half /= 2)
+#pragma unroll
+    for (int i = 0; i < half; ++i)
+#pragma unroll
+      for (int a = 0; a < MT; ++a) part_acc[i][a] += part_acc[i + half][a];
+  f32x4(&acc)[MT] = part_acc[0];
+  if (wave > 0) {
+#pragma unroll
+    for (int a = 0; a < MT; ++a) red[wave - 1][a][lane] = acc[a];
+  }
+  __syncthreads();
+  if (wave > 0 || n >= N) return;
+#pragma unroll
+  for (int a = 0; a < MT; ++a) {
+    acc[a] = (acc[a] + red[0][a][lane]) + (red[1][a][lane] + red[2][a][lane]);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int m = m0 + 16 * a + 4 * lg + r;
+      if (m < M) part[((size_t)split * M + m) * N + n] = acc[a][r];
+    }
+  }
+}
+
+// The same for rows that are not whole aligned 16-byte groups: one wavefront per output column, lanes over k, the m
+// rows in turn.
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ x, int ldx, const float* __restrict__ w,
                                                        float* __restrict__ part, int M, int N, int K, int kc) {
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -2020,8 +2100,19 @@ extern "C" int cir_gemm_f32(const float* x, int ldx, const float* w, float* y_pa
   CIR_CHECK_ARG(ldx >= k, "gemm_f32: ldx (%d) < k (%d)", ldx, k);
   CIR_CHECK_ARG(x && w && y_partial, "gemm_f32: null pointer");
   const int kc = (k + splits - 1) / splits;
+  hipStream_t s = as_stream(stream);
+  // 16-byte operand loads: every row and every split must start on 16 bytes.  Up to 64 rows a workgroup takes 16 of
+  // them (the grid is short); more rows go 64 at a time, so each weight column is read a quarter as often.
+  if (k % 4 == 0 && ldx % 4 == 0 && kc % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+      reinterpret_cast<uintptr_t>(w) % 16 == 0 && (m + 15) / 16 <= 65535) {
+    if (m <= 64)
+      gemm_f32_mfma_kernel<1><<<dim3((n + 15) / 16, splits, (m + 15) / 16), 256, 0, s>>>(x, ldx, w, y_partial, m, n, k, kc);
+    else
+      gemm_f32_mfma_kernel<4><<<dim3((n + 15) / 16, splits, (m + 63) / 64), 256, 0, s>>>(x, ldx, w, y_partial, m, n, k, kc);
+    return launch_status();
+  }
   dim3 grid((n + 3) / 4, splits);
-  gemm_f32_kernel<<<grid, 256, 0, as_stream(stream)>>>(x, ldx, w, y_partial, m, n, k, kc);
+  gemm_f32_kernel<<<grid, 256, 0, s>>>(x, ldx, w, y_partial, m, n, k, kc);
   return launch_status();
 }
 

@@ -535,6 +535,59 @@ def test_qgemm_planner_random_shapes_row_formats(device, seed):
     assert np.array_equal(ids[clear], ref64.argmax(axis=1)[clear])
 
 
+@pytest.mark.parametrize("m,n,k,splits", [
+    (1, 5, 4, 1),        # one column group short of a tile, a single 4-column group of k
+    (17, 33, 252, 1),    # rows, columns and k one past (or short of) a tile, the last piece ragged
+    (64, 688, 688, 4),   # the last size of the 16-row kernel; splits of 172 columns
+    (65, 31, 260, 1),    # the first size of the 64-row kernel
+    (130, 16, 1028, 2),  # 64-row blocks with a ragged last one; splits of 514 columns: not whole 16-byte groups
+    (3, 20, 30, 1),      # k not a multiple of 4: the one-column-per-wavefront kernel
+])
+def test_gemm_f32_shapes(device, m, n, k, splits):
+    """Dense fp32 products at the edges of their tiles against float64: |error| <= k eps sum |x w| / 2 bounds any order
+    of k fp32 products and sums (each rounds by at most eps / 2 of a partial sum no larger than sum |x w|)."""
+    from cacheir_amd import kernels
+
+    rng = np.random.default_rng(m + n + k)
+    x, w = rng.standard_normal((m, k), dtype=np.float32), rng.standard_normal((n, k), dtype=np.float32)
+    part = kernels.gemm_f32_partial(to_dev(x, device), to_dev(w, device), splits=splits)
+    got = part.sum(0).cpu().numpy().astype(np.float64)
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    bound = (k + splits) * np.finfo(np.float32).eps / 2 * (np.abs(x64) @ np.abs(w64).T)
+    assert np.all(np.abs(got - x64 @ w64.T) <= bound)
+
+
+@pytest.mark.parametrize("d,g,psize,dtype,past,q_len", [
+    (64, 2, 16, np.float32, 0, 1),     # one token: one chunk, three idle wavefronts
+    (64, 5, 16, np.float32, 127, 2),   # a second chunk of one token; five query heads (two passes of heads)
+    (128, 3, 5, np.float32, 200, 3),   # 32 lanes per token, pages that no tile divides
+    (256, 1, 16, np.float16, 90, 2),   # 64 lanes per token
+    (80, 9, 16, np.float16, 140, 2),   # lanes past the last dim; nine heads
+    (6, 2, 16, np.float32, 33, 2),     # rows that are not whole groups of four
+])
+def test_generic_attention_shapes(device, d, g, psize, dtype, past, q_len):
+    """The generic attention kernel at the edges of its lanes, chunks and head passes against the oracle (fp32: 1e-4;
+    fp16: the storage bound of the other attention tests)."""
+    from cacheir_amd import kernels
+
+    rng = np.random.default_rng(d + past)
+    hkv, batch = 2, 2
+    total = np.array([past + q_len, max(q_len, past // 2)])
+    kp, vp, pt, lens = paged.build_pool(rng, total, hkv, d, psize, dtype=dtype)
+    q = rng.standard_normal((batch * q_len, g * hkv, d)).astype(dtype)
+    out = kernels.paged_prefill_attention(to_dev(q, device), to_dev(kp, device), to_dev(vp, device), to_dev(pt, device),
+                                          to_dev(lens, device), q_len).float().cpu().numpy()
+    for b in range(batch):
+        kh = paged.gather_sequence(kp, pt[b], int(total[b])).astype(np.float32)[None]
+        vh = paged.gather_sequence(vp, pt[b], int(total[b])).astype(np.float32)[None]
+        qh = q[b * q_len:(b + 1) * q_len].astype(np.float32)[None]
+        ref = ops.attention(qh, kh, vh, g * hkv, hkv, d, causal=True).reshape(q_len, g * hkv, d)
+        if dtype == np.float32:
+            np.testing.assert_allclose(out[b * q_len:(b + 1) * q_len], ref, atol=1e-4, rtol=1e-4)
+        else:
+            close16(out[b * q_len:(b + 1) * q_len], ref)
+
+
 def test_gemm_f32(device):
     from cacheir_amd import kernels
 
