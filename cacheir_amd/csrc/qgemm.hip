@@ -32,48 +32,12 @@
 // the quads of the workgroup's k-range in lock step and share each quad of
 // activations through LDS.  grid.y splits k (fp32 partials, summed by the epilogue
 // kernels); grid.z walks 16*MT-row blocks of x.
-#include "common.hpp"
+#include "qgemm.hpp"
 
 #include <utility>
 
 namespace cir {
 namespace {
-
-__device__ __forceinline__ f16x2 as_h2(uint32_t v) { return __builtin_bit_cast(f16x2, v); }
-
-// 8 Q4_0 nibbles of one dword -> 8 fp16 values (q - 8) * 2^-12, all exact.  A nibble q
-// masked in place reads as the fp16 subnormal q * 2^-24 (16q * 2^-24 for the high nibble
-// of a byte); one packed FMA scales it by 2^12 (2^8) and subtracts 8 * 2^-12.  That is two
-// VALU ops per pair, as many as an or-in of the exponent 1024 would need with one
-// v_and_or_b32, which the compiler does not form from two literal masks.  The kernels'
-// fp16 denormal mode (float_denorm_mode_16_64 = 3, the default) keeps the subnormals.
-__device__ __forceinline__ f16x8 dq_q4(uint32_t w) {
-  const f16x2 s12 = {(f16)4096.0f, (f16)4096.0f};
-  const f16x2 s8 = {(f16)256.0f, (f16)256.0f};
-  const f16x2 c8 = {(f16)-0.001953125f, (f16)-0.001953125f};  // -8 * 2^-12
-  const uint32_t t = w >> 8;
-  const f16x2 p0 = as_h2(w & 0x000F000Fu) * s12 + c8;
-  const f16x2 p1 = as_h2(w & 0x00F000F0u) * s8 + c8;
-  const f16x2 p2 = as_h2(t & 0x000F000Fu) * s12 + c8;
-  const f16x2 p3 = as_h2(t & 0x00F000F0u) * s8 + c8;
-  return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-}
-
-// 8 Q8_0 int8 values (two dwords) -> 8 exact fp16 integers q.  After the sign flip each
-// byte is q + 128; one v_perm_b32 places bytes 0 and 2 (or 1 and 3) under 0x64 bytes,
-// giving fp16 1024 + q + 128.  Byte selectors 4..7 pick bytes 0..3 of the first
-// operand, 0..3 those of the second.
-__device__ __forceinline__ f16x8 dq_q8(uint32_t w0, uint32_t w1) {
-  const f16x2 c1152 = {(f16)-1152.0f, (f16)-1152.0f};
-  constexpr uint32_t k64 = 0x64646464u, even = 0x00060004u, odd = 0x00070005u;
-  w0 ^= 0x80808080u;
-  w1 ^= 0x80808080u;
-  const f16x2 p0 = as_h2(__builtin_amdgcn_perm(w0, k64, even)) + c1152;
-  const f16x2 p1 = as_h2(__builtin_amdgcn_perm(w0, k64, odd)) + c1152;
-  const f16x2 p2 = as_h2(__builtin_amdgcn_perm(w1, k64, even)) + c1152;
-  const f16x2 p3 = as_h2(__builtin_amdgcn_perm(w1, k64, odd)) + c1152;
-  return f16x8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
-}
 
 // Operand position e (0..7) <- Q4_0 nibble slot nu in the dword: e = 2*(nu%4) + nu/4.
 __device__ __forceinline__ int q4_elem_of_nibble(int nu) { return 2 * (nu & 3) + (nu >> 2); }
@@ -87,26 +51,6 @@ __device__ __forceinline__ int q8_elem_of_byte(int beta) {
 __device__ __forceinline__ int gguf_q4_nib(const uint8_t* blk, int e) {  // element e (0..31) of a block
   const uint8_t byte = blk[2 + (e & 15)];
   return (e < 16) ? (byte & 15) : (byte >> 4);
-}
-
-// Row formats (per-row scale and zero point) reuse the tile layout of the block
-// format with the same code width: 4-bit codes sit like Q4_0 nibbles, 8-bit codes
-// like Q8_0 bytes.  Their tiled copy holds no per-block scales; after the codes come
-// fp32 scale[rows] and fp32 offset[rows] (rows padded to a multiple of 16).
-__host__ __device__ constexpr bool is_row_fmt(int fmt) { return fmt == CIR_I4_ROW || fmt == CIR_I8_ROW; }
-__host__ __device__ constexpr int layout_fmt(int fmt) {
-  return (fmt == CIR_Q4_0 || fmt == CIR_I4_ROW) ? CIR_Q4_0 : CIR_Q8_0;
-}
-__host__ __device__ size_t quant_bytes_per_lane(int fmt) { return layout_fmt(fmt) == CIR_Q4_0 ? 16 : 32; }
-
-// Accumulators of a 4-bit layout hold 2^-12 times the dot products (dq_q4's scale); each
-// kernel multiplies them by kAccScale once, when its k range is done.  Scaling by a power
-// of two commutes with every fp32 rounding before it (no value comes near the fp32
-// subnormal range), so the results are the ones integer weights would give.
-template <int FMT> inline constexpr float kAccScale = layout_fmt(FMT) == CIR_Q4_0 ? 4096.f : 1.f;
-__host__ __device__ size_t block_bytes(int fmt) { return fmt == CIR_Q4_0 ? 18 : 34; }
-__host__ __device__ bool valid_fmt(int fmt) {
-  return fmt == CIR_Q4_0 || fmt == CIR_Q8_0 || fmt == CIR_I4_ROW || fmt == CIR_I8_ROW;
 }
 
 // ---------------------------------------------------------------- repack ----
@@ -454,8 +398,6 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 // quad i+1 and releases the slot read for quad i.
 constexpr int kXsRowBytes = 272;  // 128 fp16 + 16 B pad: the 16 rows of a fragment read hit different banks
 
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));  // plain vector: no struct memcpy, stays in VGPRs
-
 template <int MT>
 struct XsChunk {  // this thread's share of one quad of activations
   u32x4 v[MT];
@@ -707,487 +649,6 @@ __global__ __launch_bounds__(256 * KG) void qgemm_xs_kernel(const f16* __restric
 }
 
 // ------------------------------------------------------------------ GEMV -----
-__device__ __forceinline__ uint4 buf16(rsrc_t r, uint32_t voff, uint32_t soff) {
-  const u32x4 v = __builtin_amdgcn_raw_buffer_load_b128(r, voff, soff, 0);
-  return uint4{v.x, v.y, v.z, v.w};
-}
-__device__ __forceinline__ uint2 buf8(rsrc_t r, uint32_t voff, uint32_t soff) {
-  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-  const u32x2 v = __builtin_amdgcn_raw_buffer_load_b64(r, voff, soff, 0);
-  return uint2{v.x, v.y};
-}
-// ------------------------------------------------------------- large m ------
-// m > 32 (qgemm_xl_kernel): a workgroup of 4 wavefronts covers 8 weight tiles (128
-// output columns, 2 per wavefront) and 16*MT activation rows, so each weight tile is
-// read once per 16*MT rows (the m <= 32 kernel reads it once per 32).  A quad of
-// activations (16*MT rows x 128 columns fp16, 4 KiB per 16 rows) goes straight to
-// LDS by buffer DMA (no registers), double-buffered, one barrier per quad.  Chunk g
-// (16 B) of row r sits in slot g ^ (r & 15) of the row's 256 B, so the 16 rows of a
-// fragment read hit 16 different bank groups.  Weights stream through a ring of
-// DW + 1 slots as in the GEMV.  Per tile and quad the blocks are scaled and summed in
-// the m <= 32 kernel's order, so for the same split both give the same bits.
-// EPI 0: fp32 split-k partials part[split][m][n]; EPI 1: SwiGLU over interleaved
-// gate/up tiles (one split), out[m][N/2] in type TO; EPI 2: greedy-head candidates
-// (one split), the best column of each wavefront's 32 and row: value in part, index in
-// act (as int), at [m][blockIdx.x * W + wave], for argmax_cand_kernel.
-// IL: ask the scheduler to interleave one MFMA with five VALU instructions (the block scale FMAs and dequant)
-// instead of its own two-MFMA / eight-FMA order; PF: convert each block scale to fp32 once and scale with plain
-// fp32 FMAs (the compiler otherwise reads the fp16 scale in every v_fma_mix_f32; same values, same bits).  See
-// launch_qgemm_xl for where each pays.
-template <int FMT, int MT, int DW, int EPI = 0, typename TO = float, int W = 4, bool IL = false, bool PF = false>
-__global__ __launch_bounds__(64 * W) void qgemm_xl_kernel(const f16* __restrict__ x, int ldx,
-                                                     const uint8_t* __restrict__ wq, const uint16_t* __restrict__ wd,
-                                                     float* __restrict__ part, int M, int N, int K, int nq,
-                                                     TO* __restrict__ act = nullptr) {
-  static_assert(EPI >= 0 && EPI <= 2, "large-m GEMM epilogues: partials, SwiGLU or argmax candidates");
-  constexpr int NT = 2;
-  // Issue order of the block MFMAs and scale FMAs: pipelined by one block for the greedy head (Qwen2-7B lm_head
-  // at m = 128: 255.3-255.9 -> 245.6-246.2 us, alternated on one box); elsewhere it measured no better (2048-row
-  // gate|up + SwiGLU within noise) or worse (with the interleave hint: config 5's QKV 14.2 -> 15.1 us).
-  constexpr bool kPipe = !is_row_fmt(FMT) && EPI == 2;
-  constexpr int LB = Stage<FMT, NT, 1>::LB;
-  constexpr int kSlot = 16 * MT * 256;  // bytes of one quad of activations
-  __shared__ __align__(16) uint8_t smem0[kSlot];  // two arrays, not one: the compiler then
-  __shared__ __align__(16) uint8_t smem1[kSlot];  // lets reads of one run while DMA fills the other
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
-  const int KQ = K / 128, NTILES = (N + 15) / 16;
-  const int nt0 = (blockIdx.x * W + wave) * NT;
-  const int split = blockIdx.y;
-  const int m0 = blockIdx.z * 16 * MT;
-  const int q0 = split * nq;
-  const int nqs = min(nq, KQ - q0);  // quads of this split (the last may hold fewer)
-
-  // Activation DMA: instruction u (0..XU-1) of wavefront w fills LDS bytes
-  // [(w*XU + u) KiB, +1 KiB) of a slot, 16 B per lane: row r = 4 (w*XU + u) + lane/16,
-  // slot s = lane % 16 holds chunk s ^ (r & 15).  Rows past M re-read row M-1.
-  constexpr int XU = 4 * MT / W;  // KiB of a quad each wavefront brings in
-  static_assert(XU * W == 4 * MT, "the wavefronts split a quad of activations evenly");
-  const rsrc_t rx = make_rsrc(x, (uint32_t)((size_t)M * ldx * 2));
-  uint32_t xoff[XU];
-#pragma unroll
-  for (int u = 0; u < XU; ++u) {
-    const int r = 4 * (wave * XU + u) + (lane >> 4);
-    const int g = (lane & 15) ^ (r & 15);
-    xoff[u] = (uint32_t)min(m0 + r, M - 1) * (uint32_t)ldx * 2u + 16u * g;
-  }
-  auto dma_x = [&](int slot, int Q) __attribute__((always_inline)) {
-    uint8_t* sm = slot ? smem1 : smem0;
-#pragma unroll
-    for (int u = 0; u < XU; ++u)
-      buf16_to_lds(rx, sm + (wave * XU + u) * 1024, xoff[u], 256u * (uint32_t)(q0 + Q));
-  };
-
-  const uint32_t ntiles_total = (uint32_t)NTILES * KQ;
-  const rsrc_t rw = make_rsrc(wq, ntiles_total * 1024u * LB);
-  const rsrc_t rd = make_rsrc(wd, is_row_fmt(FMT) ? 0u : ntiles_total * 128u);
-  uint32_t tb[NT];
-#pragma unroll
-  for (int b = 0; b < NT; ++b) tb[b] = (uint32_t)min(nt0 + b, NTILES - 1) * KQ + q0;
-  const uint32_t vw = (uint32_t)lane * 16u * LB, vd = (uint32_t)li * 8u;
-  struct WS {
-    uint4 w[NT][LB];
-    uint2 d[NT];
-  };
-  constexpr int R = DW + 1;
-  WS ws[R];
-  auto issue = [&](int slot, int idx) __attribute__((always_inline)) {  // quad idx, clamped to the last
-    const uint32_t Q = (uint32_t)min(idx, nqs - 1);
-#pragma unroll
-    for (int b = 0; b < NT; ++b) {
-#pragma unroll
-      for (int c = 0; c < LB; ++c) ws[slot].w[b][c] = buf16(rw, vw + 16u * c, (tb[b] + Q) * 1024u * LB);
-      if constexpr (!is_row_fmt(FMT)) ws[slot].d[b] = buf8(rd, vd, (tb[b] + Q) * 128u);
-    }
-  };
-  auto each = [&]<int C>(auto&& f) __attribute__((always_inline)) {
-    [&]<int... S>(std::integer_sequence<int, S...>) { (f.template operator()<S>(), ...); }(
-        std::make_integer_sequence<int, C>{});
-  };
-
-  f32x4 acc[MT][NT];
-  f32x4 sx[MT];  // row formats: activation sums of this split
-#pragma unroll
-  for (int a = 0; a < MT; ++a) {
-    sx[a] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int b = 0; b < NT; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-  int xo[4];  // swizzled byte offset of chunk 4j + lg in row 16a + li (li & 15 = li)
-#pragma unroll
-  for (int j = 0; j < 4; ++j) xo[j] = li * 256 + (((4 * j + lg) ^ li) << 4);
-
-  auto compute = [&](const WS& st, int xslot) __attribute__((always_inline)) {
-    f16x8 wb[NT][4];
-    float dj[NT][4];
-#pragma unroll
-    for (int b = 0; b < NT; ++b)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if constexpr (layout_fmt(FMT) == CIR_Q4_0) {
-          const uint4 v = st.w[b][0];
-          wb[b][j] = dq_q4((j == 0) ? v.x : (j == 1) ? v.y : (j == 2) ? v.z : v.w);
-        } else {
-          const uint4 v = st.w[b][j >> 1];
-          wb[b][j] = dq_q8((j & 1) ? v.z : v.x, (j & 1) ? v.w : v.y);
-        }
-        if constexpr (!is_row_fmt(FMT)) {
-          const uint32_t dw = (j < 2) ? st.d[b].x : st.d[b].y;
-          dj[b][j] = static_cast<float>(__builtin_bit_cast(f16, (uint16_t)((j & 1) ? (dw >> 16) : (dw & 0xFFFFu))));
-          if constexpr (PF) asm volatile("" : "+v"(dj[b][j]));  // keeps the conversion out of the FMAs
-        }
-      }
-    const uint8_t* xq = xslot ? smem1 : smem0;
-#pragma unroll
-    for (int a = 0; a < MT; ++a) {
-      f16x8 xf[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) xf[j] = *reinterpret_cast<const f16x8*>(xq + a * 4096 + xo[j]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if constexpr (is_row_fmt(FMT)) {
-#pragma unroll
-          for (int b = 0; b < NT; ++b) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[j], wb[b][j], acc[a][b], 0, 0, 0);
-          const f16x8 ones = {1, 1, 1, 1, 1, 1, 1, 1};
-          sx[a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[j], ones, sx[a], 0, 0, 0);
-        } else if constexpr (!kPipe) {
-          f32x4 c[NT];
-#pragma unroll
-          for (int b = 0; b < NT; ++b)
-            c[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[j], wb[b][j], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-          for (int b = 0; b < NT; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[a][b][r] = fmaf(dj[b][j], c[b][r], acc[a][b][r]);
-        }
-      }
-      if constexpr (kPipe) {  // block j+1's MFMAs before block j's scale FMAs; same arithmetic and order
-        f32x4 c[2][NT];
-        auto mf = [&](int j, f32x4 (&cc)[NT]) __attribute__((always_inline)) {
-#pragma unroll
-          for (int b = 0; b < NT; ++b)
-            cc[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[j], wb[b][j], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-        };
-        auto fm = [&](int j, const f32x4 (&cc)[NT]) __attribute__((always_inline)) {
-#pragma unroll
-          for (int b = 0; b < NT; ++b)
-#pragma unroll
-            for (int r = 0; r < 4; ++r) acc[a][b][r] = fmaf(dj[b][j], cc[b][r], acc[a][b][r]);
-        };
-        mf(0, c[0]);
-        mf(1, c[1]);
-        fm(0, c[0]);
-        mf(2, c[0]);
-        fm(1, c[1]);
-        mf(3, c[1]);
-        fm(2, c[0]);
-        fm(3, c[1]);
-      }
-    }
-    if constexpr (IL) {
-#pragma unroll
-      for (int i = 0; i < MT * 4 * NT; ++i) {
-        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);  // one MFMA
-        __builtin_amdgcn_sched_group_barrier(0x002, 5, 0);  // five VALU
-      }
-    }
-  };
-
-  auto barrier = [] { __syncthreads(); };
-  // Prologue: activations of quad 0 (slot 0) and weight stages 0 .. DW-1 in flight.
-  dma_x(0, 0);
-  each.template operator()<DW>([&]<int S>() { issue(S, S); });
-  barrier();  // (the compiler waits for this wavefront's DMA before the barrier)
-  // Stage i: DMA quad i+1 into the other slot, compute quad i, refill the ring, then the
-  // barrier that publishes quad i+1 (and frees slot i & 1).  The wait before the barrier
-  // covers the DMA and the loads issued before it, not the weights issued after it.
-  // An even ring length keeps i even, so each step's slot S & 1 is known at compile time
-  // and the DMA can go out first: the compute reads the other array, which the compiler
-  // does not wait on.  (With one array, or a slot known only at run time, it waits for
-  // the DMA and every load before it; an odd ring would need 2R steps unrolled, which
-  // spilled.)
-  static_assert(R % 2 == 0, "the slot of each step is fixed only for an even ring");
-  int i = 0;
-#pragma nounroll
-  for (; i + R <= nqs; i += R) {
-    each.template operator()<R>([&]<int S>() {
-      dma_x((S + 1) & 1, min(i + S + 1, nqs - 1));
-      compute(ws[S], S & 1);
-      issue((S + DW) % R, i + S + DW);
-      barrier();
-    });
-  }
-  each.template operator()<DW>([&]<int S>() {  // at most DW quads are left, in ring slots 0 .. DW-1 (i even)
-    if (i + S < nqs) {
-      if (i + S + 1 < nqs) dma_x((S + 1) & 1, i + S + 1);
-      compute(ws[S], S & 1);
-      barrier();
-    }
-  });
-  if constexpr (kAccScale<FMT> != 1.f) {
-#pragma unroll
-    for (int a = 0; a < MT; ++a)
-#pragma unroll
-      for (int b = 0; b < NT; ++b) acc[a][b] *= kAccScale<FMT>;
-  }
-
-  if constexpr (is_row_fmt(FMT)) {
-    const float* rscale = reinterpret_cast<const float*>(wd);
-    const float* roff = rscale + (size_t)NTILES * 16;
-#pragma unroll
-    for (int b = 0; b < NT; ++b) {
-      const int n = min(nt0 + b, NTILES - 1) * 16 + li;
-      const float sc = rscale[n], of = roff[n];
-#pragma unroll
-      for (int a = 0; a < MT; ++a)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[a][b][r] = sc * fmaf(of, sx[a][r], acc[a][b][r]);
-    }
-  }
-  if constexpr (EPI == 2) {
-    float* cand_v = part;
-    int* cand_i = reinterpret_cast<int*>(act);
-    const int wv_global = blockIdx.x * W + wave;
-    const int WT = gridDim.x * W;
-#pragma unroll
-    for (int a = 0; a < MT; ++a)
-#pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        float bv = -INFINITY;
-        int bi = 0x7fffffff;
-#pragma unroll
-        for (int b = 0; b < NT; ++b) {
-          const int n = (nt0 + b) * 16 + li;
-          if (nt0 + b < NTILES && n < N) argmax_better(bv, bi, acc[a][b][r], n);
-        }
-        // the 16 lanes of this row group (same lg) hold 16 different columns
-#pragma unroll
-        for (int off = 8; off > 0; off >>= 1) {
-          const float ov = __shfl_xor(bv, off, 64);
-          const int oi = __shfl_xor(bi, off, 64);
-          argmax_better(bv, bi, ov, oi);
-        }
-        const int m = m0 + 16 * a + 4 * lg + r;
-        if (li == 0 && m < M) {
-          cand_v[(size_t)m * WT + wv_global] = bv;
-          cand_i[(size_t)m * WT + wv_global] = bi;
-        }
-      }
-  } else if constexpr (EPI == 1) {
-    const int inter = N / 2;
-    const int col = (nt0 >> 1) * 16 + li;
-    if (nt0 + 1 < NTILES && col < inter) {
-#pragma unroll
-      for (int a = 0; a < MT; ++a)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int m = m0 + 16 * a + 4 * lg + r;
-          const float g = acc[a][0][r], u = acc[a][1][r];
-          if (m < M) act[(size_t)m * inter + col] = static_cast<TO>(as_f32_value((g / (1.0f + expf(-g))) * u));
-        }
-    }
-  } else {
-#pragma unroll
-    for (int a = 0; a < MT; ++a)
-#pragma unroll
-      for (int b = 0; b < NT; ++b) {
-        const int n = (nt0 + b) * 16 + li;
-        if (nt0 + b < NTILES && n < N) {
-#pragma unroll
-          for (int r = 0; r < 4; ++r) {
-            const int m = m0 + 16 * a + 4 * lg + r;
-            if (m < M) part[((size_t)split * M + m) * N + n] = acc[a][b][r];
-          }
-        }
-      }
-  }
-}
-
-// Balanced large m (qgemm_xw_kernel): one workgroup of 4 wavefronts per CU, each
-// workgroup owning a contiguous run of 1..5 tile pairs (gate/up pairs for SwiGLU) and all
-// 16*MT rows of its row block, so the launch is one round over the CUs with every CU's
-// share of the columns within one pair of the mean (the large-m kernel's fixed 128-column
-// groups leave 2 or 3 workgroups per CU).  Per quad the weight codes and scales of the
-// run and the activations all go to LDS by buffer DMA, double-buffered in two separate
-// arrays so the compiler lets the LDS reads of one slot overlap the DMA into the other.
-// Wavefront w computes pair w over all rows and, in a 5-pair run, row tiles w*MT/4 ..
-// (w+1)*MT/4 - 1 of the fifth pair: each dequantized fragment feeds MT (or MT/4) MFMAs,
-// and in 4- and 5-pair runs the four wavefronts have the same MFMA count.  Per tile, quad and block the arithmetic is the
-// large-m kernel's in the same order, so both give the same bits over one split.  The
-// epilogue is the SwiGLU over interleaved gate/up tiles, out[m][N/2] in type TO (one
-// split, the whole of k).  Block formats only.
-constexpr int kXwPairs = 5;
-template <int FMT>
-inline constexpr int kXwTileBytes = 1024 * Stage<FMT, 1, 1>::LB;  // codes of one tile and quad
-// One slot: activations (16*MT rows x 256 B), codes of up to 10 tiles, then 2 KiB of
-// scales (two whole DMA instructions: tiles 0-7 and 8-9, the rest of the second unused).
-template <int FMT, int MT>
-inline constexpr int kXwSlot = 16 * MT * 256 + 2 * kXwPairs * kXwTileBytes<FMT> + 2048;
-
-template <int FMT, int MT, int W>
-__device__ __forceinline__ void xw_dma(uint8_t* slot, rsrc_t rx, rsrc_t rw, rsrc_t rd,
-                                       const uint32_t (&xoff)[4 * MT / W], int wave, int lane, int t0, int ntl, int KQ,
-                                       int Q) {
-  constexpr int TB = kXwTileBytes<FMT>, LB = TB / 1024;
-  constexpr int XB = 16 * MT * 256, XU = 4 * MT / W;
-  // activations: wavefront w brings KiB w*XU .. w*XU+XU-1 of the quad (rows 4 KiB-index + lane/16)
-#pragma unroll
-  for (int u = 0; u < XU; ++u) buf16_to_lds(rx, slot + (wave * XU + u) * 1024, xoff[u], 256u * (uint32_t)Q);
-  // codes: instruction i = tile i / LB, KiB i % LB; wavefront w takes i = w, w + W, ...
-#pragma unroll
-  for (int v = 0; v < (2 * kXwPairs * LB + W - 1) / W; ++v) {
-    const int i = wave + W * v;
-    if (i < ntl * LB) {
-      const int t = i / LB, c = i - t * LB;
-      buf16_to_lds(rw, slot + XB + t * TB + c * 1024, (uint32_t)lane * 16u + 1024u * c,
-                   ((uint32_t)(t0 + t) * KQ + Q) * (uint32_t)TB);
-    }
-  }
-  // scales: 128 B per tile; lane l of wavefront w (w < 2) brings 16 B of tile 8w + l/8
-  // (lanes past the run repeat its last tile into bytes nothing reads)
-  if (wave < 2 && 8 * wave < ntl) {
-    const int t = min(8 * wave + (lane >> 3), ntl - 1);
-    buf16_to_lds(rd, slot + XB + 2 * kXwPairs * TB + wave * 1024,
-                 ((uint32_t)(t0 + t) * KQ + Q) * 128u + 16u * (lane & 7), 0u);
-  }
-}
-
-constexpr int kXwWaves = 4;
-template <int FMT, int MT, typename TO>
-__global__ __launch_bounds__(64 * kXwWaves) void qgemm_xw_kernel(const f16* __restrict__ x, int ldx,
-                                                     const uint8_t* __restrict__ wq, const uint16_t* __restrict__ wd,
-                                                     int M, int N, int K, TO* __restrict__ act) {
-  static_assert(!is_row_fmt(FMT), "block formats only");
-  constexpr int W = kXwWaves;
-  static_assert(MT % W == 0, "the fifth pair's rows split over the wavefronts");
-  constexpr int TB = kXwTileBytes<FMT>, LB = TB / 1024;
-  constexpr int XB = 16 * MT * 256, WB = 2 * kXwPairs * TB, SLOT = kXwSlot<FMT, MT>;
-  constexpr int XU = 4 * MT / W;   // KiB of a quad's activations each wavefront brings in
-  constexpr int MT5 = MT / W;      // row tiles of the fifth pair per wavefront
-  __shared__ __align__(16) uint8_t slot_a[SLOT];
-  __shared__ __align__(16) uint8_t slot_b[SLOT];
-  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
-  const int KQ = K / 128, NTILES = (N + 15) / 16, NP = (NTILES + 1) / 2;
-  const int p0 = (int)((long)blockIdx.x * NP / gridDim.x);
-  const int cnt = (int)((long)(blockIdx.x + 1) * NP / gridDim.x) - p0;  // 1..5 pairs (host-checked)
-  const int t0 = 2 * p0, ntl = min(2 * cnt, NTILES - t0);
-  const int q0 = 0, nqs = KQ;
-  const int m0 = blockIdx.z * 16 * MT;
-
-  const rsrc_t rx = make_rsrc(x, (uint32_t)((size_t)M * ldx * 2));
-  const uint32_t ntiles_total = (uint32_t)NTILES * KQ;
-  const rsrc_t rw = make_rsrc(wq, ntiles_total * (uint32_t)TB);
-  const rsrc_t rd = make_rsrc(wd, ntiles_total * 128u);
-  uint32_t xoff[XU];
-#pragma unroll
-  for (int u = 0; u < XU; ++u) {
-    const int r = 4 * (wave * XU + u) + (lane >> 4);
-    const int g = (lane & 15) ^ (r & 15);
-    xoff[u] = (uint32_t)min(m0 + r, M - 1) * (uint32_t)ldx * 2u + 16u * g;
-  }
-
-  const bool own = wave < cnt;          // pair `wave` of the run, all rows
-  const bool fifth = cnt == kXwPairs;    // pair 4, row tiles wave*MT5 .. of it
-  f32x4 acc[MT][2], acc5[MT5][2];
-#pragma unroll
-  for (int a = 0; a < MT; ++a) acc[a][0] = acc[a][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int a = 0; a < MT5; ++a) acc5[a][0] = acc5[a][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-  int xo[4];
-#pragma unroll
-  for (int j = 0; j < 4; ++j) xo[j] = li * 256 + (((4 * j + lg) ^ li) << 4);
-
-  // One tile pair (local tiles tl, tl+1) over row tiles a0 .. a0+NA-1 of the slot.
-  auto pair_mma = [&]<int NA>(const uint8_t* sl, int tl, int a0, f32x4 (&ac)[NA][2]) __attribute__((always_inline)) {
-    f16x8 wb[2][4];
-    float dj[2][4];
-#pragma unroll
-    for (int b = 0; b < 2; ++b) {
-      const uint8_t* codes = sl + XB + (tl + b) * TB + lane * 16 * LB;
-      const uint2 dd = *reinterpret_cast<const uint2*>(sl + XB + WB + (tl + b) * 128 + li * 8);
-      uint4 v[LB];
-#pragma unroll
-      for (int c = 0; c < LB; ++c) v[c] = *reinterpret_cast<const uint4*>(codes + 16 * c);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if constexpr (layout_fmt(FMT) == CIR_Q4_0) {
-          wb[b][j] = dq_q4((j == 0) ? v[0].x : (j == 1) ? v[0].y : (j == 2) ? v[0].z : v[0].w);
-        } else {
-          const uint4 vv = v[j >> 1];
-          wb[b][j] = dq_q8((j & 1) ? vv.z : vv.x, (j & 1) ? vv.w : vv.y);
-        }
-        const uint32_t dw = (j < 2) ? dd.x : dd.y;
-        dj[b][j] = static_cast<float>(__builtin_bit_cast(f16, (uint16_t)((j & 1) ? (dw >> 16) : (dw & 0xFFFFu))));
-      }
-    }
-#pragma unroll
-    for (int a = 0; a < NA; ++a) {
-      f16x8 xf[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) xf[j] = *reinterpret_cast<const f16x8*>(sl + (a0 + a) * 4096 + xo[j]);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        f32x4 c[2];
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-          c[b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xf[j], wb[b][j], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) ac[a][b][r] = fmaf(dj[b][j], c[b][r], ac[a][b][r]);
-      }
-    }
-  };
-  auto compute = [&](const uint8_t* sl) __attribute__((always_inline)) {
-    if (own) pair_mma.template operator()<MT>(sl, 2 * wave, 0, acc);
-    if (fifth) pair_mma.template operator()<MT5>(sl, 2 * (kXwPairs - 1), wave * MT5, acc5);
-  };
-
-  // Quad i computes from slot i & 1 while quad i+1 comes into the other; the wait for
-  // that DMA and the barrier end the step.
-  xw_dma<FMT, MT, W>(slot_a, rx, rw, rd, xoff, wave, lane, t0, ntl, KQ, q0);
-  __syncthreads();
-  int i = 0;
-#pragma nounroll
-  for (; i + 2 <= nqs; i += 2) {
-    if (i + 1 < nqs) xw_dma<FMT, MT, W>(slot_b, rx, rw, rd, xoff, wave, lane, t0, ntl, KQ, q0 + i + 1);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(slot_a);
-    __syncthreads();
-    if (i + 2 < nqs) xw_dma<FMT, MT, W>(slot_a, rx, rw, rd, xoff, wave, lane, t0, ntl, KQ, q0 + i + 2);
-    __builtin_amdgcn_sched_barrier(0);
-    compute(slot_b);
-    __syncthreads();
-  }
-  if (i < nqs) compute(slot_a);  // an odd count: the last quad sits in slot a
-  if constexpr (kAccScale<FMT> != 1.f) {
-#pragma unroll
-    for (int a = 0; a < MT; ++a) acc[a][0] *= kAccScale<FMT>, acc[a][1] *= kAccScale<FMT>;
-#pragma unroll
-    for (int a = 0; a < MT5; ++a) acc5[a][0] *= kAccScale<FMT>, acc5[a][1] *= kAccScale<FMT>;
-  }
-
-  // SwiGLU of pair p of the run (gate tile t0 + 2p, up tile t0 + 2p + 1) over row tiles a0 .. a0+NA-1.
-  auto store = [&]<int NA>(int p, int a0, const f32x4 (&ac)[NA][2]) __attribute__((always_inline)) {
-    const int nt = t0 + 2 * p;
-    const int inter = N / 2;
-    const int col = (nt >> 1) * 16 + li;
-    if (nt + 1 < NTILES && col < inter) {
-#pragma unroll
-      for (int a = 0; a < NA; ++a)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int m = m0 + 16 * (a0 + a) + 4 * lg + r;
-          const float g = ac[a][0][r], u = ac[a][1][r];
-          if (m < M) act[(size_t)m * inter + col] = static_cast<TO>(as_f32_value((g / (1.0f + expf(-g))) * u));
-        }
-    }
-  };
-  if (own) store.template operator()<MT>(wave, 0, acc);
-  if (fifth) store.template operator()<MT5>(kXwPairs - 1, wave * MT5, acc5);
-}
-
 // m <= 8 (qgemv_kernel): a workgroup of W wavefronts owns W*NT row tiles, and each
 // wavefront streams its own NT tiles over the workgroup's k-range (grid.y splits k)
 // with no barrier inside the loop.  The m activation rows of that k-range are staged
@@ -1518,7 +979,6 @@ bool gemv_fits(int m, int k, int splits) { return m <= 8 && m * ((k / 128) / spl
 struct GemvGeom {
   int waves, tpw;
 };
-constexpr int kCUs = 256;
 // W also keeps the activation staging within 8 chunks per thread.
 GemvGeom gemv_geometry(int m, int n, int k, int splits) {
   const int ntiles = (n + 15) / 16, nq = (k / 128) / splits;
@@ -1746,49 +1206,48 @@ void launch_qgemm_xs(const f16* x, int ldx, const uint8_t* wq, const uint16_t* w
   else go.template operator()<1>();
 }
 
-// Large m: activation rows per workgroup (16 * MT).
-constexpr int xl_mt(int m) { return m <= 64 ? 4 : 8; }
-// The large-m SwiGLU launch (one split, so the column groups alone set the workgroup
-// count; at 32 < m <= 128 it serves the row formats, which the balanced kernel does not
-// take) keeps 64 rows per workgroup up to m = 128: at the Qwen2-7B gate|up (n 37888, 296
-// column groups) 128 rows per workgroup leave 296 workgroups, a second round on 40 CUs,
-// while two 64-row blocks give 592 smaller ones at 3 wavefronts per SIMD (158 VGPRs
-// against 202): 83.2-86.0 us against 90.3-90.9 (Q8_0, m = 128, same box, alternated).
-// The partials launch keeps xl_mt (QKV, n 4608: 19.3 us at 64 rows against 16.4).
-constexpr int xl_mt_swiglu(int m) { return m <= 128 ? 4 : 8; }
+// Workgroups of the large-m kernel before any k-split: groups of 128 columns x blocks of up to 128 rows.
+long xl_groups(int m, int n) { return (long)((n + 127) / 128) * ((m + 127) / 128); }
 
-// Workgroups of the large-m kernel before any k-split: groups of 128 columns x blocks of 16*MT rows.
-long xl_groups(int m, int n) { return (long)((n + 127) / 128) * ((m + 16 * xl_mt(m) - 1) / (16 * xl_mt(m))); }
-
-// m > 32 takes the large-m kernel when n spans at least 36 groups of 128 columns, when
-// its workgroups alone fill the CUs (>= 192: large m), or, where k may be split, when k
-// holds at least 64 quads (the k-split pieces then stay long).  Measured at the Qwen2-7B
-// shapes (Q8_0, m = 64 / 128) against the m <= 32 kernel run over 32-row blocks: QKV
-// (n 4608) 11.0 / 16.9 us against 15.4 / 24.5, gate|up (n 37888) 51.6 / 81.8 against
-// 72.6 / 114.9; down (n 3584, 28 groups, k 18944) at m = 128: 42.3 us over 9 splits
-// against 49.1 / 66.4 for the small kernel at 4 / 2 splits; O (n 3584, k 3584: 28 quads)
-// stays on the small kernel (12.4-12.7 us against 14.6 at 7 splits).  At m = 2048
-// (Llama-3-8B, Q4_0) the large kernel takes down 353.8 -> 287.8 us and O 113.8 -> 95.2.
-// The SwiGLU launch cannot split k (splittable = false).
+// m > 32 takes the large-m kernel when n spans at least 36 groups of 128 columns, when its workgroups alone fill the CUs
+// (>= 192), or, where k may be split, when k holds at least 64 quads, or 16 past 128 rows (the k-split pieces then stay
+// long).  Measured on MI355X (us) against the m <= 32 kernel run over 32-row blocks: Q8_0 at m = 64 / 128 QKV (n 4608)
+// 9.5 / 13.4 against 15.4 / 24.5, down (n 3584, k 18944) at m = 128 34.9 over 9 splits against 66.4; O (n 3584, k 3584:
+// 28 quads) stays on the small kernel there (12.4 against 14.6 at 7 splits) and leaves it at m = 200 (16.4 against 20.5;
+// m = 512 26.3 against 31.9).  The SwiGLU launch cannot split k (splittable = false).
 bool use_xl(int m, int n, int k, bool splittable = true) {
   if (m <= 32) return false;
-  return (n + 127) / 128 >= 36 || xl_groups(m, n) >= 192 || (splittable && k / 128 >= 64);
+  return (n + 127) / 128 >= 36 || xl_groups(m, n) >= 192 || (splittable && k / 128 >= (m > 128 ? 16 : 64));
 }
 
-// Its k-split: as many splits as keep the launch at one round of workgroups over the
-// 256 CUs (down at m = 128: 9 splits, 252 workgroups: 42.3 us against 46.5 at 8 and 43.9
-// at 10), each split at least 4 quads.  The splits need not divide k/128: split s covers
-// quads s * ceil(kq / S) onward, the last one fewer.  The count is then lowered to
-// ceil(kq / len) for that split length len, so the last split is never empty (86 quads
-// at 16 splits would leave split 15 starting past the end; 15 splits of 6 quads do not).
+// The fused SwiGLU (one split) takes it at every 32 < m <= 128, whatever n: its column runs spread over the CUs.
+bool use_xl_swiglu(int m, int n, int k) { return (m > 32 && m <= 128) || use_xl(m, n, k, false); }
+
+// Its k-split; splits need not divide k/128: split s covers quads s * ceil(kq / S) onward, the last one fewer, and S is
+// lowered to ceil(kq / len) for that length so that no split is empty (86 quads at 16 splits would leave split 15
+// starting past the end; 15 splits of 6 quads do not).
+//   * m <= 128: as many splits of at least 4 quads as keep the launch at one round of workgroups over the 256 CUs (down
+//     at m = 128: 9 splits, 252 workgroups: 42.3 us against 46.5 at 8 and 43.9 at 10).
+//   * more rows, projections (n <= 8192): the least estimate over 1..4 splits of rounds over the CUs x (1.18 us per quad
+//     + 3) plus the partials written and read back at 10 TB/s.  A grid of 160 workgroups leaves 96 CUs idle for the whole
+//     of k; 480 of a third of k do not: down (4096 x 14336, Q4_0) at m = 600 136 -> 91 us, QKV (6144 x 4096) at m = 350
+//     43 -> 31.  Wider n (the LM head) keeps one split: its partials are the logits.
 int xl_splits(int m, int n, int k) {
-  const long kq = k / 128;
-  const long by_cus = 256 / xl_groups(m, n), by_len = kq / 4;
-  long s = by_cus < by_len ? by_cus : by_len;
+  const long kq = k / 128, groups = xl_groups(m, n);
+  long s = 1;
+  if (m <= 128) {
+    const long by_cus = kCUs / groups, by_len = kq / 4;
+    s = by_cus < by_len ? by_cus : by_len;
+  } else if (n <= 8192) {
+    double best = 0;
+    for (long c = 1; c <= 4 && (c == 1 || kq / c >= 4); ++c) {
+      const double t = (double)((groups * c + kCUs - 1) / kCUs) * (1.18 * ((kq + c - 1) / c) + 3) + 8e-7 * c * m * n;
+      if (c == 1 || t < best) best = t, s = c;
+    }
+  }
   if (s <= 1) return 1;
   const long len = (kq + s - 1) / s;
-  s = (kq + len - 1) / len;
-  return (int)s;
+  return (int)((kq + len - 1) / len);
 }
 
 // The k-splits a cir_qgemm launch accepts: those dividing k/128, and on the large-m
@@ -1798,85 +1257,6 @@ bool splits_ok(int m, int n, int k, int splits) {
   if (splits < 1 || splits > kq) return false;
   if (kq % splits == 0) return true;
   return use_xl(m, n, k) && (splits - 1) * ((kq + splits - 1) / splits) < kq;
-}
-
-#ifndef CIR_XL_W
-#define CIR_XL_W 4
-#endif
-template <int FMT, int MT, int EPI, typename TO = float>
-void launch_qgemm_xl(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd, float* part, int M, int N, int K,
-                     int splits, hipStream_t s, TO* act = nullptr) {
-  // Ring of DW + 1 = 4 weight stages for both widths: an even ring lets the activation
-  // DMA go out before the compute (the kernel's even-ring path).  Q4_0 at m = 2048 (a
-  // 2048-token prefill): down 301-303 -> 289.9-290.3 us, QKV 147.8-148.2 -> 138.9-140.0
-  // against a 5-stage ring, prefill 46.7-46.8 -> 44.2 ms (6 stages: 44.4-44.7).
-  constexpr int DW = 3;
-  constexpr int W = CIR_XL_W;
-  const int NTILES = (N + 15) / 16;
-  dim3 grid((NTILES + 2 * W - 1) / (2 * W), splits, (M + 16 * MT - 1) / (16 * MT));
-  const int nq = (K / 128 + splits - 1) / splits;
-  // Q8_0 partials in one round of workgroups (decode at m <= 128) take the interleave hint: at config 5 (m = 128)
-  // QKV 15.7 -> 14.6-14.8 us, down 41.7 -> 38.8-39.0.  Where the workgroups outnumber the CUs (prefill) its extra
-  // registers cost occupancy (Q8_0 m = 2048: QKV 120.3 -> 130.8 us), and Q4_0's lighter dequant gains nothing.
-  if constexpr (FMT == CIR_Q8_0 && EPI == 0) {
-    if ((long)grid.x * grid.y * grid.z <= kCUs) {
-      qgemm_xl_kernel<FMT, MT, DW, EPI, TO, W, true><<<grid, 64 * W, 0, s>>>(x, ldx, wq, wd, part, M, N, K, nq, act);
-      return;
-    }
-  }
-  // Launches of more workgroups than CUs (prefill sizes) convert the scales once (PF): at m = 2048 (Q4_0) gate|up +
-  // SwiGLU 568 -> 536 us, QKV 150 -> 142, O 98 -> 94, down 288 -> 282; a 2048-token prefill 43.7 -> 42.2 ms.
-  // Together with the interleave hint it measured slower (config 5's Q8_0 QKV 14.3 -> 16.2 us), and in the
-  // m <= 32 kernel and the GEMV too (batch-1 step 1.749 -> 1.771 ms).
-  if constexpr (!is_row_fmt(FMT)) {
-    if ((long)grid.x * grid.y * grid.z > kCUs) {
-      qgemm_xl_kernel<FMT, MT, DW, EPI, TO, W, false, true><<<grid, 64 * W, 0, s>>>(x, ldx, wq, wd, part, M, N, K, nq, act);
-      return;
-    }
-  }
-  qgemm_xl_kernel<FMT, MT, DW, EPI, TO, W><<<grid, 64 * W, 0, s>>>(x, ldx, wq, wd, part, M, N, K, nq, act);
-}
-
-// The fused greedy head on the large-m kernel (one split): 128 columns per workgroup, one
-// candidate per wavefront and row, as many as argmax_cand_count gives the m > 16 kernel.
-// At the Qwen2-7B head (n 152064, k 3584, Q8_0) it reads the weights once per 16*MT rows
-// where the m <= 32 kernel reads them once per 32: 495.6 us at m = 128 for the latter
-// against 268.6 us for the large-m kernel's logits alone.
-template <int FMT, int MT>
-void launch_qgemm_xl_argmax(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd, float* cand_v, int* cand_i,
-                            int64_t* ids, int M, int N, int K, hipStream_t s) {
-  constexpr int DW = 3;  // as in launch_qgemm_xl
-  constexpr int W = CIR_XL_W;
-  static_assert(2 * 16 * W == 128, "argmax_cand_count assumes 128 columns per workgroup");
-  const int NTILES = (N + 15) / 16;
-  dim3 grid((NTILES + 2 * W - 1) / (2 * W), 1, (M + 16 * MT - 1) / (16 * MT));
-  qgemm_xl_kernel<FMT, MT, DW, 2, float, W>
-      <<<grid, 64 * W, 0, s>>>(x, ldx, wq, wd, cand_v, M, N, K, K / 128, reinterpret_cast<float*>(cand_i));
-  argmax_cand_kernel<<<M, 256, 0, s>>>(cand_v, cand_i, (int)grid.x * W, M, ids);
-}
-
-// The balanced large-m kernel's workgroups: one per CU while the tile pairs allow
-// (1..5 pairs each), more only when the pairs exceed 5 per CU.
-int xw_workgroups(int n) {
-  const int np = ((n + 15) / 16 + 1) / 2;
-  const int need = (np + kXwPairs - 1) / kXwPairs;
-  const int one_round = np < kCUs ? np : kCUs;
-  return need > one_round ? need : one_round;
-}
-
-// The fused SwiGLU at 32 < m <= 128 (block formats) runs the balanced kernel, 4 wavefronts
-// (8, two per pair, measured no faster).  At the Qwen2-7B gate|up (Q8_0, 12 weight copies
-// rotated): m = 128 78.6-81.0 us against 81.4-85.5 for the large-m kernel in 64-row
-// blocks (64-row blocks of the balanced kernel: 84.9), m = 64 49.2-51.0 against 54.5-56.4.
-// The gain is less than the per-CU bytes suggest (1.5 MB against 2.8 MB on the busiest
-// CU): with one workgroup per CU the quads' DMA and compute alternate more than overlap.
-bool use_xw_swiglu(int m) { return m > 32 && m <= 128; }
-
-template <int FMT, int MT, typename TO>
-void launch_qgemm_xw_swiglu(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd, TO* act, int M, int N, int K,
-                            hipStream_t s) {
-  dim3 grid(xw_workgroups(N), 1, (M + 16 * MT - 1) / (16 * MT));
-  qgemm_xw_kernel<FMT, MT, TO><<<grid, 64 * kXwWaves, 0, s>>>(x, ldx, wq, wd, M, N, K, act);
 }
 
 // Workgroup rows: 4 wavefronts x NT tiles x 16.  m <= 16 takes NT = 1 (64 rows per
@@ -1907,8 +1287,7 @@ void dispatch_qgemm(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd
   if (gemv_fits(M, K, splits)) launch_qgemv<FMT, 0>(x, ldx, wq, wd, part, M, N, K, splits, s);
   else if (M <= 16) launch_qgemm_xs<FMT, 1, 1, 4>(x, ldx, wq, wd, part, M, N, K, splits, s);
   else if (!use_xl(M, N, K)) launch_qgemm_xs<FMT, 2, 2, CIR_XS_DW>(x, ldx, wq, wd, part, M, N, K, splits, s);
-  else if (M <= 64) launch_qgemm_xl<FMT, 4, 0>(x, ldx, wq, wd, part, M, N, K, splits, s);
-  else launch_qgemm_xl<FMT, 8, 0>(x, ldx, wq, wd, part, M, N, K, splits, s);
+  else launch_qgemm_xl<FMT>(x, ldx, wq, wd, part, M, N, K, splits, s);
 }
 
 }  // namespace
@@ -2057,24 +1436,8 @@ extern "C" int cir_qgemm_swiglu(const void* x, int ldx, const void* w_tiled, int
   const f16* xh = static_cast<const f16*>(x);
   hipStream_t s = as_stream(stream);
   auto go = [&]<int FMT>() {
-    if constexpr (!is_row_fmt(FMT)) {
-      if (use_xw_swiglu(m)) {
-        auto xw = [&]<int MT>() {
-          if (odt == CIR_F16) launch_qgemm_xw_swiglu<FMT, MT, f16>(xh, ldx, q, d, static_cast<f16*>(out), m, n, k, s);
-          else launch_qgemm_xw_swiglu<FMT, MT, float>(xh, ldx, q, d, static_cast<float*>(out), m, n, k, s);
-        };
-        if (m <= 64) xw.template operator()<4>();
-        else xw.template operator()<8>();
-        return;
-      }
-    }
-    if (use_xl(m, n, k, false)) {
-      auto xl = [&]<int MT>() {
-        if (odt == CIR_F16) launch_qgemm_xl<FMT, MT, 1, f16>(xh, ldx, q, d, nullptr, m, n, k, 1, s, static_cast<f16*>(out));
-        else launch_qgemm_xl<FMT, MT, 1, float>(xh, ldx, q, d, nullptr, m, n, k, 1, s, static_cast<float*>(out));
-      };
-      if (xl_mt_swiglu(m) == 4) xl.template operator()<4>();
-      else xl.template operator()<8>();
+    if (use_xl_swiglu(m, n, k)) {
+      launch_qgemm_xl_swiglu<FMT>(xh, ldx, q, d, out, odt, m, n, k, s);
       return;
     }
     if (odt == CIR_F16) {
@@ -2149,8 +1512,8 @@ extern "C" int cir_qgemm_argmax(const void* x, int ldx, const void* w_tiled, int
       }
     }
     if (use_xl(m, n, k, false)) {
-      if (m <= 64) launch_qgemm_xl_argmax<FMT, 4>(xh, ldx, q, d, cv, ci, ids, m, n, k, s);
-      else launch_qgemm_xl_argmax<FMT, 8>(xh, ldx, q, d, cv, ci, ids, m, n, k, s);
+      const int groups = launch_qgemm_xl_argmax<FMT>(xh, ldx, q, d, cv, ci, m, n, k, s);
+      argmax_cand_kernel<<<m, 256, 0, s>>>(cv, ci, groups, m, ids);
     } else if (m <= 16) {
       launch_qgemm_argmax<FMT, 1, 1>(xh, ldx, q, d, cv, ci, ids, m, n, k, s);
     } else {
@@ -2172,18 +1535,19 @@ extern "C" const char* cir_qgemm_plan(int op, int fmt, int m, int n, int k, int 
       if (gemv_fits(m, k, splits)) return "qgemv_kernel";
       if (m <= 16) return "qgemm_xs_kernel<NT=1,MT=1>";
       if (!use_xl(m, n, k)) return "qgemm_xs_kernel<NT=2,MT=2>";
-      return m <= 64 ? "qgemm_xl_kernel<MT=4>" : "qgemm_xl_kernel<MT=8>";
+      return m <= 64 ? "qgemm_xl_kernel<MT=4>" : m <= 96 ? "qgemm_xl_kernel<MT=6>" : "qgemm_xl_kernel<MT=8>";
     case CIR_GEMM_SWIGLU:
-      if (!is_row_fmt(fmt) && use_xw_swiglu(m))
-        return m <= 64 ? "qgemm_xw_kernel<MT=4,EPI=swiglu>" : "qgemm_xw_kernel<MT=8,EPI=swiglu>";
-      if (use_xl(m, n, k, false))
-        return xl_mt_swiglu(m) == 4 ? "qgemm_xl_kernel<MT=4,EPI=swiglu>" : "qgemm_xl_kernel<MT=8,EPI=swiglu>";
+      if (use_xl_swiglu(m, n, k))
+        return m <= 64   ? "qgemm_xl_kernel<MT=4,EPI=swiglu>"
+               : m <= 96 ? "qgemm_xl_kernel<MT=6,EPI=swiglu>"
+                         : "qgemm_xl_kernel<MT=8,EPI=swiglu>";
       return m <= 16 ? "qgemm_xs_kernel<NT=2,MT=1,EPI=swiglu>" : "qgemm_xs_kernel<NT=2,MT=2,EPI=swiglu>";
     case CIR_GEMM_ARGMAX:
       if (gemv_head_fits(fmt, m, k)) return "qgemv_kernel<EPI=argmax>+argmax_cand_kernel";
       if (use_xl(m, n, k, false))
-        return m <= 64 ? "qgemm_xl_kernel<MT=4,EPI=argmax>+argmax_cand_kernel"
-                       : "qgemm_xl_kernel<MT=8,EPI=argmax>+argmax_cand_kernel";
+        return m <= 64   ? "qgemm_xl_kernel<MT=4,EPI=argmax>+argmax_cand_kernel"
+               : m <= 96 ? "qgemm_xl_kernel<MT=6,EPI=argmax>+argmax_cand_kernel"
+                         : "qgemm_xl_kernel<MT=8,EPI=argmax>+argmax_cand_kernel";
       return m <= 16 ? "qgemm_xs_kernel<NT=1,MT=1,EPI=argmax>+argmax_cand_kernel"
                      : "qgemm_xs_kernel<NT=2,MT=2,EPI=argmax>+argmax_cand_kernel";
     case CIR_GEMM_ATTN_MERGE:

@@ -1,0 +1,426 @@
+// Large-m GEMM (qgemm_xl_kernel, m > 32): a workgroup of W wavefronts owns a contiguous run
+// of up to W/H pairs of 16-column weight tiles (gate/up pairs for SwiGLU), 16*MT activation
+// rows and one k-split; H wavefronts share a pair, MT/H row tiles each.
+//   * Activations: a quad (128 columns of k) at a time to LDS by buffer DMA, NS - 1 quads ahead
+//     of the one being multiplied, NS stages, each an array of its own (the compiler then lets
+//     the reads of one run while DMA fills the others), one barrier per quad.
+//   * Weights: each wavefront loads its pair's codes and scales straight to registers, NS quads
+//     ahead, and converts the fragments of block j + 1 between the MFMAs of block j (of the
+//     next quad's block 0 during block 3), so no conversion stands between barrier and MFMA.
+//   * The order of instructions is pinned (see `sweep`): a step issues its two MFMAs, then the
+//     scale FMAs of the step before, and reads the activations of the step seven later.  Left
+//     alone the compiler puts each MFMA's FMAs right behind it with eight wait states between,
+//     and nothing overlaps within a wavefront.
+//   * Two wavefronts per SIMD: one issues a VALU instruction every four cycles at most, two
+//     together one every two, and the MFMAs of one run under the FMAs of the other.
+//   * Exact weights and per-block fp32 scales as in the m <= 32 kernel, the quads and blocks of
+//     a split in order, so a split's partials are the same bits at every m > 16.
+// What bounds it: without the loads the arithmetic alone takes 70-90% of the time, and its
+// parts (MFMA, scale FMAs, conversions) add up even where they overlap in the schedule: a loop
+// of MFMAs alone runs at 1.6 GHz and of MFMAs with FMAs at 1.4-2.0 GHz on this card, so the
+// power they draw sets the pace.  Measured (us, before -> now; before: the compiler's order, the
+// row formats' activation sums repeated by every wavefront, fixed 128-column groups): Q4_0
+// 28672 x 4096 + SwiGLU at m = 77 59.4 -> 38.5, 128 61.1 -> 47.0, 2048 533 -> 522 (922
+// TFLOP/s); Q8_0 37888 x 3584 at 77 66.7 -> 52.0, 128 65.7 -> 63.3, 2048 705 -> 677; int4 rows
+// 28672 x 4096 at 77 39.8 -> 32.5, 2048 741 -> 443; Q4_0 4096 x 14336 at 77 28.6 -> 21.0.
+// EPI 0: fp32 split-k partials part[split][m][n]; EPI 1: SwiGLU over interleaved gate/up tiles
+// (one split), out[m][N/2] in type TO; EPI 2: greedy-head candidates (one split), the best
+// column of each pair and row: value in part, index in act (as int), at [m][run * W/H + pair].
+#include "qgemm.hpp"
+
+namespace cir {
+namespace {
+
+template <int FMT>
+inline constexpr int kXlLB = layout_fmt(FMT) == CIR_Q4_0 ? 1 : 2;  // 16-byte loads of codes per lane, tile and quad
+
+template <int FMT, int MT, int H, int W, int EPI, typename TO>
+__global__ __launch_bounds__(64 * W, 2) void qgemm_xl_kernel(const f16* __restrict__ x, int ldx,
+                                                          const uint8_t* __restrict__ wq,
+                                                          const uint16_t* __restrict__ wd, float* __restrict__ part,
+                                                          TO* __restrict__ act, int M, int N, int K, int nq) {
+  constexpr int LB = kXlLB<FMT>;
+  constexpr bool kRow = is_row_fmt(FMT);
+  constexpr int NA = MT / H;                 // row tiles of a wavefront
+  constexpr int NS = H == 2 ? 3 : 2;         // stages of activations, and of weights in registers
+  constexpr int NI = (4 * MT + W - 1) / W;   // its DMA instructions per quad
+  constexpr int RL = 2 * (LB + (kRow ? 0 : 1));  // its weight loads per quad
+  constexpr int SR = (MT + W - 1) / W;       // row tiles whose sums it takes (row formats)
+  static_assert(MT % H == 0 && (H == 1 || H == 2), "whole row shares");
+  static_assert(NI + 2 * RL < 64, "vmcnt range");
+  __shared__ __align__(16) uint8_t sa[16 * MT * 256];
+  __shared__ __align__(16) uint8_t sb[16 * MT * 256];
+  __shared__ __align__(16) uint8_t sc[NS == 3 ? 16 * MT * 256 : 16];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & 63, li = lane & 15, lg = lane >> 4;
+  const int KQ = K / 128, NTILES = (N + 15) / 16, NP = (NTILES + 1) / 2;
+  const int p0 = (int)((long)blockIdx.x * NP / gridDim.x);
+  const int cnt = (int)((long)(blockIdx.x + 1) * NP / gridDim.x) - p0;  // 1 .. W/H pairs (host-checked)
+  const int split = blockIdx.y, q0 = split * nq;
+  const int nqs = min(nq, KQ - q0);  // quads of this split (the last may hold fewer)
+  const int m0 = blockIdx.z * 16 * MT;
+  const int pw = wave / H;
+  const bool own = pw < cnt;
+  const int nt = 2 * (p0 + min(pw, cnt - 1));  // this wavefront's first tile
+  const int a0 = (wave % H) * NA;               // and row tile
+
+  // Activation DMA: instruction i (0 .. 4*MT-1) fills KiB i of a stage, rows 4i + lane/16; 16-byte chunk g of row r sits
+  // in slot g ^ (r & 15), so the 16 rows of a fragment read hit 16 different slots.  Every wavefront issues NI (past the last: the last again, the same
+  // bytes to the same place), so the waits can count.  Rows past M re-read row M-1.
+  const rsrc_t rx = make_rsrc(x, (uint32_t)((size_t)M * ldx * 2));
+  uint32_t xoff[NI];
+#pragma unroll
+  for (int u = 0; u < NI; ++u) {
+    const int r = 4 * min(wave * NI + u, 4 * MT - 1) + (lane >> 4);
+    xoff[u] = (uint32_t)min(m0 + r, M - 1) * (uint32_t)ldx * 2u + 16u * ((lane & 15) ^ (r & 15));
+  }
+  auto dma = [&](uint8_t* st, int i) __attribute__((always_inline)) {
+    const uint32_t off = 256u * (uint32_t)__builtin_amdgcn_readfirstlane(q0 + i);
+#pragma unroll
+    for (int u = 0; u < NI; ++u) buf16_to_lds(rx, st + min(wave * NI + u, 4 * MT - 1) * 1024, xoff[u], off);
+  };
+
+  // Weight loads of quad i (clamped to the last) into ring slot i % NS.
+  const uint32_t ntiles_total = (uint32_t)NTILES * KQ;
+  const rsrc_t rw = make_rsrc(wq, ntiles_total * 1024u * LB);
+  const rsrc_t rd = make_rsrc(wd, kRow ? 0u : ntiles_total * 128u);
+  const uint32_t vw = (uint32_t)lane * 16u * LB, vd = (uint32_t)li * 8u;
+  uint32_t tb[2];
+#pragma unroll
+  for (int b = 0; b < 2; ++b) tb[b] = (uint32_t)min(nt + b, NTILES - 1) * KQ + q0;
+  struct Raw {
+    uint4 w[2][LB];
+    uint2 d[2];
+  };
+  Raw raw[NS];
+  auto load_w = [&](Raw& o, int i) __attribute__((always_inline)) {
+    const uint32_t q = (uint32_t)__builtin_amdgcn_readfirstlane(min(i, nqs - 1));
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+      for (int c = 0; c < LB; ++c) o.w[b][c] = buf16(rw, vw + 16u * c, (tb[b] + q) * 1024u * LB);
+      if constexpr (!kRow) o.d[b] = buf8(rd, vd, (tb[b] + q) * 128u);
+    }
+  };
+
+  f16x8 wb[2][2];  // [block parity][tile]: converted fragments
+  float dj[2][2];
+  auto convert = [&](const Raw& o, int j, int b) __attribute__((always_inline)) {
+    if constexpr (layout_fmt(FMT) == CIR_Q4_0) {
+      const uint4 v = o.w[b][0];
+      wb[j & 1][b] = dq_q4((j == 0) ? v.x : (j == 1) ? v.y : (j == 2) ? v.z : v.w);
+    } else {
+      const uint4 v = o.w[b][j >> 1];
+      wb[j & 1][b] = dq_q8((j & 1) ? v.z : v.x, (j & 1) ? v.w : v.y);
+    }
+    if constexpr (!kRow) {
+      const uint32_t dw = (j < 2) ? o.d[b].x : o.d[b].y;
+      dj[j & 1][b] = as_f32_value(
+          static_cast<float>(__builtin_bit_cast(f16, (uint16_t)((j & 1) ? (dw >> 16) : (dw & 0xFFFFu)))));
+    }
+  };
+
+  f32x4 acc[NA][2], c[2][2], sx[SR];
+#pragma unroll
+  for (int a = 0; a < SR; ++a) sx[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int a = 0; a < NA; ++a) acc[a][0] = acc[a][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+  int xo[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) xo[j] = a0 * 4096 + li * 256 + (((4 * j + lg) ^ li) << 4);
+
+  // One quad from stage `st`: step t = (block t / NA, row tile t % NA).  `cur` holds its codes, `next` the next quad's.
+  constexpr int T = 4 * NA, R = 8;  // steps; activation fragments in registers (LDS latency ~240 cycles)
+  auto sweep = [&](const uint8_t* st, const Raw& cur, const Raw& next) __attribute__((always_inline)) {
+    f16x8 xr[R];
+    auto read_x = [&](int t) __attribute__((always_inline)) {
+      xr[t % R] = *reinterpret_cast<const f16x8*>(st + (t % NA) * 4096 + xo[t / NA]);
+    };
+    auto fmas = [&](int t) __attribute__((always_inline)) {
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          acc[t % NA][b][r] = fmaf(dj[(t / NA) & 1][b], c[t & 1][b][r], acc[t % NA][b][r]);
+    };
+#pragma unroll
+    for (int t = 0; t < R - 1; ++t)
+      if (t < T) read_x(t);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      const int j = t / NA, a = t % NA;
+      if (t + R - 1 < T) read_x(t + R - 1);
+#pragma unroll
+      for (int b = 0; b < 2; ++b) {
+        if constexpr (kRow) acc[a][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xr[t % R], wb[j & 1][b], acc[a][b], 0, 0, 0);
+        else c[t & 1][b] = __builtin_amdgcn_mfma_f32_16x16x32_f16(xr[t % R], wb[j & 1][b], f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      if constexpr (!kRow) {
+        if (t > 0) fmas(t - 1);
+      }
+      // fragments of the next block, one tile in each of two steps (the block before used that set; its last FMAs, which
+      // read its scales, went out in step a = 0)
+      if (a == 1 || (a == 2 && NA > 2)) {
+#pragma unroll
+        for (int b = 0; b < 2; ++b)
+          if (NA == 2 || b == a - 1) j < 3 ? convert(cur, j + 1, b) : convert(next, 0, b);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (!kRow) fmas(T - 1);
+  };
+  static_assert(NA >= 2, "a block's last scale FMAs go out in the next block's first step, before its set is rewritten");
+  // Row formats: the activation sums of row tiles wave * SR .. (the MFMA against ones leaves each row's sum in the
+  // accumulators' layout).
+  auto row_sum = [&](const uint8_t* st) __attribute__((always_inline)) {
+    const f16x8 ones = {1, 1, 1, 1, 1, 1, 1, 1};
+#pragma unroll
+    for (int a = 0; a < SR; ++a)
+      if (wave * SR + a < MT) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          sx[a] = __builtin_amdgcn_mfma_f32_16x16x32_f16(
+              *reinterpret_cast<const f16x8*>(st + (wave * SR + a - a0) * 4096 + xo[j]), ones, sx[a], 0, 0, 0);
+      }
+  };
+
+  // Wait until at most N of this wavefront's loads are in flight, then for every wavefront (the builtin, so the
+  // compiler counts it and adds no wait of its own before the reads).
+  auto arrive = [&]<int V>() __attribute__((always_inline)) {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt((V & 15) | 0x70 | ((V >> 4) << 14));  // vmcnt(V), lgkmcnt(0)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  // Quad i: its activations are in `cur`; quad i + NS - 1's go to `far`, which quad i - 1 has left; quad i + NS's weights
+  // replace quad i's.
+  auto multiply = [&]<int S>(const uint8_t* cur, int i) __attribute__((always_inline)) {
+    __builtin_amdgcn_sched_barrier(0);
+    if (own) sweep(cur, raw[S], raw[(S + 1) % NS]);
+    if constexpr (kRow) row_sum(cur);
+    load_w(raw[S], i + NS);
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // Newer than quad i's activations: NS - 1 quads' weight loads and NS - 2 quads' DMA.
+  constexpr int kNewer = (NS - 2) * NI + (NS - 1) * RL;
+  auto step = [&]<int S>(const uint8_t* cur, uint8_t* far, int i) __attribute__((always_inline)) {
+    arrive.template operator()<kNewer>();
+    dma(far, i + NS - 1);
+    multiply.template operator()<S>(cur, i);
+  };
+  load_w(raw[0], 0);
+  dma(sa, 0);
+  load_w(raw[1], 1);
+  if constexpr (NS == 3) {
+    dma(sb, min(1, nqs - 1));
+    load_w(raw[2], 2);
+  }
+#pragma unroll
+  for (int b = 0; b < 2; ++b) convert(raw[0], 0, b);
+  int i = 0;
+  // Rounds of NS whole steps, then the last quads with shorter waits: with conditions inside the steps instead, the
+  // compiler counts waits for paths that skip an issue and drains the DMA before every read.
+  if constexpr (NS == 3) {
+#pragma nounroll
+    for (; i + 4 < nqs; i += 3) {  // uniform
+      step.template operator()<0>(sa, sc, i);
+      step.template operator()<1>(sb, sa, i + 1);
+      step.template operator()<2>(sc, sb, i + 2);
+    }
+    const int left = nqs - i;  // 1 .. 4; quads i and i + 1 are on their way to sa and sb
+    arrive.template operator()<kNewer>();
+    if (left > 2) dma(sc, i + 2);
+    multiply.template operator()<0>(sa, i);
+    if (left > 1) {
+      arrive.template operator()<2 * RL>();
+      if (left > 3) dma(sa, i + 3);
+      multiply.template operator()<1>(sb, i + 1);
+      if (left > 2) {
+        arrive.template operator()<2 * RL>();
+        multiply.template operator()<2>(sc, i + 2);
+        if (left > 3) {
+          arrive.template operator()<2 * RL>();
+          multiply.template operator()<0>(sa, i + 3);
+        }
+      }
+    }
+  } else {
+#pragma nounroll
+    for (; i + 2 < nqs; i += 2) {  // uniform
+      step.template operator()<0>(sa, sb, i);
+      step.template operator()<1>(sb, sa, i + 1);
+    }
+    const int left = nqs - i;  // 1 or 2; quad i is on its way to sa
+    arrive.template operator()<kNewer>();
+    if (left > 1) dma(sb, i + 1);
+    multiply.template operator()<0>(sa, i);
+    if (left > 1) {
+      arrive.template operator()<kNewer>();
+      multiply.template operator()<1>(sb, i + 1);
+    }
+  }
+  if constexpr (kAccScale<FMT> != 1.f) {
+#pragma unroll
+    for (int a = 0; a < NA; ++a) acc[a][0] *= kAccScale<FMT>, acc[a][1] *= kAccScale<FMT>;
+  }
+  if constexpr (kRow) {  // w = (c - zp) * s, so y = s * (sum x c + (c0 - zp) * sum x)
+    float* sums = reinterpret_cast<float*>(sa);
+    arrive.template operator()<0>();  // every read and DMA of sa is over
+#pragma unroll
+    for (int a = 0; a < SR; ++a)
+      if (wave * SR + a < MT && li == 0) *reinterpret_cast<f32x4*>(sums + (wave * SR + a) * 16 + 4 * lg) = sx[a];
+    __syncthreads();
+    const float* rscale = reinterpret_cast<const float*>(wd);
+    const float* roff = rscale + (size_t)NTILES * 16;
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int n = min(nt + b, NTILES - 1) * 16 + li;
+      const float s = rscale[n], o = roff[n];
+#pragma unroll
+      for (int a = 0; a < NA; ++a) {
+        const f32x4 rs = *reinterpret_cast<const f32x4*>(sums + (a0 + a) * 16 + 4 * lg);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[a][b][r] = s * fmaf(o, rs[r], acc[a][b][r]);
+      }
+    }
+  }
+  if constexpr (EPI == 2) {
+    // The best (value, column) of the pair's 32 columns per row; a wavefront without a pair leaves neutral candidates.
+    float* cand_v = part;
+    int* cand_i = reinterpret_cast<int*>(act);
+    const int WT = gridDim.x * (W / H), at = blockIdx.x * (W / H) + pw;
+#pragma unroll
+    for (int a = 0; a < NA; ++a)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        float bv = -INFINITY;
+        int bi = 0x7fffffff;
+#pragma unroll
+        for (int b = 0; b < 2; ++b) {
+          const int n = (nt + b) * 16 + li;
+          if (own && nt + b < NTILES && n < N) argmax_better(bv, bi, acc[a][b][r], n);
+        }
+        // the 16 lanes of this row group (same lg) hold 16 different columns
+#pragma unroll
+        for (int off = 8; off > 0; off >>= 1) {
+          const float ov = __shfl_xor(bv, off, 64);
+          const int oi = __shfl_xor(bi, off, 64);
+          argmax_better(bv, bi, ov, oi);
+        }
+        const int m = m0 + 16 * (a0 + a) + 4 * lg + r;
+        if (li == 0 && m < M) {
+          cand_v[(size_t)m * WT + at] = bv;
+          cand_i[(size_t)m * WT + at] = bi;
+        }
+      }
+    return;
+  }
+  if (!own) return;
+  if constexpr (EPI == 1) {
+    const int inter = N / 2;
+    const int col = (nt >> 1) * 16 + li;
+    if (nt + 1 < NTILES && col < inter) {
+#pragma unroll
+      for (int a = 0; a < NA; ++a)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int m = m0 + 16 * (a0 + a) + 4 * lg + r;
+          const float g = acc[a][0][r], u = acc[a][1][r];
+          if (m < M) act[(size_t)m * inter + col] = static_cast<TO>(as_f32_value((g / (1.0f + expf(-g))) * u));
+        }
+    }
+  } else {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+      const int n = (nt + b) * 16 + li;
+      if (nt + b < NTILES && n < N) {
+#pragma unroll
+        for (int a = 0; a < NA; ++a)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int m = m0 + 16 * (a0 + a) + 4 * lg + r;
+            if (m < M) part[((size_t)split * M + m) * N + n] = acc[a][b][r];
+          }
+      }
+    }
+  }
+}
+
+// Column runs of a one-row-block launch with `splits` k-splits: as many as keep it at one round of workgroups over the
+// 256 CUs, at most one pair each and never more than 5 pairs.
+int xl_runs(int np, int splits) {
+  const int need = (np + 4) / 5;
+  const int round = kCUs / splits < np ? kCUs / splits : np;
+  return need > round ? need : round;
+}
+
+// The geometry of a launch (us measured on MI355X):
+//   * one block of 64, 96 or 128 rows (m <= 128): two wavefronts per pair (H = 2), the columns in runs of at most 5 pairs
+//     over one round of workgroups; 10 wavefronts where a run holds 5 (a fifth pair split over 8 took 10 us more at
+//     Q8_0 gate|up 37888 x 3584, m = 128).  96-row blocks: Q4_0 gate|up 28672 x 4096 at m = 77 37.6 against 46.3.
+//   * more rows in a grid of at most one workgroup per CU: the same, in runs of 4 pairs.
+//   * a larger grid: four wavefronts per workgroup, each a pair over all 128 rows (H = 1), two workgroups per CU: a
+//     converted fragment feeds 8 MFMAs instead of 4 (Q4_0 gate|up at m = 2048 522 against 620, int4 rows 443 against
+//     510; while at m = 512 the 192 workgroups of Q4_0 QKV 6144 x 4096 take 44.6 with eight wavefronts, 50.6 with four).
+template <int FMT, int EPI, typename TO>
+int launch_xl(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd, float* part, TO* act, int M, int N, int K,
+              int splits, hipStream_t s) {
+  const int nq = (K / 128 + splits - 1) / splits;
+  const int np = ((N + 15) / 16 + 1) / 2, groups = (np + 3) / 4;
+  auto go = [&]<int MT, int H, int W>(int runs) {
+    const dim3 grid(runs, splits, (M + 16 * MT - 1) / (16 * MT));
+    qgemm_xl_kernel<FMT, MT, H, W, EPI, TO><<<grid, 64 * W, 0, s>>>(x, ldx, wq, wd, part, act, M, N, K, nq);
+  };
+  if (M > 128 || EPI == 2) {
+    const bool fill = (long)groups * splits * ((M + 127) / 128) > kCUs;
+    if (M > 96 && fill) go.template operator()<8, 1, 4>(groups);
+    else if (M > 96) go.template operator()<8, 2, 8>(groups);
+    else if (M > 64) go.template operator()<6, 2, 8>(groups);
+    else go.template operator()<4, 2, 8>(groups);
+    return 4 * groups;
+  }
+  const int runs = xl_runs(np, splits);
+  auto by_rows = [&]<int W>() {
+    if (M <= 64) go.template operator()<4, 2, W>(runs);
+    else if (M <= 96) go.template operator()<6, 2, W>(runs);
+    else go.template operator()<8, 2, W>(runs);
+  };
+  if (np <= 4 * runs) by_rows.template operator()<8>();
+  else by_rows.template operator()<10>();
+  return 0;
+}
+
+}  // namespace
+
+template <int FMT>
+void launch_qgemm_xl(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd, float* part, int M, int N, int K,
+                     int splits, hipStream_t s) {
+  launch_xl<FMT, 0, float>(x, ldx, wq, wd, part, nullptr, M, N, K, splits, s);
+}
+template <int FMT>
+void launch_qgemm_xl_swiglu(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd, void* act, int odt, int M,
+                            int N, int K, hipStream_t s) {
+  if (odt == CIR_F16) launch_xl<FMT, 1, f16>(x, ldx, wq, wd, nullptr, static_cast<f16*>(act), M, N, K, 1, s);
+  else launch_xl<FMT, 1, float>(x, ldx, wq, wd, nullptr, static_cast<float*>(act), M, N, K, 1, s);
+}
+template <int FMT>
+int launch_qgemm_xl_argmax(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd, float* cand_v, int* cand_i,
+                           int M, int N, int K, hipStream_t s) {
+  return launch_xl<FMT, 2, float>(x, ldx, wq, wd, cand_v, reinterpret_cast<float*>(cand_i), M, N, K, 1, s);
+}
+#define CIR_XL(F)                                                                                                  \
+  template void launch_qgemm_xl<F>(const f16*, int, const uint8_t*, const uint16_t*, float*, int, int, int, int,   \
+                                   hipStream_t);                                                                   \
+  template void launch_qgemm_xl_swiglu<F>(const f16*, int, const uint8_t*, const uint16_t*, void*, int, int, int,  \
+                                          int, hipStream_t);                                                       \
+  template int launch_qgemm_xl_argmax<F>(const f16*, int, const uint8_t*, const uint16_t*, float*, int*, int, int, \
+                                         int, hipStream_t);
+CIR_XL(CIR_Q4_0)
+CIR_XL(CIR_Q8_0)
+CIR_XL(CIR_I4_ROW)
+CIR_XL(CIR_I8_ROW)
+#undef CIR_XL
+
+}  // namespace cir

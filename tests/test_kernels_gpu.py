@@ -535,6 +535,54 @@ def test_qgemm_planner_random_shapes_row_formats(device, seed):
     assert np.array_equal(ids[clear], ref64.argmax(axis=1)[clear])
 
 
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "int4", "int8"])
+@pytest.mark.parametrize("m,n,k,splits", [
+    (33, 4623, 128, 1),      # 64-row blocks, one quad, a ragged last tile; runs of one pair
+    (65, 33000, 384, 1),     # 96-row blocks; runs of five pairs (10 wavefronts), three quads
+    (96, 32768, 640, 2),     # the last size of 96-row blocks; splits of three and two quads
+    (128, 4608, 1280, 3),    # 128-row blocks; splits of four quads, the last two
+    (129, 4500, 896, 2),     # two row blocks, one workgroup per CU: 8 wavefronts, seven quads in four and three
+    (300, 18000, 768, 1),    # past one workgroup per CU: four wavefronts over all 128 rows, six quads
+    (520, 8192, 2048, 4),    # the same over k-splits of four quads
+])
+def test_qgemm_large_m_geometries(device, fmt, m, n, k, splits):
+    """Every launch geometry of the large-m kernel, at the edges of its row blocks, column runs and quad pipeline, each
+    split's partials against float64 on the kernel's own dequantized weights.  Bound: products and scales are exact in
+    fp32, so only the order of the sums rounds; row formats sum codes and the activations' sum apart, so their terms
+    are bounded by the codes' and the offset's magnitudes instead of their difference."""
+    from cacheir_amd import hip, kernels
+
+    g = torch.Generator(device=device)
+    g.manual_seed(m + n + k)
+    rand = lambda *s: torch.randn(s, generator=g, device=device)
+    if fmt in kernels.FMT_NAMES:
+        code = kernels.FMT_NAMES[fmt]
+        d = (rand(n, k // 32) * 0.01).half().view(torch.uint8).view(n, k // 32, 2)
+        q = torch.randint(0, 256, (n, k // 32, kernels.BLOCK_BYTES[code] - 2), generator=g, device=device)
+        w = kernels.QWeight.from_blocks(torch.cat([d, q.to(torch.uint8)], dim=2).reshape(-1), code, n, k)
+    else:
+        bits = int(fmt[3:])
+        q = torch.randint(0, 256, (n, k * bits // 8), generator=g, device=device).to(torch.uint8)
+        zp = torch.randint(0, 1 << bits, (n,), generator=g, device=device).to(torch.int32)
+        scale = rand(n).abs() * 0.01
+        w = kernels.QWeight.from_rows(q, scale, zp, bits, n, k)
+        code = w.fmt
+    assert kernels.gemm_plan(hip.GEMM_PARTIALS, code, m, n, k, splits).startswith("qgemm_xl_kernel")
+    x = rand(m, k).half()
+    part = kernels.qgemm_partial(x, w, splits=splits)
+    w64, x64, per = kernels.dequant_tiled(w).double(), x.double(), -(-(k // 128) // splits)
+    for s in range(splits):
+        cols = slice(128 * s * per, 128 * min(k // 128, (s + 1) * per))
+        xs, ws = x64[:, cols], w64[:, cols]
+        if fmt in kernels.FMT_NAMES:
+            size = xs.abs() @ ws.abs().T
+        else:
+            size = xs.abs().sum(1, keepdim=True) * (scale.double() * (1 << bits) * 1.5)
+        assert bool(((part[s].double() - xs @ ws.T).abs() <= 1e-5 * size + 1e-6).all()), s
+    ids = kernels.qgemm_argmax(x, w)
+    assert torch.equal(ids, kernels.qgemm_partial(x, w, splits=1)[0].argmax(dim=1))
+
+
 @pytest.mark.parametrize("m,n,k,splits", [
     (1, 5, 4, 1),        # one column group short of a tile, a single 4-column group of k
     (17, 33, 252, 1),    # rows, columns and k one past (or short of) a tile, the last piece ragged
