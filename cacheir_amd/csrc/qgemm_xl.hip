@@ -20,9 +20,9 @@
 // of MFMAs alone runs at 1.6 GHz and of MFMAs with FMAs at 1.4-2.0 GHz on this card, so the
 // power they draw sets the pace.  Measured (us, before -> now; before: the compiler's order, the
 // row formats' activation sums repeated by every wavefront, fixed 128-column groups): Q4_0
-// 28672 x 4096 + SwiGLU at m = 77 59.4 -> 38.5, 128 61.1 -> 47.0, 2048 533 -> 522 (922
-// TFLOP/s); Q8_0 37888 x 3584 at 77 66.7 -> 52.0, 128 65.7 -> 63.3, 2048 705 -> 677; int4 rows
-// 28672 x 4096 at 77 39.8 -> 32.5, 2048 741 -> 443; Q4_0 4096 x 14336 at 77 28.6 -> 21.0.
+// 28672 x 4096 + SwiGLU at m = 77 59.4 -> 39.2, 128 61.1 -> 47.5, 2048 533 -> 519 (927
+// TFLOP/s); Q8_0 37888 x 3584 at 77 66.7 -> 51.8, 128 65.7 -> 60.7, 2048 705 -> 674; int4 rows
+// 28672 x 4096 at 77 39.8 -> 32.9, 2048 741 -> 433; Q4_0 4096 x 14336 at 77 28.6 -> 20.8.
 // EPI 0: fp32 split-k partials part[split][m][n]; EPI 1: SwiGLU over interleaved gate/up tiles
 // (one split), out[m][N/2] in type TO; EPI 2: greedy-head candidates (one split), the best
 // column of each pair and row: value in part, index in act (as int), at [m][run * W/H + pair].
@@ -65,8 +65,8 @@ __global__ __launch_bounds__(64 * W, 2) void qgemm_xl_kernel(const f16* __restri
   const int a0 = (wave % H) * NA;               // and row tile
 
   // Activation DMA: instruction i (0 .. 4*MT-1) fills KiB i of a stage, rows 4i + lane/16; 16-byte chunk g of row r sits
-  // in slot g ^ (r & 15), so the 16 rows of a fragment read hit 16 different slots.  Every wavefront issues NI (past the last: the last again, the same
-  // bytes to the same place), so the waits can count.  Rows past M re-read row M-1.
+  // in slot g ^ (r & 15), so the 16 rows of a fragment read hit 16 different slots.  Every wavefront issues NI (past the
+  // last: the last again, the same bytes to the same place), so the waits can count.  Rows past M re-read row M-1.
   const rsrc_t rx = make_rsrc(x, (uint32_t)((size_t)M * ldx * 2));
   uint32_t xoff[NI];
 #pragma unroll
@@ -75,7 +75,7 @@ __global__ __launch_bounds__(64 * W, 2) void qgemm_xl_kernel(const f16* __restri
     xoff[u] = (uint32_t)min(m0 + r, M - 1) * (uint32_t)ldx * 2u + 16u * ((lane & 15) ^ (r & 15));
   }
   auto dma = [&](uint8_t* st, int i) __attribute__((always_inline)) {
-    const uint32_t off = 256u * (uint32_t)__builtin_amdgcn_readfirstlane(q0 + i);
+    const uint32_t off = 256u * (uint32_t)__builtin_amdgcn_readfirstlane(q0 + min(i, nqs - 1));
 #pragma unroll
     for (int u = 0; u < NI; ++u) buf16_to_lds(rx, st + min(wave * NI + u, 4 * MT - 1) * 1024, xoff[u], off);
   };
@@ -194,71 +194,71 @@ __global__ __launch_bounds__(64 * W, 2) void qgemm_xl_kernel(const f16* __restri
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
-  // Quad i: its activations are in `cur`; quad i + NS - 1's go to `far`, which quad i - 1 has left; quad i + NS's weights
-  // replace quad i's.
-  auto multiply = [&]<int S>(const uint8_t* cur, int i) __attribute__((always_inline)) {
+  auto pin = []() __attribute__((always_inline)) { __builtin_amdgcn_sched_barrier(0); };
+  auto multiply = [&]<int S>(const uint8_t* cur) __attribute__((always_inline)) {
     __builtin_amdgcn_sched_barrier(0);
     if (own) sweep(cur, raw[S], raw[(S + 1) % NS]);
     if constexpr (kRow) row_sum(cur);
-    load_w(raw[S], i + NS);
-    __builtin_amdgcn_sched_barrier(0);
   };
-  // Newer than quad i's activations: NS - 1 quads' weight loads and NS - 2 quads' DMA.
+  // Quad i: its activations are in `cur`; quad i + NS - 1's go to `far`, which quad i - 1 has left; quad i + NS's weights
+  // replace quad i's.  Newer than quad i's activations: NS - 1 quads' weight loads and NS - 2 quads' DMA.  The waits may
+  // count the weight loads because the loop carries them: a load that nothing reads is dropped, and a wait that counts
+  // it lets the DMA it is there for stay in flight.
   constexpr int kNewer = (NS - 2) * NI + (NS - 1) * RL;
   auto step = [&]<int S>(const uint8_t* cur, uint8_t* far, int i) __attribute__((always_inline)) {
     arrive.template operator()<kNewer>();
     dma(far, i + NS - 1);
-    multiply.template operator()<S>(cur, i);
+    multiply.template operator()<S>(cur);
+    load_w(raw[S], i + NS);
+    pin();
   };
   load_w(raw[0], 0);
+  pin();
   dma(sa, 0);
+  pin();
   load_w(raw[1], 1);
+  pin();
   if constexpr (NS == 3) {
-    dma(sb, min(1, nqs - 1));
+    dma(sb, 1);
+    pin();
     load_w(raw[2], 2);
+    pin();
   }
 #pragma unroll
   for (int b = 0; b < 2; ++b) convert(raw[0], 0, b);
   int i = 0;
-  // Rounds of NS whole steps, then the last quads with shorter waits: with conditions inside the steps instead, the
-  // compiler counts waits for paths that skip an issue and drains the DMA before every read.
+  // Rounds of NS whole steps (past the last quad they load and DMA it again, which nothing uses), then the quads left,
+  // all on their way: no condition stands around an issue in the loop, else the compiler counts waits for paths that
+  // skip it and drains the DMA before every read.  Without a round nothing carries the loads issued above (the compiler
+  // moves some into the loop's way in), so the waits of the quads left count none of them.
+  auto rest = [&]<int V>(int i) __attribute__((always_inline)) {
+    if (i > 0) arrive.template operator()<V>();
+    else arrive.template operator()<0>();
+  };
   if constexpr (NS == 3) {
 #pragma nounroll
-    for (; i + 4 < nqs; i += 3) {  // uniform
+    for (; i + 3 <= nqs; i += 3) {  // uniform
       step.template operator()<0>(sa, sc, i);
       step.template operator()<1>(sb, sa, i + 1);
       step.template operator()<2>(sc, sb, i + 2);
     }
-    const int left = nqs - i;  // 1 .. 4; quads i and i + 1 are on their way to sa and sb
-    arrive.template operator()<kNewer>();
-    if (left > 2) dma(sc, i + 2);
-    multiply.template operator()<0>(sa, i);
-    if (left > 1) {
-      arrive.template operator()<2 * RL>();
-      if (left > 3) dma(sa, i + 3);
-      multiply.template operator()<1>(sb, i + 1);
-      if (left > 2) {
-        arrive.template operator()<2 * RL>();
-        multiply.template operator()<2>(sc, i + 2);
-        if (left > 3) {
-          arrive.template operator()<2 * RL>();
-          multiply.template operator()<0>(sa, i + 3);
-        }
+    if (i < nqs) {
+      rest.template operator()<kNewer>(i);
+      multiply.template operator()<0>(sa);
+      if (i + 1 < nqs) {
+        rest.template operator()<RL>(i);  // newer: the weights of quad i + 2
+        multiply.template operator()<1>(sb);
       }
     }
   } else {
 #pragma nounroll
-    for (; i + 2 < nqs; i += 2) {  // uniform
+    for (; i + 2 <= nqs; i += 2) {
       step.template operator()<0>(sa, sb, i);
       step.template operator()<1>(sb, sa, i + 1);
     }
-    const int left = nqs - i;  // 1 or 2; quad i is on its way to sa
-    arrive.template operator()<kNewer>();
-    if (left > 1) dma(sb, i + 1);
-    multiply.template operator()<0>(sa, i);
-    if (left > 1) {
-      arrive.template operator()<kNewer>();
-      multiply.template operator()<1>(sb, i + 1);
+    if (i < nqs) {
+      rest.template operator()<kNewer>(i);
+      multiply.template operator()<0>(sa);
     }
   }
   if constexpr (kAccScale<FMT> != 1.f) {
