@@ -737,7 +737,7 @@ def main() -> int:
                                   "arithmetic_intensity": round(flop5 / bytes5, 1),
                                   "mfma_tflops": round(tflops5, 1), "mfma_peak": MFMA_F16_PEAK_TFLOPS,
                                   "mfma_frac": round(tflops5 / MFMA_F16_PEAK_TFLOPS, 4),
-                                  "counters": measured_counters(COUNTERS_FILE, "xw")},
+                                  "counters": measured_counters(COUNTERS_FILE, "xl")},
         "step_bytes": {"weights": weight_bytes, "kv": kv_bytes * cfg.num_layers,
                        "hbm_floor_ms": round((weight_bytes + kv_bytes * cfg.num_layers) / HBM_PEAK_GBS / 1e6, 4)},
         "decode_batch1": {"ms_per_step": round(ms_b1, 4), "tokens_per_s": round(1000.0 / ms_b1, 2),
