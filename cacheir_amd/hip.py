@@ -114,8 +114,11 @@ def ptr(t: torch.Tensor | None) -> int | None:
 
 
 def stream_handle(stream: torch.cuda.Stream | None = None) -> int:
-    s = stream if stream is not None else torch.cuda.current_stream()
-    return s.cuda_stream
+    if stream is not None:
+        return stream.cuda_stream
+    # the current stream's handle as torch keeps it, 0.3 us; current_stream() builds a Stream object for it, 2.8 us of
+    # the 12 of a launch (a 48-token prompt of the tiny model, 22 launches: 273 -> 219 us)
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
 
 
 def call(name: str, *args) -> None:

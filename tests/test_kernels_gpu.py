@@ -1169,3 +1169,15 @@ def test_stream_read_calibration_runs(device):
         kernels.stream_read(buf, 0, 256, 0, out)
     with pytest.raises(Exception):  # the side buffer must hold a power of two of 16-byte chunks
         kernels.stream_read(buf, 224, 256, 0, out, side=buf[:1000], side_ratio=2)
+
+
+def test_launches_follow_the_current_stream(device):
+    """The handle a launch is given is the current stream's, inside a stream context and after it."""
+    from cacheir_amd import hip
+
+    outer = torch.cuda.current_stream().cuda_stream
+    assert hip.stream_handle() == outer
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        assert hip.stream_handle() == side.cuda_stream == torch.cuda.current_stream().cuda_stream
+    assert hip.stream_handle() == outer and hip.stream_handle(side) == side.cuda_stream
