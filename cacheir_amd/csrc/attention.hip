@@ -1132,12 +1132,14 @@ int device_cus() {
 //     four wavefronts in one group); four in one group again once the grid keeps every CU's two workgroups busy for more than one round
 //     (2 x 2048 tokens: 89.0 against 98.3); 64-vector tiles in four context groups where 128-vector tiles leave half
 //     of the CUs idle (4 x 400 tokens after 1000 at 8/8: 23.5 against 28.9, 100 after 3000: 24.3 against 28.5).
-//   * a grid below one workgroup per CU splits long contexts into pieces of kPfSplitTokens / 2 or more.
+//   * a grid below one workgroup per CU splits long contexts, by the table's capacity, into pieces of about
+//     kPfSplitTokens / 2 (of that capacity: a context that fills half its table is cut twice as fine), if the caller
+//     gave a workspace for the partials (may_split).
 struct PrefillPlan {
   int vec_waves, ctx_waves, tiles, splits;
 };
 constexpr int kPfSplitTokens = 1024;
-PrefillPlan prefill_plan(int batch, int q_len, int Hkv, int G, int max_ctx) {
+PrefillPlan prefill_plan(int batch, int q_len, int Hkv, int G, int max_ctx, bool may_split) {
   const int nvec = q_len * G;
   const long seqs = (long)Hkv * batch, cus = device_cus();
   const long groups4 = (nvec + 4 * kPfVec - 1) / (4 * kPfVec) * seqs;  // workgroups at 128 vectors each
@@ -1146,7 +1148,7 @@ PrefillPlan prefill_plan(int batch, int q_len, int Hkv, int G, int max_ctx) {
   p.vec_waves = (nvec <= 2 * kPfVec || (longctx && 2 * groups4 <= cus)) ? 2 : 4;
   p.ctx_waves = p.vec_waves == 2 ? 4 : (longctx && groups4 < 3 * cus) ? 2 : 1;
   p.tiles = (nvec + kPfVec * p.vec_waves - 1) / (kPfVec * p.vec_waves);
-  p.splits = longctx ? (int)max(1L, min(2L * max_ctx / kPfSplitTokens, cus / (p.tiles * seqs))) : 1;
+  p.splits = longctx && may_split ? (int)max(1L, min(2L * max_ctx / kPfSplitTokens, cus / (p.tiles * seqs))) : 1;
   return p;
 }
 
@@ -1154,7 +1156,7 @@ int launch_attention(const void* q, const void* k_pool, const void* v_pool, cons
                      const int32_t* seq_lens, void* out, void* workspace, size_t workspace_bytes,
                      int batch, int q_len, int Hq, int Hkv, int D, int P, int max_pages, float scale,
                      int kv_dtype, void* stream, QkvIn qkv = QkvIn{nullptr, 0, nullptr, nullptr},
-                     bool merge = true, bool exact_workspace = false) {
+                     bool merge = true, bool exact_workspace = false, bool prefill_splits = false) {
   CIR_CHECK_ARG(batch >= 0 && q_len >= 1, "attention: batch must be >= 0 and q_len >= 1");
   if (batch == 0) return 0;
   CIR_CHECK_ARG((q || qkv.part) && k_pool && v_pool && page_table && seq_lens && out, "attention: null pointer");
@@ -1171,11 +1173,15 @@ int launch_attention(const void* q, const void* k_pool, const void* v_pool, cons
   const bool mfma = mfma_path(kv_dtype, D, P, G);
   const int S = launch_splits(rows, Hkv, max_ctx, mfma);
   // The advertised size (cir_paged_attention_workspace_bytes) covers any split count;
-  // the static-scratch entry point checks the bytes this launch writes instead.
-  const size_t need = exact_workspace ? partial_bytes(rows, Hq, D, S, mfma)
-                                      : cir_paged_attention_workspace_bytes(rows, Hq, D, max_ctx);
-  CIR_CHECK_ARG(workspace && workspace_bytes >= need, "attention: workspace too small (%zu < %zu)", workspace_bytes,
-                need);
+  // the static-scratch and split-prefill entry points check the bytes this launch writes instead.
+  const bool prefill = mfma && q_len > 1;
+  PrefillPlan pl{};
+  if (prefill) pl = prefill_plan(batch, q_len, Hkv, G, max_ctx, prefill_splits);
+  const size_t need = !exact_workspace ? cir_paged_attention_workspace_bytes(rows, Hq, D, max_ctx)
+                      : prefill        ? partial_bytes(rows, Hq, D, pl.splits, mfma)
+                                       : partial_bytes(rows, Hq, D, S, mfma);
+  CIR_CHECK_ARG((workspace || (prefill && need == 0)) && workspace_bytes >= need,
+                "attention: workspace too small (%zu < %zu)", workspace_bytes, need);
   CIR_CHECK_ARG(!qkv.part || (mfma && q_len == 1 && qkv.splits >= 1 && qkv.inv_freq && qkv.positions),
                 "attention: the fused QKV input needs decode (q_len 1), fp16 pools, head_dim 128, page_size %% 16 == 0, "
                 "num_heads/num_kv_heads <= 8 and inv_freq/positions");
@@ -1183,8 +1189,7 @@ int launch_attention(const void* q, const void* k_pool, const void* v_pool, cons
   float* part_o = static_cast<float*>(workspace);
   float* part_ml = part_o + (size_t)rows * Hq * S * D;
   dim3 grid(S, Hkv, rows);
-  if (mfma && q_len > 1) {  // prefill: query tiles over each sequence's blocks
-    const PrefillPlan pl = prefill_plan(batch, q_len, Hkv, G, max_ctx);
+  if (prefill) {  // query tiles over each sequence's blocks
     const dim3 pgrid(Hkv * batch, pl.tiles, pl.splits);
     const auto kernel = pl.ctx_waves == 4   ? attn_prefill_f16_d128<2, 4, 1>
                         : pl.ctx_waves == 2 ? attn_prefill_f16_d128<4, 2, 2>
@@ -1288,6 +1293,27 @@ extern "C" int cir_paged_prefill_attention(const void* q, const void* k_pool, co
   return cir::launch_attention(q, k_pool, v_pool, page_table, seq_lens, out, workspace, workspace_bytes, batch,
                                q_len, num_heads, num_kv_heads, head_dim, page_size, max_pages, scale, kv_dtype,
                                stream);
+}
+
+extern "C" size_t cir_paged_prefill_split_bytes(int batch, int q_len, int num_heads, int num_kv_heads, int head_dim,
+                                                int page_size, int max_pages, int kv_dtype) {
+  if (batch <= 0 || q_len <= 1 || num_heads <= 0 || num_kv_heads <= 0 || page_size <= 0 || max_pages <= 0 ||
+      num_heads % num_kv_heads)
+    return 0;
+  const int G = num_heads / num_kv_heads;
+  if (!cir::mfma_path(kv_dtype, head_dim, page_size, G)) return 0;
+  const cir::PrefillPlan p = cir::prefill_plan(batch, q_len, num_kv_heads, G, max_pages * page_size, true);
+  return cir::partial_bytes(batch * q_len, num_heads, head_dim, p.splits, true);
+}
+
+extern "C" int cir_paged_prefill_attention_split(const void* q, const void* k_pool, const void* v_pool,
+                                                 const int32_t* page_table, const int32_t* seq_lens, void* out,
+                                                 void* workspace, size_t workspace_bytes, int batch, int q_len,
+                                                 int num_heads, int num_kv_heads, int head_dim, int page_size,
+                                                 int max_pages, float scale, int kv_dtype, void* stream) {
+  return cir::launch_attention(q, k_pool, v_pool, page_table, seq_lens, out, workspace, workspace_bytes, batch,
+                               q_len, num_heads, num_kv_heads, head_dim, page_size, max_pages, scale, kv_dtype,
+                               stream, cir::QkvIn{nullptr, 0, nullptr, nullptr}, true, true, true);
 }
 
 extern "C" int cir_paged_decode_attention_qkv(const float* qkv_partial, int splits, const float* inv_freq,

@@ -45,6 +45,9 @@ _SIGNATURES = {
                                                       _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _vp]),
     "cir_paged_prefill_attention": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_size, _c_int, _c_int, _c_int, _c_int,
                                              _c_int, _c_int, _c_int, _c_float, _c_int, _vp]),
+    "cir_paged_prefill_split_bytes": (_c_size, [_c_int] * 8),
+    "cir_paged_prefill_attention_split": (_c_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _c_size, _c_int, _c_int, _c_int,
+                                                   _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _vp]),
     "cir_qweight_tiled_bytes": (_c_size, [_c_int, _c_int, _c_int]),
     "cir_qweight_repack": (_c_int, [_vp, _vp, _c_int, _c_int, _c_int, _vp]),
     "cir_qweight_repack_rows": (_c_int, [_vp, _vp, _vp, _vp, _c_int, _c_int, _c_int, _vp]),

@@ -129,8 +129,12 @@ def paged_decode_attention_qkv(part, inv_freq, positions, k_pool, v_pool, page_t
 
 
 def paged_prefill_attention(q, k_pool, v_pool, page_table, seq_lens, q_len: int, *, scale: float | None = None,
-                            out=None, workspace=None, check_tables: bool = False) -> torch.Tensor:
-    """q ``[B*q_len, Hq, D]``; ``seq_lens`` are lengths after appending the q_len tokens (causal)."""
+                            out=None, workspace=None, check_tables: bool = False,
+                            own_workspace: bool = False) -> torch.Tensor:
+    """q ``[B*q_len, Hq, D]``; ``seq_lens`` are lengths after appending the q_len tokens (causal).  A few queries over
+    a long context run as context splits; their partials go to a buffer of this call, or to ``workspace`` if
+    ``own_workspace`` says that no other launch uses it meanwhile (a workspace is otherwise not written on the fp16
+    head_dim-128 path, so overlapping prefills may share one)."""
     _req(q.dim() == 3 and q_len >= 1 and q.shape[0] % q_len == 0, "q must be [batch*q_len, num_heads, head_dim]")
     rows, num_heads, head_dim = q.shape
     batch = rows // q_len
@@ -138,12 +142,22 @@ def paged_prefill_attention(q, k_pool, v_pool, page_table, seq_lens, q_len: int,
     _req(hd == head_dim and page_table.shape[0] == batch and seq_lens.shape == (batch,), "shape mismatch")
     max_pages = page_table.shape[1]
     out = torch.empty_like(q) if out is None else out
+    code = hip.dtype_code(q.dtype)
     if workspace is None:
         workspace = attention_workspace(rows, num_heads, head_dim, max_pages * psize, q.device)
+        own_workspace = True
+    need = hip.size_call("cir_paged_prefill_split_bytes", batch, q_len, num_heads, kvh, head_dim, psize, max_pages, code)
+    name = "cir_paged_prefill_attention"
+    if need:
+        if not own_workspace:
+            _req(workspace.numel() >= hip.size_call("cir_paged_attention_workspace_bytes", rows, num_heads, head_dim,
+                                                    max_pages * psize), "attention: workspace too small", RuntimeError)
+            workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
+        name = "cir_paged_prefill_attention_split"
     scale = 1.0 / math.sqrt(head_dim) if scale is None else scale
-    hip.call("cir_paged_prefill_attention", q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), page_table.data_ptr(),
-             seq_lens.data_ptr(), out.data_ptr(), workspace.data_ptr(), workspace.numel(), batch, q_len, num_heads, kvh,
-             head_dim, psize, max_pages, float(scale), hip.dtype_code(q.dtype), hip.stream_handle())
+    hip.call(name, q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), page_table.data_ptr(), seq_lens.data_ptr(),
+             out.data_ptr(), workspace.data_ptr(), workspace.numel(), batch, q_len, num_heads, kvh, head_dim, psize,
+             max_pages, float(scale), code, hip.stream_handle())
     return out
 
 

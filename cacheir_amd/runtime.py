@@ -346,7 +346,8 @@ class StepPlan:
                         qv, kp, vp, self.page_table, self.seq_lens, out=ov, workspace=self.attn_ws))
                 else:
                     self.launches.append(lambda qv=qv, ov=ov, kp=kp, vp=vp: kernels.paged_prefill_attention(
-                        qv, kp, vp, self.page_table, self.seq_lens, self.q_len, out=ov, workspace=self.attn_ws))
+                        qv, kp, vp, self.page_table, self.seq_lens, self.q_len, out=ov, workspace=self.attn_ws,
+                        own_workspace=True))
                 rt._count("rocm.paged_attention_decode" if decode else "rocm.paged_attention_prefill")
                 env[outs[0]] = out
             elif op in _MATMUL_OPS:

@@ -126,13 +126,28 @@ int cir_paged_decode_attention_qkv_parts(const float* qkv_partial, int splits, c
  * cacheir/runtime/cpu.py:361-368): q is [batch * q_len, num_heads, head_dim]; row
  * (b, s) attends to tokens t < seq_lens[b] - q_len + s + 1, where seq_lens[b] is the
  * length after the q_len new tokens were appended.  On the fp16 head_dim-128 path
- * (q_len > 1) the workspace is checked but not written: 128 query vectors of a sequence
- * share each K/V block read and the output is written directly. */
+ * (q_len > 1) the workspace is checked but not written: up to 128 query vectors of a
+ * sequence share each K/V block read and the output is written directly. */
 int cir_paged_prefill_attention(const void* q, const void* k_pool, const void* v_pool,
                                 const int32_t* page_table, const int32_t* seq_lens, void* out,
                                 void* workspace, size_t workspace_bytes,
                                 int batch, int q_len, int num_heads, int num_kv_heads, int head_dim,
                                 int page_size, int max_pages, float scale, int kv_dtype, void* stream);
+
+/* The same attention for callers that lend it the workspace for the length of the launch
+ * (two calls that overlap need two workspaces): a few query tiles over a long context then
+ * run as several context splits, whose partials go there.  The workspace holds
+ * cir_paged_prefill_split_bytes(...) bytes on the fp16 head_dim-128 path (q_len > 1; 0: no
+ * splits at these sizes, and it may be NULL), elsewhere
+ * cir_paged_attention_workspace_bytes(batch * q_len, ...), where split_bytes is 0.  At 5
+ * tokens after 5000 (28 / 4 heads) 18 us against 59 unsplit. */
+size_t cir_paged_prefill_split_bytes(int batch, int q_len, int num_heads, int num_kv_heads, int head_dim,
+                                     int page_size, int max_pages, int kv_dtype);
+int cir_paged_prefill_attention_split(const void* q, const void* k_pool, const void* v_pool,
+                                      const int32_t* page_table, const int32_t* seq_lens, void* out,
+                                      void* workspace, size_t workspace_bytes,
+                                      int batch, int q_len, int num_heads, int num_kv_heads, int head_dim,
+                                      int page_size, int max_pages, float scale, int kv_dtype, void* stream);
 
 /* ------------------------------------------------------------ block weights ---
  * GGUF Q4_0 / Q8_0 blocks (cacheir/importers/gguf.py:36,40,273-310) for a weight

@@ -80,6 +80,24 @@ def test_gemm_planner_splits_and_kernels_without_a_gpu():
 
 
 @pytest.mark.skipif(not hip.library_path().exists(), reason="libcacheir_hip.so not built")
+def test_prefill_split_bytes_fit_the_advertised_workspace():
+    """The split prefill's partials (none on the generic path, at q_len 1, or at up to 1024 tokens of table) fit the
+    workspace that cir_paged_attention_workspace_bytes advertises."""
+    size, some = hip.size_call, 0
+    for batch in (1, 3, 32):
+        for q_len in (1, 2, 33, 700):
+            for hq, hkv in ((32, 8), (28, 4), (8, 8), (9, 1)):
+                for pages in (4, 64, 65, 130, 1000):
+                    args = (batch, q_len, hq, hkv, 128, 16, pages)
+                    need = size("cir_paged_prefill_split_bytes", *args, hip.CIR_F16)
+                    assert need <= size("cir_paged_attention_workspace_bytes", batch * q_len, hq, 128, pages * 16), args
+                    assert need == 0 or (q_len > 1 and hq // hkv <= 8 and pages > 64), args
+                    assert size("cir_paged_prefill_split_bytes", *args, hip.CIR_F32) == 0
+                    some += need > 0
+    assert some > 20
+
+
+@pytest.mark.skipif(not hip.library_path().exists(), reason="libcacheir_hip.so not built")
 def test_default_splits_are_always_accepted():
     """Whatever k-split the library proposes for a shape, its own launch accepts (no empty last split): the
     Qwen2.5-3B down (n 2048, k 11008: 86 quads) at m = 64 once got 16 splits, which start split 15 past the end."""

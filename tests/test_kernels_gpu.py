@@ -272,6 +272,41 @@ def test_prefill_attention_paired_tiles(device, q_len, batch):
         close16(out[b * q_len:(b + 1) * q_len], ref)
 
 
+def test_prefill_attention_leaves_a_shared_workspace_alone(device):
+    """Overlapping prefills may share a workspace on the fp16 head_dim-128 path: a call that is not told that the
+    workspace is its own does not write it, at sizes that split the context (9 tokens after 1100: 2 query tiles).  The
+    split call's result (its own buffer, or the workspace if it may) agrees bit for bit with itself and within the
+    storage bound with the oracle and the unsplit C call, which leaves the workspace alone too."""
+    from cacheir_amd import hip, kernels
+
+    rng = np.random.default_rng(17)
+    past, q_len, hq, hkv = 1100, 9, 14, 2
+    kp, vp, pt, lens = paged.build_pool(rng, [past + q_len], hkv, 128, 16)
+    q = rng.standard_normal((q_len, hq, 128)).astype(np.float16)
+    args = [to_dev(a, device) for a in (q, kp, vp, pt, lens)]
+    max_pages = pt.shape[1]
+    ws = kernels.attention_workspace(q_len, hq, 128, max_pages * 16, device)
+    ws.fill_(0xA5)
+    out = kernels.paged_prefill_attention(*args, q_len, workspace=ws)
+    assert bool((ws == 0xA5).all()), "a shared workspace was written"
+    plain = torch.empty_like(out)
+    hip.call("cir_paged_prefill_attention", *(t.data_ptr() for t in (*args, plain, ws)), ws.numel(), 1, q_len, hq, hkv,
+             128, 16, max_pages, 128 ** -0.5, hip.CIR_F16, hip.stream_handle())
+    assert bool((ws == 0xA5).all()), "the unsplit call wrote its workspace"
+    need = hip.size_call("cir_paged_prefill_split_bytes", 1, q_len, hq, hkv, 128, 16, max_pages, hip.CIR_F16)
+    assert 0 < need <= ws.numel()
+    own = kernels.paged_prefill_attention(*args, q_len, workspace=ws, own_workspace=True)
+    assert torch.equal(own, out) and torch.equal(own, kernels.paged_prefill_attention(*args, q_len))
+    assert not bool((ws[:need] == 0xA5).all()) and bool((ws[need:] == 0xA5).all())
+    with pytest.raises(RuntimeError, match="workspace too small"):
+        kernels.paged_prefill_attention(*args, q_len, workspace=ws[:1024])
+    kh = paged.gather_sequence(kp, pt[0], past + q_len).astype(np.float32)[None]
+    vh = paged.gather_sequence(vp, pt[0], past + q_len).astype(np.float32)[None]
+    ref = ops.attention(q.astype(np.float32)[None], kh, vh, hq, hkv, 128, causal=True).reshape(q_len, hq, 128)
+    close16(out.float().cpu().numpy(), ref)
+    close16(plain.float().cpu().numpy(), ref)
+
+
 # -------------------------------------------------------------- block weights --
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
 def test_dequant_bit_exact(device, fmt):
