@@ -316,21 +316,24 @@ __device__ __forceinline__ void row_sums(const f16x8 (&x)[MT][4], f32x4 (&sx)[MT
 }
 
 // Dense fp32 (the reference's unquantized artifacts): y = x W^T on the fp32 MFMA 16x16x4, whose products and sums are
-// fp32.  A workgroup of four wavefronts owns 16 output columns and 16 * MT rows and shares out k: wavefront w takes
-// the 64-column pieces w, w + 4, ... of the split, loads a piece's operands (16 bytes a lane, 256 contiguous bytes a
-// row) before the first product, and the four sums meet in LDS.  Lane 16g + r holds columns
-// 4g .. 4g + 3 of 16-column step u for row r of either operand, so MFMA e of a step covers columns 4g + e: a fixed
-// permutation of k, the same for both.  Every step (and at MT = 1 every MFMA of it) of a piece has an accumulator of its
-// own, added pairwise at the end, so a sum's chain stays as short as the lanes-then-tree order of the plain kernel below
-// (one accumulator: 1.3-1.6 times its error).  Launches of these sizes are bound by latency (one load round trip per piece);
-// the tiny model's 48-row products (k 256, n 256 - 1376) took 53-72 us one wavefront per column with the rows in turn.
-template <int MT>
-__global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restrict__ x, int ldx,
-                                                            const float* __restrict__ w, float* __restrict__ part,
-                                                            int M, int N, int K, int kc) {
-  constexpr int U = 4;                // 16-column steps per piece
-  constexpr int E = MT == 1 ? 4 : 1;  // accumulators per step
-  __shared__ f32x4 red[3][MT][64];
+// fp32.  A workgroup owns 16 output columns and 16 * MT rows and shares out k in 64-column pieces: wavefront w takes every
+// fourth piece from w / UW on and of it 4 / UW of the 16-column steps (16 bytes a lane), all loaded before the first
+// product, and the sums meet in LDS.  Lane 16g + r holds columns 4g .. 4g + 3 of a step for row r of either operand, so
+// MFMA e of a step covers columns 4g + e: a fixed permutation of k, the same for both.  Every MFMA of a piece has an
+// accumulator of its own, added in one tree, so a sum is 64 chains of k / 64 products at any m, as many as in the plain
+// kernel below, and a row has the same bits under every MT and UW.  Error against 64 bits (rms of the difference over the
+// result's, n 256): 2.7 * 2^-24 at k = 4096 and 4.9 * 2^-24 at 16384, as the plain kernel's; with one accumulator per step
+// (16 chains, four times as long) 4.9 and 9.7.  Launches of these sizes are bound by latency (one load round trip per
+// piece); the tiny model's 48-row products (k 256, n 256 - 1376) took 53-72 us one wavefront per column with the rows in
+// turn, 3.0-3.8 here.  UW = 4 keeps four times the loads in flight: one row of 4096 x 4096 15.0 us (17.3 at UW = 2, 29.4 at
+// UW = 1; the plain kernel 25.9), of 4096 x 14336 35.8 (73.3).
+template <int MT, int UW>
+__global__ __launch_bounds__(256 * UW) void gemm_f32_mfma_kernel(const float* __restrict__ x, int ldx,
+                                                                 const float* __restrict__ w, float* __restrict__ part,
+                                                                 int M, int N, int K, int kc) {
+  constexpr int U = 4 / UW;  // 16-column steps per wavefront and piece
+  constexpr int E = 4;       // accumulators per step: one per MFMA of it
+  __shared__ f32x4 red[4 * UW - 1][MT][64];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
   const int li = lane & 15, lg = lane >> 4;
   const int n = blockIdx.x * 16 + li, m0 = blockIdx.z * 16 * MT;
@@ -340,12 +343,15 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
   const float* xr[MT];
 #pragma unroll
   for (int a = 0; a < MT; ++a) xr[a] = x + (size_t)min(m0 + 16 * a + li, M - 1) * ldx;
-  f32x4 part_acc[U * E][MT];
+  f32x4 acc[U][E][MT];
 #pragma unroll
-  for (int i = 0; i < U * E; ++i)
+  for (int u = 0; u < U; ++u)
 #pragma unroll
-    for (int a = 0; a < MT; ++a) part_acc[i][a] = f32x4{0.f, 0.f, 0.f, 0.f};
-  for (int kb = k0 + 16 * U * wave; kb < k1; kb += 64 * U) {
+    for (int e = 0; e < E; ++e)
+#pragma unroll
+      for (int a = 0; a < MT; ++a) acc[u][e][a] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // wavefront wave: piece wave / UW of every four, steps (wave % UW) * U ..
+  for (int kb = k0 + 16 * U * wave; kb < k1; kb += 256) {
     f32x4 wv[U], xv[U][MT];
 #pragma unroll
     for (int u = 0; u < U; ++u) {
@@ -364,34 +370,56 @@ __global__ __launch_bounds__(256) void gemm_f32_mfma_kernel(const float* __restr
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int e = 0; e < 4; ++e)
+      for (int e = 0; e < E; ++e)
 #pragma unroll
         for (int a = 0; a < MT; ++a)
-          part_acc[u * E + e % E][a] =
-              __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u][a][e], wv[u][e], part_acc[u * E + e % E][a], 0, 0, 0);
+          acc[u][e][a] = __builtin_amdgcn_mfma_f32_16x16x4f32(xv[u][a][e], wv[u][e], acc[u][e][a], 0, 0, 0);
   }
+  // The tree, the same for every UW: the MFMAs of a step, the steps of a piece, the pieces.
+  f32x4 sum[U][MT];
 #pragma unroll
-  for (int half = U * E / 2; half > 0; half /= 2)
+  for (int a = 0; a < MT; ++a) {
 #pragma unroll
-    for (int i = 0; i < half; ++i)
+    for (int u = 0; u < U; ++u) sum[u][a] = (acc[u][0][a] + acc[u][2][a]) + (acc[u][1][a] + acc[u][3][a]);
 #pragma unroll
-      for (int a = 0; a < MT; ++a) part_acc[i][a] += part_acc[i + half][a];
-  f32x4(&acc)[MT] = part_acc[0];
+    for (int step = 1; step < U; step *= 2)
+#pragma unroll
+      for (int u = 0; u + step < U; u += 2 * step) sum[u][a] += sum[u + step][a];
+  }
   if (wave > 0) {
 #pragma unroll
-    for (int a = 0; a < MT; ++a) red[wave - 1][a][lane] = acc[a];
+    for (int a = 0; a < MT; ++a) red[wave - 1][a][lane] = sum[0][a];
   }
   __syncthreads();
   if (wave > 0 || n >= N) return;
 #pragma unroll
   for (int a = 0; a < MT; ++a) {
-    acc[a] = (acc[a] + red[0][a][lane]) + (red[1][a][lane] + red[2][a][lane]);
+    f32x4 t[4 * UW];
+    t[0] = sum[0][a];
+#pragma unroll
+    for (int i = 1; i < 4 * UW; ++i) t[i] = red[i - 1][a][lane];
+#pragma unroll
+    for (int step = 1; step < 4 * UW; step *= 2)
+#pragma unroll
+      for (int i = 0; i < 4 * UW; i += 2 * step) t[i] += t[i + step];
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int m = m0 + 16 * a + 4 * lg + r;
-      if (m < M) part[((size_t)split * M + m) * N + n] = acc[a][r];
+      if (m < M) part[((size_t)split * M + m) * N + n] = t[0][r];
     }
   }
+}
+
+// 16-row tiles per workgroup: the least count of rounds over the CUs times a round's cost (MT = 2 takes 1.42 times and
+// MT = 4 2.5 times a round of MT = 1: 2048 x 2048 in one round 9.6, 13.5 and 21.9 us).  Us at MT = 1, 2, 4: 4096 x 4096 at
+// m = 64 63 / 50 / 44, at 65 71 / 61 / 70, at 512 451 / 343 / 307; 2048 x 2048 at m = 32 9.7 / 13.5, at 96 23.8 / 24.3 /
+// 21.9; 768 x 3072 at 128 23.7 / 19.0 / 30.2.  Short k pays MT = 4's longer start: 1024 x 256 at 2048 rows 33 / 31 / 36.
+int gemm_f32_rows(int m, int n, int kc, int splits) {
+  const long cols = (long)((n + 15) / 16) * splits;
+  auto cost = [&](int mt, double c) { return c * ((cols * ((m + 16 * mt - 1) / (16 * mt)) + kCUs - 1) / kCUs); };
+  const double t1 = cost(1, 1.0), t2 = cost(2, 1.42), t4 = kc >= 2048 ? cost(4, 2.5) : t2;
+  if (t4 < t2 && t4 < t1) return 4;
+  return t2 < t1 ? 2 : 1;
 }
 
 // The same for rows that are not whole aligned 16-byte groups: one wavefront per output column, lanes over k, the m
@@ -1490,14 +1518,24 @@ extern "C" int cir_gemm_f32(const float* x, int ldx, const float* w, float* y_pa
   CIR_CHECK_ARG(x && w && y_partial, "gemm_f32: null pointer");
   const int kc = (k + splits - 1) / splits;
   hipStream_t s = as_stream(stream);
-  // 16-byte operand loads: every row and every split must start on 16 bytes.  Up to 64 rows a workgroup takes 16 of
-  // them (the grid is short); more rows go 64 at a time, so each weight column is read a quarter as often.
+  // 16-byte operand loads: every row and every split must start on 16 bytes.
   if (k % 4 == 0 && ldx % 4 == 0 && kc % 4 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
       reinterpret_cast<uintptr_t>(w) % 16 == 0 && (m + 15) / 16 <= 65535) {
-    if (m <= 64)
-      gemm_f32_mfma_kernel<1><<<dim3((n + 15) / 16, splits, (m + 15) / 16), 256, 0, s>>>(x, ldx, w, y_partial, m, n, k, kc);
-    else
-      gemm_f32_mfma_kernel<4><<<dim3((n + 15) / 16, splits, (m + 63) / 64), 256, 0, s>>>(x, ldx, w, y_partial, m, n, k, kc);
+    auto go = [&]<int MT, int UW>() {
+      gemm_f32_mfma_kernel<MT, UW><<<dim3((n + 15) / 16, splits, (m + 16 * MT - 1) / (16 * MT)), 256 * UW, 0, s>>>(
+          x, ldx, w, y_partial, m, n, k, kc);
+    };
+    switch (gemm_f32_rows(m, n, kc, splits)) {
+      case 1:
+        if (kc <= 256) go.template operator()<1, 2>();  // one piece per wavefront either way: 2.45 against 2.50 us
+        else go.template operator()<1, 4>();
+        break;
+      case 2:
+        if (kc <= 256) go.template operator()<2, 1>();  // fewer partials to meet: 1376 x 256 at 2048 rows 39.2 against 42.7
+        else go.template operator()<2, 4>();
+        break;
+      default: go.template operator()<4, 2>();
+    }
     return launch_status();
   }
   dim3 grid((n + 3) / 4, splits);

@@ -621,9 +621,10 @@ def test_qgemm_large_m_geometries(device, fmt, m, n, k, splits):
 @pytest.mark.parametrize("m,n,k,splits", [
     (1, 5, 4, 1),        # one column group short of a tile, a single 4-column group of k
     (17, 33, 252, 1),    # rows, columns and k one past (or short of) a tile, the last piece ragged
-    (64, 688, 688, 4),   # the last size of the 16-row kernel; splits of 172 columns
-    (65, 31, 260, 1),    # the first size of the 64-row kernel
-    (130, 16, 1028, 2),  # 64-row blocks with a ragged last one; splits of 514 columns: not whole 16-byte groups
+    (64, 688, 688, 4),   # splits of 172 columns
+    (65, 31, 260, 1),    # two to a wavefront's pieces, the last one ragged
+    (130, 16, 1028, 2),  # a ragged last block; splits of 514 columns: not whole 16-byte groups
+    (130, 16, 1032, 2),  # the same at splits of 516
     (3, 20, 30, 1),      # k not a multiple of 4: the one-column-per-wavefront kernel
 ])
 def test_gemm_f32_shapes(device, m, n, k, splits):
@@ -638,6 +639,39 @@ def test_gemm_f32_shapes(device, m, n, k, splits):
     x64, w64 = x.astype(np.float64), w.astype(np.float64)
     bound = (k + splits) * np.finfo(np.float32).eps / 2 * (np.abs(x64) @ np.abs(w64).T)
     assert np.all(np.abs(got - x64 @ w64.T) <= bound)
+
+
+@pytest.mark.parametrize("m", [1, 2, 64, 65, 130])
+@pytest.mark.parametrize("k", [4096, 16384])
+def test_gemm_f32_chains_stay_short(device, m, k):
+    """The rounding error of dense fp32 products is that of 64 chains of k / 64 products and a tree, at every row count.
+    A partial sum of i random products has rms sqrt(i) and rounds with a relative rms of 0.42 * 2^-24, so a chain of c
+    adds c^2 / 2 of its square and the k / c chains together 0.42 * 2^-24 * sqrt(c / 2) of the result's rms; the tree
+    adds one rounding a level.  1.3 times that: 16 chains would stand at 1.9 times, one at 7 times and more."""
+    from cacheir_amd import kernels
+
+    g = torch.Generator(device=device)
+    g.manual_seed(m + k)
+    x, w = torch.randn(m, k, generator=g, device=device), torch.randn(512, k, generator=g, device=device)
+    ref = x.double() @ w.double().T
+    err = (kernels.gemm_f32_partial(x, w)[0].double() - ref).pow(2).mean().sqrt() / ref.pow(2).mean().sqrt()
+    assert err.item() <= 1.3 * 0.42 * 2.0 ** -24 * (k / 128 + 6) ** 0.5
+
+
+@pytest.mark.parametrize("n,k", [(4096, 252), (4097, 2052), (300, 1000)])
+def test_gemm_f32_rows_do_not_depend_on_the_batch(device, n, k):
+    """A row of a dense fp32 product has the same bits in every batch: one row, 17 and 130 rows, and 528 (16, 32 and 64
+    rows per workgroup, the last only from k = 2048 on), each with a ragged last tile of columns or piece of k."""
+    from cacheir_amd import kernels
+
+    g = torch.Generator(device=device)
+    g.manual_seed(n)
+    x, w = torch.randn(528, k, generator=g, device=device), torch.randn(n, k, generator=g, device=device)
+    full = kernels.gemm_f32_partial(x, w)[0]
+    for m in (1, 17, 130):
+        assert torch.equal(kernels.gemm_f32_partial(x[:m].contiguous(), w)[0], full[:m]), m
+    assert bool(((full.double() - x.double() @ w.double().T).abs()
+                 <= (k + 1) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)).all())
 
 
 @pytest.mark.parametrize("d,g,psize,dtype,past,q_len", [
