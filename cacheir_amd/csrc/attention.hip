@@ -686,6 +686,7 @@ __global__ __launch_bounds__(64 * VW * CW, 2) void attn_prefill_f16_d128(
   }
 
   const float one = as_f32_value(1.f);
+  bool huge = false;             // uniform: some query's |m| is 2^24 or more
   float m = -INFINITY, l = 0.f;  // query l32: running max (both lanes of the query), this lane's share of the sum
   f32x16 acc[D / 32];            // O[query l32][32 dt + 8 j + 4 h + e], element 4 j + e
 #pragma unroll
@@ -749,17 +750,29 @@ __global__ __launch_bounds__(64 * VW * CW, 2) void attn_prefill_f16_d128(
       const float alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
       l *= alpha;
       m = mn;
+      huge = __builtin_amdgcn_ballot_w64(fabsf(m) >= 0x1p24f && m != -INFINITY) != 0;
 #pragma unroll
       for (int dt = 0; dt < D / 32; ++dt) acc[dt] *= alpha;
     }
-    const float ms = m == -INFINITY ? 0.f : m;
+    // p = exp2(c sc - m) by one FMA.  m is the rounded product, so the largest p is 2^r with r the rounding error of
+    // m, up to half an ulp: a factor that all p of the query share, until p leaves fp16.  From |m| = 2^24 on (r up to
+    // one) the difference is taken of the rounded products instead, which makes it exactly zero at the maximum.
+    float ms = m == -INFINITY ? 0.f : m, pc = sc;
+    if (__builtin_expect(huge, 0)) {
+#pragma unroll
+      for (int j = 0; j < NB; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) c[j][r] = as_f32_value(c[j][r] * sc) - ms;
+      ms = 0.f;
+      pc = 1.f;
+    }
 #pragma unroll
     for (int j = 0; j < NB; ++j) {
       float ps = 0.f;
       f16x8 pa[2];
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        pa[r >> 3][r & 7] = static_cast<f16>(__builtin_amdgcn_exp2f(fmaf(c[j][r], sc, -ms)));
+        pa[r >> 3][r & 7] = static_cast<f16>(__builtin_amdgcn_exp2f(fmaf(c[j][r], pc, -ms)));
         // l sums the rounded p; the multiply by one (opaque) makes it one v_fma_mix_f32 reading the fp16 value
         ps = fmaf(static_cast<float>(pa[r >> 3][r & 7]), one, ps);
       }

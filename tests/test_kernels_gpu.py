@@ -272,6 +272,39 @@ def test_prefill_attention_paired_tiles(device, q_len, batch):
         close16(out[b * q_len:(b + 1) * q_len], ref)
 
 
+@pytest.mark.parametrize("batch,g,hkv,q_len,past", [
+    (1, 4, 2, 9, 1100),   # 64-vector tiles in four context groups, context splits
+    (2, 8, 8, 140, 1000), # two context groups
+    (3, 2, 2, 70, 30),    # one group
+])
+@pytest.mark.parametrize("scale", [128 ** -0.5, -2.0])
+def test_prefill_attention_huge_scores(device, batch, g, hkv, q_len, past, scale):
+    """Scores of 1e8 and more (q and k of the size of fp16's largest values), where half an ulp of the maximum is more
+    than fp16 holds as an exponent: every query still picks its largest score.  All but the maximum underflow (the
+    scores are far apart), so the output is the V row of the largest exact score."""
+    from cacheir_amd import kernels
+
+    rng = np.random.default_rng(q_len)
+    total = np.array([past + q_len + 5 * b for b in range(batch)])
+    kp, vp, pt, lens = paged.build_pool(rng, total, hkv, 128, 16)
+    kp = np.clip(kp.astype(np.float32) * 14000, -6e4, 6e4).astype(np.float16)
+    hq = g * hkv
+    q = np.clip(rng.standard_normal((batch * q_len, hq, 128)) * 14000, -6e4, 6e4).astype(np.float16)
+    out = kernels.paged_prefill_attention(to_dev(q, device), to_dev(kp, device), to_dev(vp, device), to_dev(pt, device),
+                                          to_dev(lens, device), q_len, scale=scale).cpu().numpy()
+    for b in range(batch):
+        n = int(total[b])
+        kh = np.repeat(paged.gather_sequence(kp, pt[b], n).astype(np.float64), g, axis=1)
+        vh = np.repeat(paged.gather_sequence(vp, pt[b], n), g, axis=1)
+        s = np.einsum("qhd,khd->qhk", q[b * q_len:(b + 1) * q_len].astype(np.float64), kh) * scale
+        s[(np.arange(n)[None] > (n - q_len + np.arange(q_len))[:, None])[:, None].repeat(hq, 1)] = -np.inf
+        top = np.sort(s, axis=-1)[..., -2:]
+        clear = top[..., 1] - top[..., 0] > 1e-5 * np.abs(top[..., 1]) + 64  # fp32 sums tell the two largest apart
+        assert clear.mean() > 0.9
+        want = np.take_along_axis(vh.transpose(1, 0, 2)[None], s.argmax(-1)[..., None, None], axis=2)[:, :, 0]
+        assert np.array_equal(out[b * q_len:(b + 1) * q_len][clear], want[clear])
+
+
 def test_prefill_attention_leaves_a_shared_workspace_alone(device):
     """Overlapping prefills may share a workspace on the fp16 head_dim-128 path: a call that is not told that the
     workspace is its own does not write it, at sizes that split the context (9 tokens after 1100: 2 query tiles).  The
