@@ -938,7 +938,7 @@ __global__ __launch_bounds__(64 * kGenWaves) void attn_chunk_generic(
       const f32x4 t = load_dims<VEC>(q + (head0 + min(h, nh - 1)) * D + (nd ? d0 : 0), nd);
       qv[h] = nd ? t : zero;
       o[h] = zero;
-      m[h] = -INFINITY;
+      m[h] = -FLT_MAX;  // finite: a score of -inf then weighs exp2(-inf) = 0 even where it stands alone
       l[h] = 0.f;
     }
     for (int j0 = wave * TPW; j0 < n; j0 += kGenU * kGenWaves * TPW) {  // uniform; tokens j0 + i * kGenWaves * TPW + grp
@@ -971,7 +971,7 @@ __global__ __launch_bounds__(64 * kGenWaves) void attn_chunk_generic(
         }
         if constexpr (LPT <= 16) mx = fmaxf(mx, __shfl_xor(mx, 16, 64));
         if constexpr (LPT <= 32) mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
-        const float a = exp2f(m[h] - mx);  // finite mx: token j0 of the wavefront exists
+        const float a = exp2f(m[h] - mx);
         l[h] *= a;
         o[h] *= a;
         m[h] = mx;
@@ -1002,26 +1002,26 @@ __global__ __launch_bounds__(64 * kGenWaves) void attn_chunk_generic(
     __syncthreads();
     for (int idx = threadIdx.x; idx < nh * D; idx += 64 * kGenWaves) {
       const int h = idx / D, d = idx - h * D;
-      float M = -INFINITY;
+      float M = sm_m[0][h];
 #pragma unroll
-      for (int w = 0; w < kGenWaves; ++w) M = fmaxf(M, sm_m[w][h]);
+      for (int w = 1; w < kGenWaves; ++w) M = fmaxf(M, sm_m[w][h]);
       float den = 0.f, acc = 0.f;
-      if (M != -INFINITY) {
 #pragma unroll
-        for (int w = 0; w < kGenWaves; ++w) {
-          const float f = exp2f(sm_m[w][h] - M);
-          den = fmaf(sm_l[w][h], f, den);
-          acc = fmaf(sm_o[w][h][d], f, acc);
-        }
+      for (int w = 0; w < kGenWaves; ++w) {
+        const float f = exp2f(sm_m[w][h] - M);
+        den = fmaf(sm_l[w][h], f, den);
+        acc = fmaf(sm_o[w][h][d], f, acc);
       }
+      // No weight at all: no tokens (the output is 0), or scores of -inf alone (NaN, as a softmax over them gives).
+      const bool none = den == 0.f, nan = none && n > 0;
       if (NC == 1) {
-        out[(head0 + h) * D + d] = from_f32<T>(as_f32_value(acc * (den > 0.f ? 1.f / den : 0.f)));
+        out[(head0 + h) * D + d] = from_f32<T>(as_f32_value(acc * (nan ? NAN : none ? 0.f : 1.f / den)));
       } else {
         part_o[((head0 + h) * NC + chunk) * D + d] = acc;
         if (d == 0) {
           float* ml = part_ml + ((head0 + h) * NC + chunk) * 2;
-          ml[0] = M;
-          ml[1] = den;
+          ml[0] = none ? -INFINITY : M;
+          ml[1] = nan ? 1.f : den;
         }
       }
     }
@@ -1034,7 +1034,9 @@ __global__ __launch_bounds__(64 * kGenWaves) void attn_chunk_generic(
 // Latency-bound (a few KiB per workgroup), so no load waits for another: thread s
 // reads split s's (m, l), the weights 2^(m_s - M) go through LDS, and each output
 // element's S partials are loaded 8 at a time before they are summed.  Sums run in
-// split order, as the serial form for S > kMergeFast does.  o * inv is rounded to fp32
+// split order, as the serial form for S > kMergeFast does.  A row whose scores are all
+// -inf (every M -inf, some l > 0: the generic kernel's partials) gives NaN, as a softmax
+// over them does; one without tokens (every l 0) gives 0.  o * inv is rounded to fp32
 // before the fp16 conversion (as_f32_value: no single-rounding mixed-precision multiply),
 // the same two roundings the O projection's merge (qgemm.hip, attn_merged_chunk) makes.
 constexpr int kMergeFast = 128;
@@ -1058,7 +1060,9 @@ __global__ __launch_bounds__(128) void attn_merge(const float* __restrict__ part
     float den = 0.f;
     if (M != -INFINITY)
       for (int s = 0; s < S; ++s) den = fmaf(sl[s], sw[s], den);
-    const float inv = den > 0.f ? 1.f / den : 0.f;
+    float inv = den > 0.f ? 1.f / den : 0.f;
+    if (M == -INFINITY)
+      for (int s = 0; s < S; ++s) inv = sl[s] > 0.f ? NAN : inv;
     const float* po = part_o + ((size_t)row * Hq + head) * S * D;
     for (int d = t; d < D; d += 128) {
       float o = 0.f;
@@ -1079,7 +1083,9 @@ __global__ __launch_bounds__(128) void attn_merge(const float* __restrict__ part
   float den = 0.f;
   if (M != -INFINITY)
     for (int s = 0; s < S; ++s) den = fmaf(ml[2 * s + 1], exp2f(ml[2 * s] - M), den);
-  const float inv = den > 0.f ? 1.f / den : 0.f;
+  float inv = den > 0.f ? 1.f / den : 0.f;
+  if (M == -INFINITY)
+    for (int s = 0; s < S; ++s) inv = ml[2 * s + 1] > 0.f ? NAN : inv;
   const float* po = part_o + ((size_t)row * Hq + head) * S * D;
   for (int d = threadIdx.x; d < D; d += blockDim.x) {
     float o = 0.f;

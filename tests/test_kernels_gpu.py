@@ -674,6 +674,36 @@ def test_gemm_f32_shapes(device, m, n, k, splits):
     assert np.all(np.abs(got - x64 @ w64.T) <= bound)
 
 
+@pytest.mark.parametrize("d,dtype", [(64, np.float32), (64, np.float16), (128, np.float32), (256, np.float16)])
+def test_generic_attention_minus_infinity_scores(device, d, dtype):
+    """A score of -inf (k = -inf, as an overflow leaves it) has weight 0 wherever the token stands: alone in a wavefront
+    (token 4 of 5), a whole 128-token chunk, a whole wavefront's share.  A row whose scores are all -inf gives NaN, as
+    the softmax over them does, in one chunk and in several; an empty row gives 0."""
+    from cacheir_amd import kernels
+
+    rng = np.random.default_rng(d)
+    hkv, g = 2, 3
+    ctx = [5, 140, 300, 5, 300, 0]
+    gone = [[4], list(range(128, 140)), list(range(0, 128)) + [200], range(5), range(300), []]
+    kp, vp, pt, lens = paged.build_pool(rng, ctx, hkv, d, 16, dtype=dtype)
+    for b, toks in enumerate(gone):
+        for t in toks:
+            kp[pt[b, t // 16], :, t % 16, 0] = -np.inf
+    q = rng.standard_normal((len(ctx), g * hkv, d)).astype(dtype)
+    q[:, :, 0] = np.abs(q[:, :, 0]) + 0.5
+    out = kernels.paged_decode_attention(*(to_dev(a, device) for a in (q, kp, vp, pt, lens))).float().cpu().numpy()
+    assert np.isnan(out[3:5]).all() and (out[5] == 0).all()
+    for b in range(3):
+        keep = np.setdiff1d(np.arange(ctx[b]), list(gone[b]))
+        kh = paged.gather_sequence(kp, pt[b], ctx[b])[keep].astype(np.float32)[None]
+        vh = paged.gather_sequence(vp, pt[b], ctx[b])[keep].astype(np.float32)[None]
+        ref = ops.attention(q[b].astype(np.float32)[None, None], kh, vh, g * hkv, hkv, d, causal=False)
+        if dtype == np.float32:
+            np.testing.assert_allclose(out[b], ref.reshape(g * hkv, d), atol=1e-4, rtol=1e-4)
+        else:
+            close16(out[b], ref.reshape(g * hkv, d))
+
+
 @pytest.mark.parametrize("m", [1, 2, 64, 65, 130])
 @pytest.mark.parametrize("k", [4096, 16384])
 def test_gemm_f32_chains_stay_short(device, m, k):
