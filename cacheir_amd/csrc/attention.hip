@@ -776,6 +776,7 @@ __global__ __launch_bounds__(64 * VW * CW, 2) void attn_prefill_f16_d128(
         // l sums the rounded p; the multiply by one (opaque) makes it one v_fma_mix_f32 reading the fp16 value
         ps = fmaf(static_cast<float>(pa[r >> 3][r & 7]), one, ps);
       }
+      if (j > 0 && blk + j >= wblk) break;  // uniform: past the wavefront's last token (p = 0 would meet its values)
       l += ps;
       if (j > 0) load_v(j);
 #pragma unroll

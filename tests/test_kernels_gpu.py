@@ -305,6 +305,37 @@ def test_prefill_attention_huge_scores(device, batch, g, hkv, q_len, past, scale
         assert np.array_equal(out[b * q_len:(b + 1) * q_len][clear], want[clear])
 
 
+@pytest.mark.parametrize("batch,g,hkv,q_len,past,at", [
+    (1, 1, 2, 140, 0, 35),      # one context group: tokens 0-31 share a 64-token step with the infinite one
+    (1, 4, 2, 40, 20, 33),      # the same after 20 tokens, 8 tokens per tile
+    (2, 8, 8, 140, 1000, 1070), # two context groups
+])
+def test_prefill_attention_later_infinities_stay_out(device, batch, g, hkv, q_len, past, at):
+    """A value of infinity (as an overflow leaves it) at a later token does not reach the queries whose tile of 32 query
+    vectors ends in an earlier 32-token block: they agree with the oracle over the finite values."""
+    from cacheir_amd import kernels
+
+    rng = np.random.default_rng(at)
+    total = [past + q_len] * batch
+    kp, vp, pt, lens = paged.build_pool(rng, total, hkv, 128, 16)
+    hq = g * hkv
+    q = rng.standard_normal((batch * q_len, hq, 128)).astype(np.float16)
+    bad = vp.copy()
+    for b in range(batch):
+        bad[pt[b, at // 16], :, at % 16, :] = np.inf
+    out = kernels.paged_prefill_attention(to_dev(q, device), to_dev(kp, device), to_dev(bad, device), to_dev(pt, device),
+                                          to_dev(lens, device), q_len).float().cpu().numpy()
+    last = (np.arange(q_len) * g + g - 1) // 32 * 32 + 31  # the last query vector of a token's (last) tile
+    early = (past + np.minimum(last // g, q_len - 1)) // 32 < at // 32
+    assert early.sum() >= 8
+    for b in range(batch):
+        kh = paged.gather_sequence(kp, pt[b], total[b]).astype(np.float32)[None]
+        vh = paged.gather_sequence(vp, pt[b], total[b]).astype(np.float32)[None]
+        qh = q[b * q_len:(b + 1) * q_len].astype(np.float32)[None]
+        ref = ops.attention(qh, kh, vh, hq, hkv, 128, causal=True).reshape(q_len, hq, 128)
+        close16(out[b * q_len:(b + 1) * q_len][early], ref[early])
+
+
 def test_prefill_attention_leaves_a_shared_workspace_alone(device):
     """Overlapping prefills may share a workspace on the fp16 head_dim-128 path: a call that is not told that the
     workspace is its own does not write it, at sizes that split the context (9 tokens after 1100: 2 query tiles).  The
