@@ -201,9 +201,9 @@ __global__ __launch_bounds__(64 * W, 2) void qgemm_xl_kernel(const f16* __restri
     if constexpr (kRow) row_sum(cur);
   };
   // Quad i: its activations are in `cur`; quad i + NS - 1's go to `far`, which quad i - 1 has left; quad i + NS's weights
-  // replace quad i's.  Newer than quad i's activations: NS - 1 quads' weight loads and NS - 2 quads' DMA.  The waits may
-  // count the weight loads because the loop carries them: a load that nothing reads is dropped, and a wait that counts
-  // it lets the DMA it is there for stay in flight.
+  // replace quad i's.  Newer than quad i's activations: NS - 1 quads' weight loads and NS - 2 quads' DMA.  A load that
+  // nothing reads would be dropped, and a wait that counts it would let the DMA it is there for stay in flight: `hold`
+  // reads the ring slots that no quad does, so whatever the compiler peels or unrolls, each counted load is issued.
   constexpr int kNewer = (NS - 2) * NI + (NS - 1) * RL;
   auto step = [&]<int S>(const uint8_t* cur, uint8_t* far, int i) __attribute__((always_inline)) {
     arrive.template operator()<kNewer>();
@@ -211,6 +211,14 @@ __global__ __launch_bounds__(64 * W, 2) void qgemm_xl_kernel(const f16* __restri
     multiply.template operator()<S>(cur);
     load_w(raw[S], i + NS);
     pin();
+  };
+  auto hold = [](const Raw& o) __attribute__((always_inline)) {
+#pragma unroll
+    for (int b = 0; b < 2; ++b) {
+#pragma unroll
+      for (int c = 0; c < LB; ++c) asm volatile("" ::"v"(o.w[b][c].x), "v"(o.w[b][c].y), "v"(o.w[b][c].z), "v"(o.w[b][c].w));
+      if constexpr (!kRow) asm volatile("" ::"v"(o.d[b].x), "v"(o.d[b].y));
+    }
   };
   load_w(raw[0], 0);
   pin();
@@ -248,8 +256,14 @@ __global__ __launch_bounds__(64 * W, 2) void qgemm_xl_kernel(const f16* __restri
       if (i + 1 < nqs) {
         rest.template operator()<RL>(i);  // newer: the weights of quad i + 2
         multiply.template operator()<1>(sb);
+      } else {
+        hold(raw[1]);
       }
+    } else {
+      hold(raw[0]);
+      hold(raw[1]);
     }
+    hold(raw[2]);
   } else {
 #pragma nounroll
     for (; i + 2 <= nqs; i += 2) {
@@ -259,7 +273,10 @@ __global__ __launch_bounds__(64 * W, 2) void qgemm_xl_kernel(const f16* __restri
     if (i < nqs) {
       rest.template operator()<kNewer>(i);
       multiply.template operator()<0>(sa);
+    } else {
+      hold(raw[0]);
     }
+    hold(raw[1]);
   }
   if constexpr (kAccScale<FMT> != 1.f) {
 #pragma unroll

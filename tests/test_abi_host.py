@@ -125,6 +125,33 @@ def _llvm_tool(name: str):
     return None
 
 
+def _code_objects(tmp_path):
+    """The gfx950 code objects in the built library: .hip_fatbin holds one clang offload bundle per source file."""
+    import struct
+
+    fat = tmp_path / "fatbin.bin"
+    subprocess.run([_llvm_tool("llvm-objcopy"), f"--dump-section=.hip_fatbin={fat}", str(hip.library_path()),
+                    str(tmp_path / "lib_copy.so")], check=True, capture_output=True)
+    data = fat.read_bytes()
+    magic = b"__CLANG_OFFLOAD_BUNDLE__"
+    start = data.find(magic)
+    assert start >= 0, "no offload bundle in .hip_fatbin"
+    while start >= 0:
+        pos = start + len(magic)
+        (entries,) = struct.unpack_from("<Q", data, pos)
+        pos += 8
+        for _ in range(entries):
+            off, size, tlen = struct.unpack_from("<QQQ", data, pos)
+            pos += 24
+            triple = data[pos:pos + tlen].decode()
+            pos += tlen
+            if "gfx950" in triple:
+                obj = tmp_path / f"co{start}.o"
+                obj.write_bytes(data[start + off:start + off + size])
+                yield obj
+        start = data.find(magic, start + 1)
+
+
 @pytest.mark.skipif(not hip.library_path().exists(), reason="libcacheir_hip.so not built")
 @pytest.mark.skipif(_llvm_tool("llvm-objcopy") is None or _llvm_tool("llvm-readelf") is None,
                     reason="LLVM binutils not available")
@@ -134,45 +161,59 @@ def test_no_kernel_spills_to_scratch(tmp_path):
     trip and has cost 1.5x on a kernel here).  Reads the library's own device code: the .hip_fatbin section holds
     one clang offload bundle per source file; each bundle's gfx950 entry is an ELF code object whose notes list
     the kernels."""
-    import struct
-
-    fat = tmp_path / "fatbin.bin"
-    subprocess.run([_llvm_tool("llvm-objcopy"), f"--dump-section=.hip_fatbin={fat}", str(hip.library_path()),
-                    str(tmp_path / "lib_copy.so")], check=True, capture_output=True)
-    data = fat.read_bytes()
-    magic = b"__CLANG_OFFLOAD_BUNDLE__"
-    starts, i = [], data.find(magic)
-    while i >= 0:
-        starts.append(i)
-        i = data.find(magic, i + 1)
-    assert starts, "no offload bundle in .hip_fatbin"
     kernels_seen, spills = 0, []
-    for b, start in enumerate(starts):
-        pos = start + len(magic)
-        (entries,) = struct.unpack_from("<Q", data, pos)
-        pos += 8
-        for _ in range(entries):
-            off, size, tlen = struct.unpack_from("<QQQ", data, pos)
-            pos += 24
-            triple = data[pos:pos + tlen].decode()
-            pos += tlen
-            if "gfx950" not in triple:
-                continue
-            obj = tmp_path / f"co{b}.o"
-            obj.write_bytes(data[start + off:start + off + size])
-            notes = subprocess.run([_llvm_tool("llvm-readelf"), "--notes", str(obj)], check=True,
-                                   capture_output=True, text=True).stdout
-            name = None
-            for line in notes.splitlines():
-                line = line.strip()
-                if line.startswith(".name:"):
-                    name = line.split(":", 1)[1].strip()
-                elif line.startswith(".private_segment_fixed_size:"):
-                    kernels_seen += 1
-                    if int(line.split(":", 1)[1]) != 0:
-                        spills.append((name, int(line.split(":", 1)[1])))
+    for obj in _code_objects(tmp_path):
+        notes = subprocess.run([_llvm_tool("llvm-readelf"), "--notes", str(obj)], check=True,
+                               capture_output=True, text=True).stdout
+        name = None
+        for line in notes.splitlines():
+            line = line.strip()
+            if line.startswith(".name:"):
+                name = line.split(":", 1)[1].strip()
+            elif line.startswith(".private_segment_fixed_size:"):
+                kernels_seen += 1
+                if int(line.split(":", 1)[1]) != 0:
+                    spills.append((name, int(line.split(":", 1)[1])))
     assert kernels_seen >= 100, f"only {kernels_seen} kernels found in the code objects"
     assert not spills, spills[:10]
+
+
+@pytest.mark.skipif(not hip.library_path().exists(), reason="libcacheir_hip.so not built")
+@pytest.mark.skipif(_llvm_tool("llvm-objcopy") is None or _llvm_tool("llvm-objdump") is None,
+                    reason="LLVM binutils not available")
+def test_large_m_kernel_issues_every_load_its_waits_count(tmp_path):
+    """The large-m kernel's barriers wait for all but a fixed number of newer loads, which is safe only if every load
+    counted is issued: a load that the compiler drops lets the activations' DMA it stands behind go on past the barrier.
+    In every instance's code: NS quads of weight loads ahead of the loop and NS in it, 2 NS - 1 of activation DMA, and
+    one barrier with the counted wait per quad of the loop."""
+    seen = 0
+    for obj in _code_objects(tmp_path):
+        names = subprocess.run([_llvm_tool("llvm-readelf"), "-Ws", str(obj)], check=True, capture_output=True,
+                               text=True).stdout
+        if "qgemm_xl_kernel" not in names:
+            continue
+        text = subprocess.run([_llvm_tool("llvm-objdump"), "-d", "--no-show-raw-insn", str(obj)], check=True,
+                              capture_output=True, text=True).stdout
+        for part in re.split(r"^[0-9a-f]+ <", text, flags=re.M)[1:]:
+            name = part.split(">:", 1)[0]
+            t = re.search(r"qgemm_xl_kernelILi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)ELi(\d+)E", name)
+            if not t:
+                continue
+            fmt, mt, h, w, _ = map(int, t.groups())
+            stages, dma = (3 if h == 2 else 2), -(-4 * mt // w)
+            rows = fmt in (hip.CIR_I4_ROW, hip.CIR_I8_ROW)
+            loads = 2 * ((1 if fmt in (hip.CIR_Q4_0, hip.CIR_I4_ROW) else 2) + (0 if rows else 1))
+            code = [line.split("//")[0].strip() for line in part.splitlines()]
+            vmem = [c for c in code if c.startswith("buffer_load")]
+            to_lds = sum(c.endswith(" lds") for c in vmem)
+            assert len(vmem) - to_lds == 2 * stages * loads, name
+            assert to_lds == (2 * stages - 1) * dma, name
+            waits = [re.search(r"vmcnt\((\d+)\)", a) for a, b in zip(code, code[1:]) if b.startswith("s_barrier")]
+            counted = (stages - 2) * dma + (stages - 1) * loads
+            assert sum(m is not None and int(m.group(1)) == counted for m in waits) >= stages, name
+            assert all(m is None or int(m.group(1)) <= counted for m in waits), name
+            seen += 1
+    assert seen >= 90, f"only {seen} instances found"
 
 
 def llama(layers=3, **kw):
