@@ -1191,16 +1191,19 @@ int launch_attention(const void* q, const void* k_pool, const void* v_pool, cons
   const int G = Hq / Hkv;
   hipStream_t s = as_stream(stream);
   const bool mfma = mfma_path(kv_dtype, D, P, G);
-  const int S = launch_splits(rows, Hkv, max_ctx, mfma);
+  // The prefill kernel's DMA takes 16-byte groups of the pools by 32-bit offsets inside a page; pools on other addresses
+  // (or pages of 4 GiB a head) run the decode kernel over the rows, which reads them by plain loads.
+  const bool prefill = mfma && q_len > 1 && P < (1 << 24) &&
+                       (reinterpret_cast<uintptr_t>(k_pool) | reinterpret_cast<uintptr_t>(v_pool)) % 16 == 0;
+  const int S = mfma && q_len > 1 ? 1 : launch_splits(rows, Hkv, max_ctx, mfma);
   // The advertised size (cir_paged_attention_workspace_bytes) covers any split count;
   // the static-scratch and split-prefill entry points check the bytes this launch writes instead.
-  const bool prefill = mfma && q_len > 1;
   PrefillPlan pl{};
   if (prefill) pl = prefill_plan(batch, q_len, Hkv, G, max_ctx, prefill_splits);
   const size_t need = !exact_workspace ? cir_paged_attention_workspace_bytes(rows, Hq, D, max_ctx)
                       : prefill        ? partial_bytes(rows, Hq, D, pl.splits, mfma)
                                        : partial_bytes(rows, Hq, D, S, mfma);
-  CIR_CHECK_ARG((workspace || (prefill && need == 0)) && workspace_bytes >= need,
+  CIR_CHECK_ARG((workspace || need == 0) && workspace_bytes >= need,
                 "attention: workspace too small (%zu < %zu)", workspace_bytes, need);
   CIR_CHECK_ARG(!qkv.part || (mfma && q_len == 1 && qkv.splits >= 1 && qkv.inv_freq && qkv.positions),
                 "attention: the fused QKV input needs decode (q_len 1), fp16 pools, head_dim 128, page_size %% 16 == 0, "

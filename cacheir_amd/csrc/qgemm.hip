@@ -1277,6 +1277,13 @@ bool use_xl(int m, int n, int k, bool splittable = true) {
 // The fused SwiGLU (one split) takes it at every 32 < m <= 128, whatever n: its column runs spread over the CUs.
 bool use_xl_swiglu(int m, int n, int k) { return (m > 32 && m <= 128) || use_xl(m, n, k, false); }
 
+// What else the large-m kernel asks of a launch: its DMA takes 16-byte groups of x, and its offsets count 32 bits from a
+// block of 128 rows of x and from a run of up to 10 weight tiles.  Launches that do not fit run the m <= 32 kernel over
+// 32-row blocks, which reads x by plain loads and takes 64-bit addresses, at any m.
+bool xl_fits(const void* x, int ldx, int k) {
+  return reinterpret_cast<uintptr_t>(x) % 16 == 0 && ldx <= (1 << 23) && k <= (1 << 24);
+}
+
 // Its k-split; splits need not divide k/128: split s covers quads s * ceil(kq / S) onward, the last one fewer, and S is
 // lowered to ceil(kq / len) for that length so that no split is empty (86 quads at 16 splits would leave split 15
 // starting past the end; 15 splits of 6 quads do not).
@@ -1340,7 +1347,7 @@ void dispatch_qgemm(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd
                     int splits, hipStream_t s) {
   if (gemv_fits(M, K, splits)) launch_qgemv<FMT, 0>(x, ldx, wq, wd, part, M, N, K, splits, s);
   else if (M <= 16) launch_qgemm_xs<FMT, 1, 1, 4>(x, ldx, wq, wd, part, M, N, K, splits, s);
-  else if (!use_xl(M, N, K)) launch_qgemm_xs<FMT, 2, 2, CIR_XS_DW>(x, ldx, wq, wd, part, M, N, K, splits, s);
+  else if (!use_xl(M, N, K) || !xl_fits(x, ldx, K)) launch_qgemm_xs<FMT, 2, 2, CIR_XS_DW>(x, ldx, wq, wd, part, M, N, K, splits, s);
   else launch_qgemm_xl<FMT>(x, ldx, wq, wd, part, M, N, K, splits, s);
 }
 
@@ -1428,6 +1435,9 @@ extern "C" int cir_qgemm(const void* x, int ldx, const void* w_tiled, int fmt, f
                 k / 128);
   CIR_CHECK_ARG(ldx >= k && ldx % 8 == 0, "qgemm: ldx (%d) must be >= k and a multiple of 8", ldx);
   CIR_CHECK_ARG(x && w_tiled && y_partial, "qgemm: null pointer");
+  CIR_CHECK_ARG((k / 128) % splits == 0 || xl_fits(x, ldx, k),
+                "qgemm: splits (%d) that do not divide k/128 (%d) need x on 16 bytes, ldx <= 2^23 and k <= 2^24", splits,
+                k / 128);
   CIR_CHECK_ARG(splits <= 65535 && (m + 15) / 16 <= 65535, "qgemm: grid too large");
   const size_t tiles = (size_t)((n + 15) / 16) * (k / 128);
   const uint8_t* q = static_cast<const uint8_t*>(w_tiled);
@@ -1490,7 +1500,7 @@ extern "C" int cir_qgemm_swiglu(const void* x, int ldx, const void* w_tiled, int
   const f16* xh = static_cast<const f16*>(x);
   hipStream_t s = as_stream(stream);
   auto go = [&]<int FMT>() {
-    if (use_xl_swiglu(m, n, k)) {
+    if (use_xl_swiglu(m, n, k) && xl_fits(x, ldx, k)) {
       launch_qgemm_xl_swiglu<FMT>(xh, ldx, q, d, out, odt, m, n, k, s);
       return;
     }
@@ -1575,7 +1585,7 @@ extern "C" int cir_qgemm_argmax(const void* x, int ldx, const void* w_tiled, int
         return;
       }
     }
-    if (use_xl(m, n, k, false)) {
+    if (use_xl(m, n, k, false) && xl_fits(x, ldx, k)) {
       const int groups = launch_qgemm_xl_argmax<FMT>(xh, ldx, q, d, cv, ci, m, n, k, s);
       argmax_cand_kernel<<<m, 256, 0, s>>>(cv, ci, groups, m, ids);
     } else if (m <= 16) {

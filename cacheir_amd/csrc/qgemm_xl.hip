@@ -67,12 +67,14 @@ __global__ __launch_bounds__(64 * W, 2) void qgemm_xl_kernel(const f16* __restri
   // Activation DMA: instruction i (0 .. 4*MT-1) fills KiB i of a stage, rows 4i + lane/16; 16-byte chunk g of row r sits
   // in slot g ^ (r & 15), so the 16 rows of a fragment read hit 16 different slots.  Every wavefront issues NI (past the
   // last: the last again, the same bytes to the same place), so the waits can count.  Rows past M re-read row M-1.
-  const rsrc_t rx = make_rsrc(x, (uint32_t)((size_t)M * ldx * 2));
+  // Offsets are 32 bits from the row block's first row and, for the weights, from the run's first tile (xl_fits).
+  const int mrows = min(16 * MT, M - m0);
+  const rsrc_t rx = make_rsrc(x + (size_t)m0 * ldx, (uint32_t)mrows * (uint32_t)ldx * 2u);
   uint32_t xoff[NI];
 #pragma unroll
   for (int u = 0; u < NI; ++u) {
     const int r = 4 * min(wave * NI + u, 4 * MT - 1) + (lane >> 4);
-    xoff[u] = (uint32_t)min(m0 + r, M - 1) * (uint32_t)ldx * 2u + 16u * ((lane & 15) ^ (r & 15));
+    xoff[u] = (uint32_t)min(r, mrows - 1) * (uint32_t)ldx * 2u + 16u * ((lane & 15) ^ (r & 15));
   }
   auto dma = [&](uint8_t* st, int i) __attribute__((always_inline)) {
     const uint32_t off = 256u * (uint32_t)__builtin_amdgcn_readfirstlane(q0 + min(i, nqs - 1));
@@ -81,13 +83,14 @@ __global__ __launch_bounds__(64 * W, 2) void qgemm_xl_kernel(const f16* __restri
   };
 
   // Weight loads of quad i (clamped to the last) into ring slot i % NS.
-  const uint32_t ntiles_total = (uint32_t)NTILES * KQ;
-  const rsrc_t rw = make_rsrc(wq, ntiles_total * 1024u * LB);
-  const rsrc_t rd = make_rsrc(wd, kRow ? 0u : ntiles_total * 128u);
+  const int run_tiles = min(2 * cnt, NTILES - 2 * p0);
+  const size_t tile0 = (size_t)(2 * p0) * KQ;
+  const rsrc_t rw = make_rsrc(wq + tile0 * 1024 * LB, (uint32_t)run_tiles * KQ * 1024u * LB);
+  const rsrc_t rd = make_rsrc(kRow ? wd : wd + tile0 * 64, kRow ? 0u : (uint32_t)run_tiles * KQ * 128u);
   const uint32_t vw = (uint32_t)lane * 16u * LB, vd = (uint32_t)li * 8u;
   uint32_t tb[2];
 #pragma unroll
-  for (int b = 0; b < 2; ++b) tb[b] = (uint32_t)min(nt + b, NTILES - 1) * KQ + q0;
+  for (int b = 0; b < 2; ++b) tb[b] = (uint32_t)(min(nt + b, NTILES - 1) - 2 * p0) * KQ + q0;
   struct Raw {
     uint4 w[2][LB];
     uint2 d[2];

@@ -303,6 +303,8 @@ def qgemm_partial(x: torch.Tensor, w: QWeight, splits: int | None = None, out: t
     if out is None:
         out = torch.empty((splits, m, w.n), dtype=torch.float32, device=x.device)
     _req(out.numel() >= splits * m * w.n and out.dtype == torch.float32, "partial buffer too small")
+    if x.data_ptr() % 16 and (w.k // 128) % splits:  # only the large-m kernel takes such splits, and it reads x by DMA
+        x = x.clone(memory_format=torch.contiguous_format)
     hip.call("cir_qgemm", x.data_ptr(), x.stride(0), w.tiled.data_ptr(), w.fmt, out.data_ptr(), m, w.n, w.k, splits,
              hip.stream_handle())
     return out.view(-1)[: splits * m * w.n].view(splits, m, w.n)

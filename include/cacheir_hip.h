@@ -194,7 +194,9 @@ size_t cir_qgemm_workspace_bytes(int m, int n, int splits);
  * GEMM.  For the same split both give the same partials bit for bit.
  * splits must divide k/128, except where the large-m GEMM runs (cir_qgemm_plan names
  * qgemm_xl_kernel): there split s covers quads s*ceil(k/128/splits) onward (the last
- * fewer) and any count that leaves no split empty is taken.  Requires k % 128 == 0. */
+ * fewer) and any count that leaves no split empty is taken; x must then start on 16 bytes
+ * (an x on any other address, or rows more than 2^23 elements apart, run the m <= 32 kernel).
+ * Requires k % 128 == 0. */
 int cir_qgemm(const void* x, int ldx, const void* w_tiled, int fmt, float* y_partial,
               int m, int n, int k, int splits, void* stream);
 

@@ -336,6 +336,30 @@ def test_prefill_attention_later_infinities_stay_out(device, batch, g, hkv, q_le
         close16(out[b * q_len:(b + 1) * q_len][early], ref[early])
 
 
+def test_prefill_attention_pools_off_16_bytes(device):
+    """Pools that start 8 bytes past a 16-byte address (the prefill kernel's DMA takes whole groups) agree with the oracle,
+    at sizes that would split the context."""
+    from cacheir_amd import kernels
+
+    rng = np.random.default_rng(23)
+    past, q_len, hq, hkv = 1100, 9, 14, 2
+    kp, vp, pt, lens = paged.build_pool(rng, [past + q_len], hkv, 128, 16)
+    q = rng.standard_normal((q_len, hq, 128)).astype(np.float16)
+
+    def shifted(a):
+        t = torch.empty(a.size + 4, dtype=torch.float16, device=device)[4:].view(a.shape)
+        t.copy_(to_dev(a, device))
+        assert t.data_ptr() % 16 == 8
+        return t
+
+    out = kernels.paged_prefill_attention(to_dev(q, device), shifted(kp), shifted(vp), to_dev(pt, device),
+                                          to_dev(lens, device), q_len).float().cpu().numpy()
+    kh = paged.gather_sequence(kp, pt[0], past + q_len).astype(np.float32)[None]
+    vh = paged.gather_sequence(vp, pt[0], past + q_len).astype(np.float32)[None]
+    ref = ops.attention(q.astype(np.float32)[None], kh, vh, hq, hkv, 128, causal=True).reshape(q_len, hq, 128)
+    close16(out, ref)
+
+
 def test_prefill_attention_leaves_a_shared_workspace_alone(device):
     """Overlapping prefills may share a workspace on the fp16 head_dim-128 path: a call that is not told that the
     workspace is its own does not write it, at sizes that split the context (9 tokens after 1100: 2 query tiles).  The
@@ -680,6 +704,45 @@ def test_qgemm_large_m_geometries(device, fmt, m, n, k, splits):
         assert bool(((part[s].double() - xs @ ws.T).abs() <= 1e-5 * size + 1e-6).all()), s
     ids = kernels.qgemm_argmax(x, w)
     assert torch.equal(ids, kernels.qgemm_partial(x, w, splits=1)[0].argmax(dim=1))
+
+
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
+@pytest.mark.parametrize("shift,ldx", [(4, 0), (0, 1 << 23), (0, (1 << 23) + 8), (0, 1 << 24)])
+@pytest.mark.parametrize("m", [40, 130])
+def test_qgemm_activations_the_large_m_kernel_cannot_address(device, fmt, shift, ldx, m):
+    """Activations that do not start on 16 bytes, or whose row pitch takes 128 rows past 32-bit offsets (the pitch at
+    the limit runs the large-m kernel): partials, SwiGLU and greedy ids as for the same activations packed, at sizes of
+    the large-m kernel; a k-split that does not divide takes a packed copy."""
+    from cacheir_amd import hip, kernels
+
+    n, k, code = 4736, 640, kernels.FMT_NAMES[fmt]
+    g = torch.Generator(device=device)
+    g.manual_seed(m)
+    d = (torch.rand(n, k // 32, generator=g, device=device) * 0.01).half().view(torch.uint8).view(n, k // 32, 2)
+    q = torch.randint(0, 256, (n, k // 32, kernels.BLOCK_BYTES[code] - 2), generator=g, device=device)
+    w = kernels.QWeight.from_blocks(torch.cat([d, q.to(torch.uint8)], dim=2).reshape(-1), code, n, k)
+    assert kernels.gemm_plan(hip.GEMM_PARTIALS, code, m, n, k, 1).startswith("qgemm_xl_kernel")
+    pitch = ldx or k
+    packed = torch.randn(m, k, generator=g, device=device).half()
+    store = torch.empty((m - 1) * pitch + k + shift, dtype=torch.float16, device=device)
+    x = store[shift:].as_strided((m, k), (pitch, 1), shift)
+    x.copy_(packed)
+    assert x.data_ptr() % 16 == 2 * shift
+    size = packed.double().abs() @ kernels.dequant_tiled(w).double().abs().T
+    ref = packed.double() @ kernels.dequant_tiled(w).double().T
+    one = kernels.qgemm_partial(x, w, splits=1)[0]
+    assert bool(((one.double() - ref).abs() <= 1e-5 * size + 1e-6).all())
+    two = kernels.qgemm_partial(x, w, splits=5).sum(0)
+    assert bool(((two.double() - ref).abs() <= 1e-5 * size + 1e-6).all())
+    if ldx <= 1 << 23:  # 2 splits of 3 and 2 quads
+        assert torch.equal(kernels.qgemm_partial(x, w, splits=2), kernels.qgemm_partial(packed, w, splits=2))
+    assert torch.equal(kernels.qgemm_argmax(x, w), one.argmax(dim=1))
+    # silu(g) u of gate and up in turns of 16 columns: |silu'| <= 1.1 and |silu(g)| <= |g| carry the products' bound on
+    part = lambda t, i: t.view(m, n // 32, 2, 16)[:, :, i].reshape(m, n // 2)
+    gate, up = part(ref, 0), part(ref, 1)
+    want = torch.nn.functional.silu(gate) * up
+    bound = 1.1e-5 * part(size, 0) * up.abs() + 1e-5 * gate.abs() * part(size, 1) + 1e-5 * want.abs() + 1e-6
+    assert bool(((kernels.qgemm_swiglu(x, w, torch.float32).double() - want).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("m,n,k,splits", [
