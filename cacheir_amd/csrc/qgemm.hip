@@ -1263,19 +1263,11 @@ void launch_qgemm_xs(const f16* x, int ldx, const uint8_t* wq, const uint16_t* w
 // Workgroups of the large-m kernel before any k-split: groups of 128 columns x blocks of up to 128 rows.
 long xl_groups(int m, int n) { return (long)((n + 127) / 128) * ((m + 127) / 128); }
 
-// m > 32 takes the large-m kernel when n spans at least 36 groups of 128 columns, when its workgroups alone fill the CUs
-// (>= 192), or, where k may be split, when k holds at least 64 quads, or 16 past 128 rows (the k-split pieces then stay
-// long).  Measured on MI355X (us) against the m <= 32 kernel run over 32-row blocks: Q8_0 at m = 64 / 128 QKV (n 4608)
-// 9.5 / 13.4 against 15.4 / 24.5, down (n 3584, k 18944) at m = 128 34.9 over 9 splits against 66.4; O (n 3584, k 3584:
-// 28 quads) stays on the small kernel there (12.4 against 14.6 at 7 splits) and leaves it at m = 200 (16.4 against 20.5;
-// m = 512 26.3 against 31.9).  The SwiGLU launch cannot split k (splittable = false).
-bool use_xl(int m, int n, int k, bool splittable = true) {
-  if (m <= 32) return false;
-  return (n + 127) / 128 >= 36 || xl_groups(m, n) >= 192 || (splittable && k / 128 >= (m > 128 ? 16 : 64));
-}
-
-// The fused SwiGLU (one split) takes it at every 32 < m <= 128, whatever n: its column runs spread over the CUs.
-bool use_xl_swiglu(int m, int n, int k) { return (m > 32 && m <= 128) || use_xl(m, n, k, false); }
+// One k-split: the large-m kernel runs where m > 32 and n spans at least 36 groups of 128 columns, or its workgroups
+// alone fill most CUs (>= 192); the m <= 32 kernel over 32-row blocks elsewhere (it has four times the workgroups: SwiGLU
+// 4096 x 8192 on int4 rows at m = 128 26 us against 43).  Partials, SwiGLU and greedy head decide alike, so that their
+// results are each other's bit for bit.
+bool use_xl_one(int m, int n) { return m > 32 && ((n + 127) / 128 >= 36 || xl_groups(m, n) >= 192); }
 
 // What else the large-m kernel asks of a launch: its DMA takes 16-byte groups of x, and its offsets count 32 bits from a
 // block of 128 rows of x and from a run of up to 10 weight tiles.  Launches that do not fit run the m <= 32 kernel over
@@ -1284,31 +1276,75 @@ bool xl_fits(const void* x, int ldx, int k) {
   return reinterpret_cast<uintptr_t>(x) % 16 == 0 && ldx <= (1 << 23) && k <= (1 << 24);
 }
 
-// Its k-split; splits need not divide k/128: split s covers quads s * ceil(kq / S) onward, the last one fewer, and S is
-// lowered to ceil(kq / len) for that length so that no split is empty (86 quads at 16 splits would leave split 15
-// starting past the end; 15 splits of 6 quads do not).
-//   * m <= 128: as many splits of at least 4 quads as keep the launch at one round of workgroups over the 256 CUs (down
-//     at m = 128: 9 splits, 252 workgroups: 42.3 us against 46.5 at 8 and 43.9 at 10).
-//   * more rows, projections (n <= 8192): the least estimate over 1..4 splits of rounds over the CUs x (1.18 us per quad
-//     + 3) plus the partials written and read back at 10 TB/s.  A grid of 160 workgroups leaves 96 CUs idle for the whole
-//     of k; 480 of a third of k do not: down (4096 x 14336, Q4_0) at m = 600 136 -> 91 us, QKV (6144 x 4096) at m = 350
-//     43 -> 31.  Wider n (the LM head) keeps one split: its partials are the logits.
-int xl_splits(int m, int n, int k) {
+// Workgroup rows: 4 wavefronts x NT tiles x 16.  m <= 16 takes NT = 1 (64 rows per
+// workgroup, MT = 1); larger m takes NT = 2, MT = 2 (128 rows x 32 activation rows):
+// each activation quad then feeds 8 weight tiles.  Measured on MI355X at the
+// Llama-3-8B shapes (m = 1, 8, 32) against NT = 4 and ring depths 2..6.
+constexpr int xs_rows_per_group(int m) { return m <= 16 ? 64 : 128; }
+
+// k-split of the m <= 32 kernel: the smallest power of two that gives >= 192 workgroups, keeping at least
+// 4 quads per split (split-k partials cost 4*m*n bytes each, so no more than needed).
+// The threshold, swept on the config-4 step at m = 32 (same box, two passes each):
+// 96 / 128 / 192 / 256 / 384 gave 3.80 / 3.69 / 3.45-3.54 / 3.58 / 3.70 ms.
+int xs_splits(int m, int n, int k) {
+  const int kq = k / 128;
+  const long groups = (long)((n + xs_rows_per_group(m) - 1) / xs_rows_per_group(m)) * ((m + 31) / 32);
+  int s = 1;
+  while (groups * s < 192 && kq % (2 * s) == 0 && kq / (2 * s) >= 4) s *= 2;
+  return s;
+}
+
+// The kernel and k-split of cir_qgemm past m = 32.  The large-m kernel's splits need not divide k/128: split s covers
+// quads s * ceil(kq / S) onward, the last one fewer, and only counts that leave no split empty are proposed (86 quads at
+// 16 splits would leave split 15 starting past the end; 15 splits of 6 quads do not).
+//   * m <= 128: the large-m kernel where n spans 36 groups, or k holds at least 64 quads (the k-split pieces then stay
+//     long), over as many splits of at least 4 quads as keep the launch at one round of workgroups over the 256 CUs (Q8_0
+//     down, n 3584, k 18944, at m = 128: 9 splits, 252 workgroups: 42.3 us against 46.5 at 8 and 43.9 at 10; QKV, n 4608,
+//     at m = 64 / 128 9.5 / 13.4 against 15.4 / 24.5 on the m <= 32 kernel, whose O, n 3584, k 3584, takes 12.4 against
+//     14.6 at 7 splits).
+//   * more rows, projections (n <= 8192), also where k holds 16 quads: the least estimate of rounds over the CUs x (1.18 us
+//     per quad + 3) plus the partials written and read back at 10 TB/s, over 1 .. 4 splits.  A grid of 160 workgroups
+//     leaves 96 CUs idle for the whole of k; 480 of a third of k do not: down (4096 x 14336, Q4_0) at m = 600 136 -> 91 us,
+//     QKV (6144 x 4096) at m = 350 43 -> 31.  Wider n (the LM head) keeps one split: its partials are the logits.
+struct XlChoice {
+  bool xl;
+  int splits;
+};
+XlChoice choose_xl(int m, int n, int k) {
   const long kq = k / 128, groups = xl_groups(m, n);
-  long s = 1;
+  const bool one = use_xl_one(m, n);
+  auto whole = [&](long s) {  // the count of splits of that length that hold a quad
+    const long len = (kq + s - 1) / s;
+    return (int)((kq + len - 1) / len);
+  };
   if (m <= 128) {
-    const long by_cus = kCUs / groups, by_len = kq / 4;
-    s = by_cus < by_len ? by_cus : by_len;
-  } else if (n <= 8192) {
-    double best = 0;
-    for (long c = 1; c <= 4 && (c == 1 || kq / c >= 4); ++c) {
-      const double t = (double)((groups * c + kCUs - 1) / kCUs) * (1.18 * ((kq + c - 1) / c) + 3) + 8e-7 * c * m * n;
-      if (c == 1 || t < best) best = t, s = c;
-    }
+    if (!one && kq < 64) return {false, xs_splits(m, n, k)};
+    const long by_cus = kCUs / groups, by_len = kq / 4, s = by_cus < by_len ? by_cus : by_len;
+    if (s > 1) return {true, whole(s)};
+    return {one, one ? 1 : xs_splits(m, n, k)};
   }
-  if (s <= 1) return 1;
-  const long len = (kq + s - 1) / s;
-  return (int)((kq + len - 1) / len);
+  int split = 1;
+  double best = 0;
+  for (int c = 1; n <= 8192 && c <= 4 && (c == 1 || kq / c >= 4); ++c) {
+    const double t = (double)((groups * c + kCUs - 1) / kCUs) * (1.18 * ((kq + c - 1) / c) + 3) + 8e-7 * c * m * n;
+    if (c == 1 || t < best) best = t, split = c;
+  }
+  split = whole(split);
+  if (one || (kq >= 16 && split > 1)) return {true, split};
+  return {false, xs_splits(m, n, k)};
+}
+
+// The large-m kernel also takes every count of splits that does not divide k/128 where k is long enough for it (64 quads,
+// 16 past 128 rows).
+bool xl_any_splits(int m, int n, int k) {
+  return m > 32 && (use_xl_one(m, n) || k / 128 >= (m > 128 ? 16 : 64));
+}
+
+// Does a partials launch with `splits` run the large-m kernel?
+bool use_xl(int m, int n, int k, int splits) {
+  if (m <= 32 || splits == 1) return use_xl_one(m, n);
+  if ((k / 128) % splits) return xl_any_splits(m, n, k);
+  return choose_xl(m, n, k).xl;
 }
 
 // The k-splits a cir_qgemm launch accepts: those dividing k/128, and on the large-m
@@ -1317,29 +1353,14 @@ bool splits_ok(int m, int n, int k, int splits) {
   const int kq = k / 128;
   if (splits < 1 || splits > kq) return false;
   if (kq % splits == 0) return true;
-  return use_xl(m, n, k) && (splits - 1) * ((kq + splits - 1) / splits) < kq;
+  return xl_any_splits(m, n, k) && (splits - 1) * ((kq + splits - 1) / splits) < kq;
 }
 
-// Workgroup rows: 4 wavefronts x NT tiles x 16.  m <= 16 takes NT = 1 (64 rows per
-// workgroup, MT = 1); larger m takes NT = 2, MT = 2 (128 rows x 32 activation rows):
-// each activation quad then feeds 8 weight tiles.  Measured on MI355X at the
-// Llama-3-8B shapes (m = 1, 8, 32) against NT = 4 and ring depths 2..6.
-constexpr int xs_rows_per_group(int m) { return m <= 16 ? 64 : 128; }
-
-// k-split: the smallest power of two that gives >= 192 workgroups, keeping at least
-// 4 quads per split (split-k partials cost 4*m*n bytes each, so no more than needed).
-// The threshold, swept on the config-4 step at m = 32 (same box, two passes each):
-// 96 / 128 / 192 / 256 / 384 gave 3.80 / 3.69 / 3.45-3.54 / 3.58 / 3.70 ms.
 int default_splits(int m, int n, int k) {
   if (m <= 8) {
     if (const int s = gemv_splits(m, n, k)) return s;
   }
-  if (use_xl(m, n, k)) return xl_splits(m, n, k);
-  const int kq = k / 128;
-  const long groups = (long)((n + xs_rows_per_group(m) - 1) / xs_rows_per_group(m)) * ((m + 31) / 32);
-  int s = 1;
-  while (groups * s < 192 && kq % (2 * s) == 0 && kq / (2 * s) >= 4) s *= 2;
-  return s;
+  return m > 32 ? choose_xl(m, n, k).splits : xs_splits(m, n, k);
 }
 
 template <int FMT>
@@ -1347,7 +1368,7 @@ void dispatch_qgemm(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd
                     int splits, hipStream_t s) {
   if (gemv_fits(M, K, splits)) launch_qgemv<FMT, 0>(x, ldx, wq, wd, part, M, N, K, splits, s);
   else if (M <= 16) launch_qgemm_xs<FMT, 1, 1, 4>(x, ldx, wq, wd, part, M, N, K, splits, s);
-  else if (!use_xl(M, N, K) || !xl_fits(x, ldx, K)) launch_qgemm_xs<FMT, 2, 2, CIR_XS_DW>(x, ldx, wq, wd, part, M, N, K, splits, s);
+  else if (!use_xl(M, N, K, splits) || !xl_fits(x, ldx, K)) launch_qgemm_xs<FMT, 2, 2, CIR_XS_DW>(x, ldx, wq, wd, part, M, N, K, splits, s);
   else launch_qgemm_xl<FMT>(x, ldx, wq, wd, part, M, N, K, splits, s);
 }
 
@@ -1500,7 +1521,7 @@ extern "C" int cir_qgemm_swiglu(const void* x, int ldx, const void* w_tiled, int
   const f16* xh = static_cast<const f16*>(x);
   hipStream_t s = as_stream(stream);
   auto go = [&]<int FMT>() {
-    if (use_xl_swiglu(m, n, k) && xl_fits(x, ldx, k)) {
+    if (use_xl_one(m, n) && xl_fits(x, ldx, k)) {
       launch_qgemm_xl_swiglu<FMT>(xh, ldx, q, d, out, odt, m, n, k, s);
       return;
     }
@@ -1585,7 +1606,7 @@ extern "C" int cir_qgemm_argmax(const void* x, int ldx, const void* w_tiled, int
         return;
       }
     }
-    if (use_xl(m, n, k, false) && xl_fits(x, ldx, k)) {
+    if (use_xl_one(m, n) && xl_fits(x, ldx, k)) {
       const int groups = launch_qgemm_xl_argmax<FMT>(xh, ldx, q, d, cv, ci, m, n, k, s);
       argmax_cand_kernel<<<m, 256, 0, s>>>(cv, ci, groups, m, ids);
     } else if (m <= 16) {
@@ -1608,17 +1629,17 @@ extern "C" const char* cir_qgemm_plan(int op, int fmt, int m, int n, int k, int 
       if (!splits_ok(m, n, k, splits)) return "invalid";
       if (gemv_fits(m, k, splits)) return "qgemv_kernel";
       if (m <= 16) return "qgemm_xs_kernel<NT=1,MT=1>";
-      if (!use_xl(m, n, k)) return "qgemm_xs_kernel<NT=2,MT=2>";
+      if (!use_xl(m, n, k, splits)) return "qgemm_xs_kernel<NT=2,MT=2>";
       return m <= 64 ? "qgemm_xl_kernel<MT=4>" : m <= 96 ? "qgemm_xl_kernel<MT=6>" : "qgemm_xl_kernel<MT=8>";
     case CIR_GEMM_SWIGLU:
-      if (use_xl_swiglu(m, n, k))
+      if (use_xl_one(m, n))
         return m <= 64   ? "qgemm_xl_kernel<MT=4,EPI=swiglu>"
                : m <= 96 ? "qgemm_xl_kernel<MT=6,EPI=swiglu>"
                          : "qgemm_xl_kernel<MT=8,EPI=swiglu>";
       return m <= 16 ? "qgemm_xs_kernel<NT=2,MT=1,EPI=swiglu>" : "qgemm_xs_kernel<NT=2,MT=2,EPI=swiglu>";
     case CIR_GEMM_ARGMAX:
       if (gemv_head_fits(fmt, m, k)) return "qgemv_kernel<EPI=argmax>+argmax_cand_kernel";
-      if (use_xl(m, n, k, false))
+      if (use_xl_one(m, n))
         return m <= 64   ? "qgemm_xl_kernel<MT=4,EPI=argmax>+argmax_cand_kernel"
                : m <= 96 ? "qgemm_xl_kernel<MT=6,EPI=argmax>+argmax_cand_kernel"
                          : "qgemm_xl_kernel<MT=8,EPI=argmax>+argmax_cand_kernel";

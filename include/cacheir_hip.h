@@ -229,7 +229,9 @@ int cir_qgemm_attn(const float* attn_part_o, const float* attn_part_ml, int attn
  * gate rows 16c..16c+15, then up rows 16c..16c+15, for c = 0, 1, ... (make it by
  * permuting the GGUF block rows before cir_qweight_repack).  out dtype odt
  * (CIR_F16 / CIR_F32), [m][inter].  inter % 16 == 0, k % 128 == 0.  Bitwise equal to
- * cir_qgemm (splits 1) over the same tiles followed by cir_epilogue_swiglu. */
+ * cir_qgemm (splits 1) over the same tiles followed by cir_epilogue_swiglu at m > 16, and
+ * below k = 4096 at any m (from there on this launch may sum even and odd quads apart
+ * where cir_qgemm at m <= 16 does not). */
 int cir_qgemm_swiglu(const void* x, int ldx, const void* w_tiled, int fmt, void* out, int odt, int m,
                      int inter, int k, void* stream);
 

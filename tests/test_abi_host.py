@@ -98,6 +98,21 @@ def test_prefill_split_bytes_fit_the_advertised_workspace():
 
 
 @pytest.mark.skipif(not hip.library_path().exists(), reason="libcacheir_hip.so not built")
+def test_one_split_runs_one_kernel_under_every_epilogue():
+    """Past 32 rows cir_qgemm at one split, the fused SwiGLU and the greedy head run the same kernel, so their results are
+    each other's bit for bit (the m <= 32 and the large-m kernel may sum the quads in different orders)."""
+    from cacheir_amd import kernels
+
+    for fmt in (hip.CIR_Q4_0, hip.CIR_Q8_0, hip.CIR_I4_ROW, hip.CIR_I8_ROW):
+        for m in (33, 64, 65, 96, 97, 128, 129, 200, 512, 2048):
+            for n in (128, 1024, 2048, 3584, 4096, 4576, 4608, 8192, 37888, 128256):
+                for k in (128, 2048, 4096, 8192, 18944):
+                    names = {kernels.gemm_plan(op, fmt, m, n, k, 1).split("<")[0]
+                             for op in (hip.GEMM_PARTIALS, hip.GEMM_SWIGLU, hip.GEMM_ARGMAX)}
+                    assert len(names) == 1 and names <= {"qgemm_xs_kernel", "qgemm_xl_kernel"}, (fmt, m, n, k, names)
+
+
+@pytest.mark.skipif(not hip.library_path().exists(), reason="libcacheir_hip.so not built")
 def test_default_splits_are_always_accepted():
     """Whatever k-split the library proposes for a shape, its own launch accepts (no empty last split): the
     Qwen2.5-3B down (n 2048, k 11008: 86 quads) at m = 64 once got 16 splits, which start split 15 past the end."""

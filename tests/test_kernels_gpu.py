@@ -1097,6 +1097,36 @@ def test_qgemm_swiglu_matches_gemm_then_epilogue(device, fmt, m, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("fmt", ["q4_0", "q8_0", "int4", "int8"])
+@pytest.mark.parametrize("m,inter,k", [(33, 512, 4096), (77, 1024, 8192), (128, 2288, 4096), (128, 2304, 4096), (200, 512, 4096),
+                                       (300, 2288, 8192)])
+def test_one_split_epilogues_agree_bitwise(device, fmt, m, inter, k):
+    """Past 32 rows the fused SwiGLU equals the one-split partials with the SwiGLU epilogue, and the greedy ids their
+    argmax, bit for bit in every format: narrow products (the m <= 32 kernel, two k-groups) and the last and first
+    widths on either side of the large-m kernel's 36 column groups."""
+    from cacheir_amd import kernels
+
+    n = 2 * inter
+    g = torch.Generator(device=device)
+    g.manual_seed(m + k)
+    if fmt in kernels.FMT_NAMES:
+        code = kernels.FMT_NAMES[fmt]
+        d = (torch.randn(n, k // 32, generator=g, device=device) * 0.01).half().view(torch.uint8).view(n, k // 32, 2)
+        q = torch.randint(0, 256, (n, k // 32, kernels.BLOCK_BYTES[code] - 2), generator=g, device=device)
+        w = kernels.QWeight.from_blocks(torch.cat([d, q.to(torch.uint8)], dim=2).reshape(-1), code, n, k)
+    else:
+        bits = int(fmt[3:])
+        q = torch.randint(0, 256, (n, k * bits // 8), generator=g, device=device).to(torch.uint8)
+        zp = torch.randint(0, 1 << bits, (n,), generator=g, device=device).to(torch.int32)
+        w = kernels.QWeight.from_rows(q, torch.rand(n, generator=g, device=device) * 0.01, zp, bits, n, k)
+    x = torch.randn(m, k, generator=g, device=device).half()
+    part = kernels.qgemm_partial(x, w, splits=1)
+    rows = part.view(m, n // 32, 2, 16).transpose(1, 2).reshape(1, m, n).contiguous()  # gate columns, then up columns
+    assert torch.equal(kernels.qgemm_swiglu(x, w, torch.float32), kernels.epilogue_swiglu(rows, torch.float32))
+    assert torch.equal(kernels.qgemm_argmax(x, w), part[0].argmax(dim=1))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
 @pytest.mark.parametrize("m,inter", [(40, 17600), (128, 17600), (100, 5008), (128, 2304), (130, 17600)])
 def test_qgemm_swiglu_large_m_column_runs(device, fmt, m, inter):
