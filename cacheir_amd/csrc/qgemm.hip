@@ -1265,9 +1265,13 @@ long xl_groups(int m, int n) { return (long)((n + 127) / 128) * ((m + 127) / 128
 
 // One k-split: the large-m kernel runs where m > 32 and n spans at least 36 groups of 128 columns, or its workgroups
 // alone fill most CUs (>= 192); the m <= 32 kernel over 32-row blocks elsewhere (it has four times the workgroups: SwiGLU
-// 4096 x 8192 on int4 rows at m = 128 26 us against 43).  Partials, SwiGLU and greedy head decide alike, so that their
+// 4096 x 8192 on int4 rows at m = 128 26 us against 43), but for Q8_0 at up to 64 rows and less than 32 quads (SwiGLU 4096 x
+// 2048 13.2 against 14.2: its two k-groups start there).  Partials, SwiGLU and greedy head decide alike, so that their
 // results are each other's bit for bit.
-bool use_xl_one(int m, int n) { return m > 32 && ((n + 127) / 128 >= 36 || xl_groups(m, n) >= 192); }
+bool use_xl_one(int fmt, int m, int n, int k) {
+  if (m > 32 && m <= 64 && fmt == CIR_Q8_0 && k < 4096) return true;
+  return m > 32 && ((n + 127) / 128 >= 36 || xl_groups(m, n) >= 192);
+}
 
 // What else the large-m kernel asks of a launch: its DMA takes 16-byte groups of x, and its offsets count 32 bits from a
 // block of 128 rows of x and from a run of up to 10 weight tiles.  Launches that do not fit run the m <= 32 kernel over
@@ -1294,6 +1298,24 @@ int xs_splits(int m, int n, int k) {
   return s;
 }
 
+// Estimated us of a launch past 128 rows with the epilogue that reads its partials, fitted to 746 launches at 17 row
+// counts (129 - 2048) and 27 shapes (n 512 - 12288, k 896 - 18944) in Q4_0, Q8_0 and int4 rows.  The m <= 32 kernel (rms of
+// the fit 6%) takes its quads one after the other and steps with the workgroups per CU; the large-m kernel (7%) takes
+// a round of whole quads per workgroup, two workgroups of four wavefronts to a CU past 256.
+double xs_time(int m, int n, int k, int s) {
+  const long wg = (long)((n + 127) / 128) * ((m + 31) / 32) * s, round = (wg + kCUs - 1) / kCUs;
+  const int q = (k / 128) / s;
+  const double quad = round > 1 ? 0.45 * round - 0.08 * wg / kCUs : q >= 32 && q % 2 == 0 ? 0.5 : 0.55;  // (xs_kgroups)
+  return 5.3 + q * quad + 3.6e-6 * s * m * n;
+}
+double xl_time(int m, int n, int k, int s) {
+  const long wg = xl_groups(m, n) * s;
+  const int q = (k / 128 + s - 1) / s;
+  const double t = wg <= kCUs ? 9.5 + 1.13 * q
+                              : 10.6 + q * (1.12 * ((wg + 2 * kCUs - 1) / (2 * kCUs)) + 0.95 * wg / (2 * kCUs));
+  return t + 1.35e-6 * s * m * n;
+}
+
 // The kernel and k-split of cir_qgemm past m = 32.  The large-m kernel's splits need not divide k/128: split s covers
 // quads s * ceil(kq / S) onward, the last one fewer, and only counts that leave no split empty are proposed (86 quads at
 // 16 splits would leave split 15 starting past the end; 15 splits of 6 quads do not).
@@ -1302,17 +1324,20 @@ int xs_splits(int m, int n, int k) {
 //     down, n 3584, k 18944, at m = 128: 9 splits, 252 workgroups: 42.3 us against 46.5 at 8 and 43.9 at 10; QKV, n 4608,
 //     at m = 64 / 128 9.5 / 13.4 against 15.4 / 24.5 on the m <= 32 kernel, whose O, n 3584, k 3584, takes 12.4 against
 //     14.6 at 7 splits).
-//   * more rows, projections (n <= 8192), also where k holds 16 quads: the least estimate of rounds over the CUs x (1.18 us
-//     per quad + 3) plus the partials written and read back at 10 TB/s, over 1 .. 4 splits.  A grid of 160 workgroups
+//   * more rows, projections (n <= 8192): the least estimate of rounds over the CUs x (1.18 us per quad + 3) plus the
+//     partials written and read back at 10 TB/s, over 1 .. 4 splits and up to 16 in one round.  A grid of 160 workgroups
 //     leaves 96 CUs idle for the whole of k; 480 of a third of k do not: down (4096 x 14336, Q4_0) at m = 600 136 -> 91 us,
 //     QKV (6144 x 4096) at m = 350 43 -> 31.  Wider n (the LM head) keeps one split: its partials are the logits.
+//     Where one split would not run the large-m kernel, it must also win by 7% over the m <= 32 kernel's split by the
+//     estimates above.  Us, m <= 32 kernel against large-m kernel at its best split, Q4_0: 512 x 4096 at m = 200 10.0 / 17.7,
+//     2048 x 2048 at 512 13.7 / 21.5, 4096 x 4096 at 200 22.5 / 23.7, at 350 35.1 / 30.8, at 640 47.4 / 44.6.
 struct XlChoice {
   bool xl;
   int splits;
 };
-XlChoice choose_xl(int m, int n, int k) {
+XlChoice choose_xl(int m, int n, int k) {  // (for any format)
   const long kq = k / 128, groups = xl_groups(m, n);
-  const bool one = use_xl_one(m, n);
+  const bool one = use_xl_one(CIR_Q4_0, m, n, k);
   auto whole = [&](long s) {  // the count of splits of that length that hold a quad
     const long len = (kq + s - 1) / s;
     return (int)((kq + len - 1) / len);
@@ -1325,24 +1350,26 @@ XlChoice choose_xl(int m, int n, int k) {
   }
   int split = 1;
   double best = 0;
-  for (int c = 1; n <= 8192 && c <= 4 && (c == 1 || kq / c >= 4); ++c) {
+  for (int c = 1; n <= 8192 && c <= 16 && (c == 1 || kq / c >= 4) && (c <= 4 || groups * c <= kCUs); ++c) {
     const double t = (double)((groups * c + kCUs - 1) / kCUs) * (1.18 * ((kq + c - 1) / c) + 3) + 8e-7 * c * m * n;
     if (c == 1 || t < best) best = t, split = c;
   }
   split = whole(split);
-  if (one || (kq >= 16 && split > 1)) return {true, split};
-  return {false, xs_splits(m, n, k)};
+  if (one) return {true, split};
+  const int small = xs_splits(m, n, k);
+  if (split == 1 || xs_time(m, n, k, small) < 1.07 * xl_time(m, n, k, split)) return {false, small};
+  return {true, split};
 }
 
 // The large-m kernel also takes every count of splits that does not divide k/128 where k is long enough for it (64 quads,
 // 16 past 128 rows).
 bool xl_any_splits(int m, int n, int k) {
-  return m > 32 && (use_xl_one(m, n) || k / 128 >= (m > 128 ? 16 : 64));
+  return m > 32 && (use_xl_one(CIR_Q4_0, m, n, k) || k / 128 >= (m > 128 ? 16 : 64));
 }
 
 // Does a partials launch with `splits` run the large-m kernel?
-bool use_xl(int m, int n, int k, int splits) {
-  if (m <= 32 || splits == 1) return use_xl_one(m, n);
+bool use_xl(int fmt, int m, int n, int k, int splits) {
+  if (m <= 32 || splits == 1) return use_xl_one(fmt, m, n, k);
   if ((k / 128) % splits) return xl_any_splits(m, n, k);
   return choose_xl(m, n, k).xl;
 }
@@ -1368,7 +1395,7 @@ void dispatch_qgemm(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd
                     int splits, hipStream_t s) {
   if (gemv_fits(M, K, splits)) launch_qgemv<FMT, 0>(x, ldx, wq, wd, part, M, N, K, splits, s);
   else if (M <= 16) launch_qgemm_xs<FMT, 1, 1, 4>(x, ldx, wq, wd, part, M, N, K, splits, s);
-  else if (!use_xl(M, N, K, splits) || !xl_fits(x, ldx, K)) launch_qgemm_xs<FMT, 2, 2, CIR_XS_DW>(x, ldx, wq, wd, part, M, N, K, splits, s);
+  else if (!use_xl(FMT, M, N, K, splits) || !xl_fits(x, ldx, K)) launch_qgemm_xs<FMT, 2, 2, CIR_XS_DW>(x, ldx, wq, wd, part, M, N, K, splits, s);
   else launch_qgemm_xl<FMT>(x, ldx, wq, wd, part, M, N, K, splits, s);
 }
 
@@ -1521,7 +1548,7 @@ extern "C" int cir_qgemm_swiglu(const void* x, int ldx, const void* w_tiled, int
   const f16* xh = static_cast<const f16*>(x);
   hipStream_t s = as_stream(stream);
   auto go = [&]<int FMT>() {
-    if (use_xl_one(m, n) && xl_fits(x, ldx, k)) {
+    if (use_xl_one(FMT, m, n, k) && xl_fits(x, ldx, k)) {
       launch_qgemm_xl_swiglu<FMT>(xh, ldx, q, d, out, odt, m, n, k, s);
       return;
     }
@@ -1606,7 +1633,7 @@ extern "C" int cir_qgemm_argmax(const void* x, int ldx, const void* w_tiled, int
         return;
       }
     }
-    if (use_xl_one(m, n) && xl_fits(x, ldx, k)) {
+    if (use_xl_one(FMT, m, n, k) && xl_fits(x, ldx, k)) {
       const int groups = launch_qgemm_xl_argmax<FMT>(xh, ldx, q, d, cv, ci, m, n, k, s);
       argmax_cand_kernel<<<m, 256, 0, s>>>(cv, ci, groups, m, ids);
     } else if (m <= 16) {
@@ -1629,17 +1656,17 @@ extern "C" const char* cir_qgemm_plan(int op, int fmt, int m, int n, int k, int 
       if (!splits_ok(m, n, k, splits)) return "invalid";
       if (gemv_fits(m, k, splits)) return "qgemv_kernel";
       if (m <= 16) return "qgemm_xs_kernel<NT=1,MT=1>";
-      if (!use_xl(m, n, k, splits)) return "qgemm_xs_kernel<NT=2,MT=2>";
+      if (!use_xl(fmt, m, n, k, splits)) return "qgemm_xs_kernel<NT=2,MT=2>";
       return m <= 64 ? "qgemm_xl_kernel<MT=4>" : m <= 96 ? "qgemm_xl_kernel<MT=6>" : "qgemm_xl_kernel<MT=8>";
     case CIR_GEMM_SWIGLU:
-      if (use_xl_one(m, n))
+      if (use_xl_one(fmt, m, n, k))
         return m <= 64   ? "qgemm_xl_kernel<MT=4,EPI=swiglu>"
                : m <= 96 ? "qgemm_xl_kernel<MT=6,EPI=swiglu>"
                          : "qgemm_xl_kernel<MT=8,EPI=swiglu>";
       return m <= 16 ? "qgemm_xs_kernel<NT=2,MT=1,EPI=swiglu>" : "qgemm_xs_kernel<NT=2,MT=2,EPI=swiglu>";
     case CIR_GEMM_ARGMAX:
       if (gemv_head_fits(fmt, m, k)) return "qgemv_kernel<EPI=argmax>+argmax_cand_kernel";
-      if (use_xl_one(m, n))
+      if (use_xl_one(fmt, m, n, k))
         return m <= 64   ? "qgemm_xl_kernel<MT=4,EPI=argmax>+argmax_cand_kernel"
                : m <= 96 ? "qgemm_xl_kernel<MT=6,EPI=argmax>+argmax_cand_kernel"
                          : "qgemm_xl_kernel<MT=8,EPI=argmax>+argmax_cand_kernel";

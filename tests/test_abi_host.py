@@ -113,6 +113,24 @@ def test_one_split_runs_one_kernel_under_every_epilogue():
 
 
 @pytest.mark.skipif(not hip.library_path().exists(), reason="libcacheir_hip.so not built")
+def test_narrow_products_past_128_rows_keep_the_small_kernel():
+    """Past 128 rows a narrow product leaves the large-m kernel (128 rows x 128 columns a workgroup) too few workgroups,
+    also split: these stay on the m <= 32 kernel, which measured 1.2 to 1.9 times as fast on them.  Counts that do not
+    divide k/128 stay accepted from 16 quads on."""
+    from cacheir_amd import kernels
+
+    for m, n, k in ((129, 512, 2048), (2048, 512, 2048), (200, 1024, 2048), (512, 2048, 2048), (200, 512, 4096), (350, 512, 4096),
+                    (129, 3072, 3072), (200, 1024, 4096)):
+        s = kernels.choose_splits(m, n, k)
+        assert kernels.gemm_plan(hip.GEMM_PARTIALS, hip.CIR_Q4_0, m, n, k, s).startswith("qgemm_xs_kernel"), (m, n, k, s)
+        assert kernels.gemm_plan(hip.GEMM_PARTIALS, hip.CIR_Q4_0, m, n, k, 3).startswith(
+            "qgemm_xl_kernel" if k // 128 % 3 else "qgemm_xs_kernel"), (m, n, k)
+    for m, n, k, splits in ((600, 4096, 14336, 3), (350, 6144, 4096, 3), (512, 3584, 3584, 2), (1024, 4608, 3584, 2)):
+        assert kernels.choose_splits(m, n, k) == splits
+        assert kernels.gemm_plan(hip.GEMM_PARTIALS, hip.CIR_Q4_0, m, n, k, splits).startswith("qgemm_xl_kernel")
+
+
+@pytest.mark.skipif(not hip.library_path().exists(), reason="libcacheir_hip.so not built")
 def test_default_splits_are_always_accepted():
     """Whatever k-split the library proposes for a shape, its own launch accepts (no empty last split): the
     Qwen2.5-3B down (n 2048, k 11008: 86 quads) at m = 64 once got 16 splits, which start split 15 past the end."""
