@@ -26,8 +26,9 @@
 //   * the 8 wavefronts merge (max, sum, O) through LDS with log-sum-exp weights.
 // Prefill (q_len > 1) on fp16 pools runs attn_prefill_f16_d128 instead: 128 query
 // vectors of a sequence per workgroup over its blocks, both products on MFMA.
-// fp32 pools and other head sizes (tiny-model parity path) use a plain VALU kernel
-// over 128-token chunks that always writes partials, merged by the same kernel.
+// fp32 pools and other head sizes (tiny-model parity path) use a VALU kernel over
+// 128-token chunks: a context of one chunk is written out directly, more chunks leave
+// partials for the same merge kernel.
 //
 // Reference semantics: cacheir/backends/triton_kernels.py:174-217 (paged gather
 // pool[page_table[b, t // P], kvh, t % P], GQA kvh = h // (Hq/Hkv), positions
@@ -1122,10 +1123,10 @@ int launch_splits(int rows, int Hkv, int max_ctx, bool mfma) {
   return mfma ? choose_splits(rows, Hkv, max_ctx) : generic_chunks(max_ctx);
 }
 
-// Bytes of split partials (O, then (max, sum)) a launch writes: none when the MFMA
-// kernel runs unsplit and writes the output itself.
-size_t partial_bytes(int rows, int Hq, int D, int S, bool mfma) {
-  if (mfma && S == 1) return 0;
+// Bytes of split partials (O, then (max, sum)) a launch writes: none when it runs
+// unsplit (one chunk on the generic path) and the kernel writes the output itself.
+size_t partial_bytes(int rows, int Hq, int D, int S) {
+  if (S == 1) return 0;
   return (size_t)rows * Hq * S * ((size_t)D + 2) * sizeof(float);
 }
 
@@ -1201,8 +1202,8 @@ int launch_attention(const void* q, const void* k_pool, const void* v_pool, cons
   PrefillPlan pl{};
   if (prefill) pl = prefill_plan(batch, q_len, Hkv, G, max_ctx, prefill_splits);
   const size_t need = !exact_workspace ? cir_paged_attention_workspace_bytes(rows, Hq, D, max_ctx)
-                      : prefill        ? partial_bytes(rows, Hq, D, pl.splits, mfma)
-                                       : partial_bytes(rows, Hq, D, S, mfma);
+                      : prefill        ? partial_bytes(rows, Hq, D, pl.splits)
+                                       : partial_bytes(rows, Hq, D, S);
   CIR_CHECK_ARG((workspace || need == 0) && workspace_bytes >= need,
                 "attention: workspace too small (%zu < %zu)", workspace_bytes, need);
   CIR_CHECK_ARG(!qkv.part || (mfma && q_len == 1 && qkv.splits >= 1 && qkv.inv_freq && qkv.positions),
@@ -1326,7 +1327,7 @@ extern "C" size_t cir_paged_prefill_split_bytes(int batch, int q_len, int num_he
   const int G = num_heads / num_kv_heads;
   if (!cir::mfma_path(kv_dtype, head_dim, page_size, G)) return 0;
   const cir::PrefillPlan p = cir::prefill_plan(batch, q_len, num_kv_heads, G, max_pages * page_size, true);
-  return cir::partial_bytes(batch * q_len, num_heads, head_dim, p.splits, true);
+  return cir::partial_bytes(batch * q_len, num_heads, head_dim, p.splits);
 }
 
 extern "C" int cir_paged_prefill_attention_split(const void* q, const void* k_pool, const void* v_pool,
@@ -1429,7 +1430,7 @@ extern "C" int cir_paged_decode_attention_noalloc(const void* q, const void* k_p
   CIR_CHECK_ARG(batch <= 65535, "attention_noalloc: grid too large");
   const bool mfma = cir::mfma_path(kv_dtype, head_dim, page_size, num_heads / num_kv_heads);
   const int S = cir::launch_splits(batch, num_kv_heads, max_pages * page_size, mfma);
-  const size_t need = cir::partial_bytes(batch, num_heads, head_dim, S, mfma);
+  const size_t need = cir::partial_bytes(batch, num_heads, head_dim, S);
   CIR_CHECK_ARG(need <= kScratchBytes,
                 "attention_noalloc: the split partials need %zu bytes, more than the %zu bytes of static scratch "
                 "(batch %d, %d heads, head_dim %d, %d splits); use cir_paged_decode_attention with a workspace",

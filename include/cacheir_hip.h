@@ -72,10 +72,11 @@ int cir_paged_decode_attention(const void* q, const void* k_pool, const void* v_
  * hipMalloc).  No counterpart in the reference.  It allocates nothing: the split
  * partials go to a static device array of CIR_ATTENTION_NOALLOC_MAX_BYTES per GPU,
  * looked up on the first call on each device (make the stream's device current).
- * Sizes whose partials, rows * num_heads * S * (head_dim + 2) * 4 bytes with S the
- * split count, exceed it return hipErrorInvalidValue before launching (the fp16
- * head_dim-128 path never splits beyond 256 workgroups, so it fits at any batch; the
- * generic path needs 4 * num_heads * (head_dim + 2) bytes per 128 tokens per row).
+ * Sizes whose partials, rows * num_heads * S * (head_dim + 2) * 4 bytes with S > 1 the
+ * split count (none at S = 1), exceed it return hipErrorInvalidValue before launching
+ * (the fp16 head_dim-128 path never splits beyond 256 workgroups, so it fits at any
+ * batch; the generic path, once its table holds more than 128 tokens, needs
+ * 4 * num_heads * (head_dim + 2) bytes per 128 tokens per row).
  * Results are bitwise those of cir_paged_decode_attention.  Every call on one GPU
  * shares the array: calls that overlap on one GPU (two streams, two host threads)
  * race and must be serialised by the caller.  Nothing in the array needs clearing:

@@ -98,6 +98,16 @@ def test_prefill_split_bytes_fit_the_advertised_workspace():
 
 
 @pytest.mark.skipif(not hip.library_path().exists(), reason="libcacheir_hip.so not built")
+@pytest.mark.parametrize("pages,takes", [(8, True), (9, False)])
+def test_noalloc_attention_counts_no_partials_at_one_chunk(pages, takes):
+    """A generic launch over one 128-token chunk writes its output itself, so no batch of it needs the static scratch
+    (2048 rows of 32 heads: 34 MB of partials, had it written them); two chunks do.  Null pointers end both calls."""
+    with pytest.raises(RuntimeError) as e:
+        hip.call("cir_paged_decode_attention_noalloc", *[None] * 6, 2048, 32, 8, 128, 16, pages, 1.0, hip.CIR_F32, None)
+    assert ("static scratch" not in str(e.value)) == takes, e.value
+
+
+@pytest.mark.skipif(not hip.library_path().exists(), reason="libcacheir_hip.so not built")
 def test_one_split_runs_one_kernel_under_every_epilogue():
     """Past 32 rows cir_qgemm at one split, the fused SwiGLU and the greedy head run the same kernel, so their results are
     each other's bit for bit (the m <= 32 and the large-m kernel may sum the quads in different orders)."""

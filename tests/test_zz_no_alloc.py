@@ -72,3 +72,20 @@ def test_noalloc_attention_rejects_sizes_beyond_its_scratch(device):
     small = kernels.paged_decode_attention_noalloc(q, kp, kp, pt[:, :4].contiguous(), lens)
     torch.cuda.synchronize()
     assert torch.isfinite(small).all()
+
+
+def test_noalloc_attention_takes_any_batch_at_one_chunk(device):
+    """One chunk of context on the generic path leaves no partials: 2048 rows of 32 heads, whose partials would not have
+    fitted the scratch, give the bits of the workspace entry point."""
+    from cacheir_amd import kernels
+
+    rng = np.random.default_rng(5)
+    batch, hq, hkv, d, psize = 2048, 32, 8, 128, 16
+    kp, vp, pt, lens = (torch.from_numpy(a).to(device)
+                        for a in paged.build_pool(rng, [128, 1, 17, 100], hkv, d, psize, dtype=np.float32))
+    rows = torch.arange(batch, device=device) % 4
+    pt, lens = pt[rows].contiguous(), lens[rows].contiguous()
+    assert pt.shape[1] == 8
+    q = torch.randn((batch, hq, d), device=device)
+    assert torch.equal(kernels.paged_decode_attention_noalloc(q, kp, vp, pt, lens),
+                       kernels.paged_decode_attention(q, kp, vp, pt, lens))
