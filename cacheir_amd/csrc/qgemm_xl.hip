@@ -401,14 +401,16 @@ int launch_xl(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd, floa
     else go.template operator()<4, 2, 8>(groups);
     return 4 * groups;
   }
-  const int runs = xl_runs(np, splits);
-  auto by_rows = [&]<int W>() {
-    if (M <= 64) go.template operator()<4, 2, W>(runs);
-    else if (M <= 96) go.template operator()<6, 2, W>(runs);
-    else go.template operator()<8, 2, W>(runs);
-  };
-  if (np <= 4 * runs) by_rows.template operator()<8>();
-  else by_rows.template operator()<10>();
+  if constexpr (EPI != 2) {
+    const int runs = xl_runs(np, splits);
+    auto by_rows = [&]<int W>() {
+      if (M <= 64) go.template operator()<4, 2, W>(runs);
+      else if (M <= 96) go.template operator()<6, 2, W>(runs);
+      else go.template operator()<8, 2, W>(runs);
+    };
+    if (np <= 4 * runs) by_rows.template operator()<8>();
+    else by_rows.template operator()<10>();
+  }
   return 0;
 }
 
