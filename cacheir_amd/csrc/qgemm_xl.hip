@@ -368,22 +368,25 @@ __global__ __launch_bounds__(64 * W, 2) void qgemm_xl_kernel(const f16* __restri
   }
 }
 
-// Column runs of a one-row-block launch with `splits` k-splits: as many as keep it at one round of workgroups over the
-// 256 CUs, at most one pair each and never more than 5 pairs.
-int xl_runs(int np, int splits) {
-  const int need = (np + 4) / 5;
-  const int round = kCUs / splits < np ? kCUs / splits : np;
-  return need > round ? need : round;
-}
-
 // The geometry of a launch (us measured on MI355X):
-//   * one block of 64, 96 or 128 rows (m <= 128): two wavefronts per pair (H = 2), the columns in runs of at most 5 pairs
-//     over one round of workgroups; 10 wavefronts where a run holds 5 (a fifth pair split over 8 took 10 us more at
-//     Q8_0 gate|up 37888 x 3584, m = 128).  96-row blocks: Q4_0 gate|up 28672 x 4096 at m = 77 37.6 against 46.3.
-//   * more rows in a grid of at most one workgroup per CU: the same, in runs of 4 pairs.
-//   * a larger grid: four wavefronts per workgroup, each a pair over all 128 rows (H = 1), two workgroups per CU: a
-//     converted fragment feeds 8 MFMAs instead of 4 (Q4_0 gate|up at m = 2048 522 against 620, int4 rows 443 against
-//     510; while at m = 512 the 192 workgroups of Q4_0 QKV 6144 x 4096 take 44.6 with eight wavefronts, 50.6 with four).
+//   * one block of 64, 96 or 128 rows (m <= 128) whose columns one round of workgroups over the 256 CUs holds in runs of
+//     at most 5 pairs: such runs, as many as there are CUs (at most one pair each), two wavefronts per pair (H = 2); 10
+//     wavefronts where a run holds 5 (a fifth pair split over 8 took 10 us more at Q8_0 gate|up 37888 x 3584, m = 128).
+//     96-row blocks: Q4_0 gate|up 28672 x 4096 at m = 77 37.6 against 46.3.
+//   * more columns (n > 40960 at one split): four wavefronts per workgroup, each a pair over all rows (H = 1), several
+//     workgroups per CU.  A head's logits, 128256 x 4096, with 5 pairs to a workgroup of 10 wavefronts against this: Q4_0
+//     m = 33 156 / 93, 64 172 / 108, 128 262 / 191; Q8_0 177 / 132, 187 / 140, 286 / 216; int4 131 / 80, 143 / 95, 213 / 170;
+//     Q4_0 SwiGLU 45056 x 4096 at 64 73 / 44.  (57344 x 4096 and 151936 x 1024 alike; at 81920, whose last round of runs
+//     is full, 0.75-1.12 times.)  Within one round the runs win: Q4_0 40960 x 4096 at 64 44 against 49.
+//   * more than 128 rows in a grid of at most one workgroup per CU: H = 2 in runs of 4 pairs.
+//   * more rows in a larger grid: H = 1 over 128 rows, two workgroups per CU: a converted fragment feeds 8 MFMAs instead
+//     of 4 (Q4_0 gate|up at m = 2048 522 against 620, int4 rows 443 against 510; while at m = 512 the 192 workgroups of
+//     Q4_0 QKV 6144 x 4096 take 44.6 with eight wavefronts, 50.6 with four).
+//   * the greedy head (EPI 2), in runs of 4 pairs at any m (the candidates' count): H = 1 past 96 rows as above, at 65-96
+//     rows for 8-bit codes past one workgroup per CU, at up to 64 rows past two (Q8_0: one).  H = 2 against H = 1, Q8_0
+//     128256 x 4096 at m = 33 172 / 137, 64 174 / 143, 96 207 / 178, 40960 x 4096 at 64 80 / 65; int8 rows 128256 x 4096 at
+//     64 137 / 130, 96 193 / 163; Q4_0 at 33 113 / 104, 64 116 / 109.  H = 2 stays for 4-bit codes at 65-96 rows (40960 x
+//     4096: Q4_0 72 against 76, int4 62 against 66) and below those counts (Q4_0 28672 x 4096 at 64 39 against 43).
 template <int FMT, int EPI, typename TO>
 int launch_xl(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd, float* part, TO* act, int M, int N, int K,
               int splits, hipStream_t s) {
@@ -393,25 +396,36 @@ int launch_xl(const f16* x, int ldx, const uint8_t* wq, const uint16_t* wd, floa
     const dim3 grid(runs, splits, (M + 16 * MT - 1) / (16 * MT));
     qgemm_xl_kernel<FMT, MT, H, W, EPI, TO><<<grid, 64 * W, 0, s>>>(x, ldx, wq, wd, part, act, M, N, K, nq);
   };
-  if (M > 128 || EPI == 2) {
-    const bool fill = (long)groups * splits * ((M + 127) / 128) > kCUs;
+  const bool fill = (long)groups * splits * ((M + 127) / 128) > kCUs;
+  if constexpr (EPI == 2) {
+    constexpr bool k8 = layout_fmt(FMT) == CIR_Q8_0;
     if (M > 96 && fill) go.template operator()<8, 1, 4>(groups);
     else if (M > 96) go.template operator()<8, 2, 8>(groups);
-    else if (M > 64) go.template operator()<6, 2, 8>(groups);
+    else if (M > 64) {
+      if constexpr (k8) {
+        if (fill) go.template operator()<6, 1, 4>(groups);
+      }
+      if (!k8 || !fill) go.template operator()<6, 2, 8>(groups);
+    } else if (groups > (FMT == CIR_Q8_0 ? 1 : 2) * kCUs) go.template operator()<4, 1, 4>(groups);
     else go.template operator()<4, 2, 8>(groups);
     return 4 * groups;
-  }
-  if constexpr (EPI != 2) {
-    const int runs = xl_runs(np, splits);
-    auto by_rows = [&]<int W>() {
-      if (M <= 64) go.template operator()<4, 2, W>(runs);
-      else if (M <= 96) go.template operator()<6, 2, W>(runs);
-      else go.template operator()<8, 2, W>(runs);
+  } else {
+    if (M > 128) {
+      if (fill) go.template operator()<8, 1, 4>(groups);
+      else go.template operator()<8, 2, 8>(groups);
+      return 0;
+    }
+    const int runs = kCUs / splits < np ? kCUs / splits : np;  // one round, at most one pair each
+    auto by_rows = [&]<int H, int W>(int n_runs) {
+      if (M <= 64) go.template operator()<4, H, W>(n_runs);
+      else if (M <= 96) go.template operator()<6, H, W>(n_runs);
+      else go.template operator()<8, H, W>(n_runs);
     };
-    if (np <= 4 * runs) by_rows.template operator()<8>();
-    else by_rows.template operator()<10>();
+    if (np <= 4 * runs) by_rows.template operator()<2, 8>(runs);
+    else if (np <= 5 * runs) by_rows.template operator()<2, 10>(runs);
+    else by_rows.template operator()<1, 4>(groups);
+    return 0;
   }
-  return 0;
 }
 
 }  // namespace

@@ -530,11 +530,11 @@ def test_qgemm_large_m_ragged_splits(device, fmt, m, n, k, splits):
 
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
 def test_qgemm_large_m_multi_round_matches_one_round(device, fmt):
-    """Launches of more workgroups than CUs (1100 rows: 36 column groups x 9 row blocks = 324 workgroups) take the
-    large-m kernel's plain-FMA scaling form; 512-row slices of the same inputs at one split (144 workgroups, one
-    round: the default form, for Q8_0 partials the interleave-hinted one) must give the same bits, for the partials
-    and for the fused SwiGLU.  At 4 splits both launches are multi-round: the slices check the row blocks (the last
-    one partly filled).  The partials' sum also within the fp16 bound of the oracle."""
+    """Launches of more workgroups than CUs (1100 rows: 36 column groups x 9 row blocks = 324 workgroups) run four
+    wavefronts per workgroup, each over all 128 rows of its pair; 512-row slices of the same inputs at one split (144
+    workgroups) run eight, half the rows each, and must give the same bits, for the partials and for the fused SwiGLU.
+    At 4 splits both launches are multi-round: the slices check the row blocks (the last one partly filled).  The
+    partials' sum also within the fp16 bound of the oracle."""
     from cacheir_amd import hip, kernels
 
     rng = np.random.default_rng(1100 if fmt == "q4_0" else 1101)
@@ -667,6 +667,10 @@ def test_qgemm_planner_random_shapes_row_formats(device, seed):
     (129, 4500, 896, 2),     # two row blocks, one workgroup per CU: 8 wavefronts, seven quads in four and three
     (300, 18000, 768, 1),    # past one workgroup per CU: four wavefronts over all 128 rows, six quads
     (520, 8192, 2048, 4),    # the same over k-splits of four quads
+    (33, 41003, 256, 1),     # more columns than one round of runs holds: four wavefronts, 64-row blocks
+    (64, 66000, 384, 1),     # the same in the greedy head, past two workgroups per CU
+    (96, 41003, 384, 2),     # 96-row blocks
+    (128, 41003, 128, 1),    # 128-row blocks, one quad
 ])
 def test_qgemm_large_m_geometries(device, fmt, m, n, k, splits):
     """Every launch geometry of the large-m kernel, at the edges of its row blocks, column runs and quad pipeline, each
@@ -1128,11 +1132,12 @@ def test_one_split_epilogues_agree_bitwise(device, fmt, m, inter, k):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("fmt", ["q4_0", "q8_0"])
-@pytest.mark.parametrize("m,inter", [(40, 17600), (128, 17600), (100, 5008), (128, 2304), (130, 17600)])
+@pytest.mark.parametrize("m,inter", [(40, 17600), (128, 17600), (100, 5008), (128, 2304), (130, 17600), (40, 20512),
+                                     (77, 20512), (128, 20512)])
 def test_qgemm_swiglu_large_m_column_runs(device, fmt, m, inter):
     """The fused SwiGLU at m > 32 over intermediate sizes that give each workgroup 4-5 gate/up pairs (17600: 1100
     pairs over 256 workgroups), 1-2 pairs (5008) and one (2304), with 64- and 128-row blocks and a second, partly
-    filled row block at m = 130: bitwise equal to the partials of cir_qgemm (splits 1) + cir_epilogue_swiglu, and
+    filled row block at m = 130, and groups of four pairs where one round of five does not hold them (20512): bitwise equal to the partials of cir_qgemm (splits 1) + cir_epilogue_swiglu, and
     within the fp16 bound of the fp64 oracle on a sample of columns."""
     from cacheir_amd import kernels
 
