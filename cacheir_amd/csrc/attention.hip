@@ -1144,18 +1144,25 @@ int device_cus() {
 }
 
 // Prefill launch: wavefronts on query tiles x wavefronts sharing their context, tiles per (sequence, KV head) and
-// context splits.  Measured on MI355X, us per launch (32/8 heads unless said):
-//   * up to kPfSplitTokens of context a workgroup walks few stages and its start and merge dominate: four wavefronts,
-//     two workgroups per CU, no merge (8 x 512 tokens 39.7 against 51.2 with 8 wavefronts, 5 x 301 at 28/4 15.1
-//     against 20.4).  The choice looks at the sequence alone there, so a batch gives the bits of its sequences
-//     launched one by one.
+// context splits.  All of it follows from the batch, the table's width and the CUs, so past kPfSplitTokens of table the
+// bits of a row may differ between batches and between table widths; up to there the sequence's own sizes decide, and a
+// batch gives the bits of its sequences launched one by one.  Measured on MI355X, us per launch (32/8 heads unless said):
+//   * up to kPfSplitTokens of table a workgroup walks few stages and its start and merge dominate: four wavefronts, two
+//     workgroups per CU, in one context group (8 x 512 tokens 39.7 against 51.2 with 8 wavefronts, 5 x 301 at 28/4 15.1
+//     against 20.4), or in two groups on 64-vector tiles where a sequence has no more vectors (<2,2,1> against <2,4,1>,
+//     whose 128 KiB of LDS leave one workgroup per CU: 64 x 4 tokens after 100 7.8 / 13.8, after 500 24.2 / 31.2, 128 x 2
+//     after 900 82.7 / 99.3; in a grid of at most one workgroup per CU 1 x 2 after 500 11.6 / 11.2, after 900 18.0 / 16.4).
 //   * longer contexts: 8 wavefronts in two context groups (2 x 509 tokens after 3500 at 28/4: 78.6 against 94.8 with
 //     four wavefronts in one group); four in one group again once the grid keeps every CU's two workgroups busy for more than one round
 //     (2 x 2048 tokens: 89.0 against 98.3); 64-vector tiles in four context groups where 128-vector tiles leave half
-//     of the CUs idle (4 x 400 tokens after 1000 at 8/8: 23.5 against 28.9, 100 after 3000: 24.3 against 28.5).
+//     of the CUs idle (4 x 400 tokens after 1000 at 8/8: 23.5 against 28.9, 100 after 3000: 24.3 against 28.5), in two
+//     where the splits share out the context or the grid exceeds the CUs (64 x 4 after 1500 66 / 72, after 4000 180 / 187;
+//     split 16 x 5 after 1500 22.9 / 24.4; unsplit 1 x 2 after 1500 25.9 / 21.9).
 //   * a grid below one workgroup per CU splits long contexts, by the table's capacity, into pieces of about
 //     kPfSplitTokens / 2 (of that capacity: a context that fills half its table is cut twice as fine), if the caller
-//     gave a workspace for the partials (may_split).
+//     gave a workspace for the partials (may_split).  The host does not see the lengths, so a short context in a wide
+//     table pays the merge launch for nothing: 1 x 5 tokens in a table of 2048, split against unsplit, after 100 10.5 /
+//     7.7, after 600 11.7 / 12.6, after 1500 13.2 / 22.1.
 struct PrefillPlan {
   int vec_waves, ctx_waves, tiles, splits;
 };
@@ -1167,9 +1174,10 @@ PrefillPlan prefill_plan(int batch, int q_len, int Hkv, int G, int max_ctx, bool
   const bool longctx = max_ctx > kPfSplitTokens;
   PrefillPlan p;
   p.vec_waves = (nvec <= 2 * kPfVec || (longctx && 2 * groups4 <= cus)) ? 2 : 4;
-  p.ctx_waves = p.vec_waves == 2 ? 4 : (longctx && groups4 < 3 * cus) ? 2 : 1;
   p.tiles = (nvec + kPfVec * p.vec_waves - 1) / (kPfVec * p.vec_waves);
   p.splits = longctx && may_split ? (int)max(1L, min(2L * max_ctx / kPfSplitTokens, cus / (p.tiles * seqs))) : 1;
+  if (p.vec_waves == 2) p.ctx_waves = longctx && p.splits == 1 && p.tiles * seqs <= cus ? 4 : 2;
+  else p.ctx_waves = longctx && groups4 < 3 * cus ? 2 : 1;
   return p;
 }
 
@@ -1215,9 +1223,9 @@ int launch_attention(const void* q, const void* k_pool, const void* v_pool, cons
   dim3 grid(S, Hkv, rows);
   if (prefill) {  // query tiles over each sequence's blocks
     const dim3 pgrid(Hkv * batch, pl.tiles, pl.splits);
-    const auto kernel = pl.ctx_waves == 4   ? attn_prefill_f16_d128<2, 4, 1>
-                        : pl.ctx_waves == 2 ? attn_prefill_f16_d128<4, 2, 2>
-                                            : attn_prefill_f16_d128<4, 1, 2>;
+    const auto kernel = pl.vec_waves == 2
+                            ? (pl.ctx_waves == 4 ? attn_prefill_f16_d128<2, 4, 1> : attn_prefill_f16_d128<2, 2, 1>)
+                            : (pl.ctx_waves == 2 ? attn_prefill_f16_d128<4, 2, 2> : attn_prefill_f16_d128<4, 1, 2>);
     part_ml = part_o + (size_t)rows * Hq * pl.splits * D;
     kernel<<<pgrid, 64 * pl.vec_waves * pl.ctx_waves, 0, s>>>(
         static_cast<const f16*>(q), static_cast<const f16*>(k_pool), static_cast<const f16*>(v_pool), page_table,

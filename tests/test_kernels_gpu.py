@@ -208,6 +208,9 @@ def test_prefill_attention_fp16_random_shapes(device, seed):
     (6, 8, 8, 257, 800, None),     # a grid past three workgroups per CU: 4 wavefronts over a long context
     (2, 3, 2, 50, 40, -0.1),       # a negative scale (folded into q's sign)
     (1, 1, 1, 65, 0, 0.0),         # a zero scale: uniform weights over the visible tokens
+    (70, 4, 4, 4, 20, None),       # 64-vector tiles in two context groups past one workgroup per CU
+    (70, 4, 4, 4, 140, None),      # the same with a table of more than 1024 tokens
+    (20, 4, 8, 4, 800, None),      # in four context groups: unsplit, at most one workgroup per CU
 ])
 def test_prefill_attention_geometries(device, batch, g, hkv, q_len, past, scale):
     """Each launch geometry of the fp16 prefill kernel against the oracle, at sizes whose tiles, stages and splits end
@@ -230,46 +233,45 @@ def test_prefill_attention_geometries(device, batch, g, hkv, q_len, past, scale)
         close16(out[b * q_len:(b + 1) * q_len], ref)
 
 
-@pytest.mark.parametrize("q_len,batch", [(600, 14), (590, 14), (512, 16), (600, 10)])
-def test_prefill_attention_paired_tiles(device, q_len, batch):
-    """A prefill grid of at least two workgroups per CU runs tile pairs (tiles - 1 - x, then x) in one workgroup:
-    an even and an odd tile count (600 / 590 tokens x 8 query heads over 1 KV head: 38 / 37 tiles of 128 query
-    vectors, the odd one with a middle tile run once; 266 paired workgroups, 2 K/V blocks per LDS buffer), and 16
-    sequences of 32 tiles (256 paired workgroups, at most one per CU: 4 blocks per buffer), after 0-300 tokens of
-    context.  The batch agrees with the oracle, and bit for bit with each sequence launched alone (unpaired, one
-    workgroup per CU at most: 4 blocks per buffer).  10 sequences of 38 tiles (380 workgroups) run unpaired with
-    2 blocks per buffer, against the same checks."""
-    from cacheir_amd import kernels
+@pytest.mark.parametrize("q_len,batch,hkv,past,pages,same", [
+    (600, 14, 1, 300, 57, True),    # 128-vector tiles in one context group: 532 workgroups, 38 alone
+    (590, 10, 1, 300, 56, True),    # a ragged last tile
+    (512, 16, 1, 300, 64, True),    # a table of 1024 tokens, the widest that the batch does not decide about
+    (5, 80, 4, 700, 45, True),      # 64-vector tiles in two context groups: 320 workgroups, 4 alone
+    (5, 80, 4, 700, 65, False),     # a wider table: the batch unsplit, a sequence alone over context splits
+    (140, 12, 2, 1100, 78, False),  # the batch in two context groups over 128-vector tiles, alone 64-vector tiles
+])
+def test_prefill_attention_batch_agrees_with_sequences_alone(device, q_len, batch, hkv, past, pages, same):
+    """A batch of prompts (8 query heads per KV head, ragged context before the new tokens) against the oracle and against
+    each sequence launched alone: bit for bit with a table of up to 1024 tokens, where the sequence's own sizes pick the
+    launch form, within the fp16 storage bound with a wider one, where the forms differ."""
+    from cacheir_amd import hip, kernels
 
     rng = np.random.default_rng(q_len)
-    hkv, g = 1, 8
+    g = 8
     hq = g * hkv
-    tiles = -(-q_len * g // 128)
-    cus = torch.cuda.get_device_properties(0).multi_processor_count
-    one_tile = tiles * hkv * batch
-    paired = one_tile >= 2 * cus
-    assert paired == (batch != 10)
-    workgroups = (tiles + 1) // 2 * hkv * batch if paired else one_tile
-    assert (workgroups <= cus) == (q_len == 512)  # 4 K/V blocks per LDS buffer
-    past = rng.integers(0, 301, batch)
-    total = past + q_len
+    assert same == (pages * 16 <= 1024)
+    alone_bytes, batch_bytes = (hip.size_call("cir_paged_prefill_split_bytes", n, q_len, hq, hkv, 128, 16, pages,
+                                              hip.CIR_F16) for n in (1, batch))
+    assert batch_bytes == 0 and (alone_bytes == 0) == same
+    total = rng.integers(0, past + 1, batch) + q_len
     kp, vp, pt, lens = paged.build_pool(rng, total, hkv, 128, 16)
+    assert pt.shape[1] <= pages
+    pt = np.pad(pt, ((0, 0), (0, pages - pt.shape[1])))
     q = rng.standard_normal((batch * q_len, hq, 128)).astype(np.float16)
     kpd, vpd, ptd = to_dev(kp, device), to_dev(vp, device), to_dev(pt, device)
     out = kernels.paged_prefill_attention(to_dev(q, device), kpd, vpd, ptd, to_dev(lens, device), q_len,
                                           check_tables=True)
     for b in range(batch):
-        alone = kernels.paged_prefill_attention(to_dev(q[b * q_len:(b + 1) * q_len], device), kpd, vpd,
-                                                ptd[b:b + 1].contiguous(), to_dev(lens[b:b + 1], device), q_len,
-                                                check_tables=True)
-        assert torch.equal(alone, out[b * q_len:(b + 1) * q_len]), f"sequence {b}"
-    out = out.float().cpu().numpy()
-    for b in range(batch):
+        rows = slice(b * q_len, (b + 1) * q_len)
+        alone = kernels.paged_prefill_attention(to_dev(q[rows], device), kpd, vpd, ptd[b:b + 1].contiguous(),
+                                                to_dev(lens[b:b + 1], device), q_len, check_tables=True)
+        assert not same or torch.equal(alone, out[rows]), f"sequence {b}"
         kh = paged.gather_sequence(kp, pt[b], int(total[b])).astype(np.float32)[None]
         vh = paged.gather_sequence(vp, pt[b], int(total[b])).astype(np.float32)[None]
-        qh = q[b * q_len:(b + 1) * q_len].astype(np.float32)[None]
-        ref = ops.attention(qh, kh, vh, hq, hkv, 128, causal=True).reshape(q_len, hq, 128)
-        close16(out[b * q_len:(b + 1) * q_len], ref)
+        ref = ops.attention(q[rows].astype(np.float32)[None], kh, vh, hq, hkv, 128, causal=True).reshape(q_len, hq, 128)
+        close16(out[rows].float().cpu().numpy(), ref)
+        close16(alone.float().cpu().numpy(), ref)
 
 
 @pytest.mark.parametrize("batch,g,hkv,q_len,past", [
@@ -836,7 +838,7 @@ def test_gemm_f32_rows_do_not_depend_on_the_batch(device, n, k):
 
 
 @pytest.mark.parametrize("d,g,psize,dtype,past,q_len", [
-    (64, 2, 16, np.float32, 0, 1),     # one token: one chunk, three idle wavefronts
+    (64, 2, 16, np.float32, 0, 1),     # one token: one chunk, written out directly by one of the four wavefronts
     (64, 5, 16, np.float32, 127, 2),   # a second chunk of one token; five query heads (two passes of heads)
     (128, 3, 5, np.float32, 200, 3),   # 32 lanes per token, pages that no tile divides
     (256, 1, 16, np.float16, 90, 2),   # 64 lanes per token
