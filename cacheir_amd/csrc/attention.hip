@@ -24,7 +24,7 @@
 //     ds_bpermute shuffles, in fp16 with two heads per dword (l sums the same
 //     rounded values); the four token groups are summed once at the end;
 //   * the 8 wavefronts merge (max, sum, O) through LDS with log-sum-exp weights.
-// Prefill (q_len > 1) on fp16 pools runs attn_prefill_f16_d128 instead: 128 query
+// Prefill (q_len > 1) on fp16 pools runs attn_prefill_f16_d128 instead: 64 or 128 query
 // vectors of a sequence per workgroup over its blocks, both products on MFMA.
 // fp32 pools and other head sizes (tiny-model parity path) use a VALU kernel over
 // 128-token chunks: a context of one chunk is written out directly, more chunks leave
@@ -577,9 +577,11 @@ __global__ __launch_bounds__(64 * kWaves) void attn_f16_d128(
 // balances itself.
 //
 // What bounds it: 32 vectors x 32 tokens cost a wavefront 512 matrix cycles, ~450 VALU
-// cycles of softmax and 16 KiB of LDS reads (128 of the CU's LDS cycles), so at 8
-// wavefronts per CU the three pipes are near balance and the time is what they do not
-// overlap.  The earlier kernel (16 vectors per wavefront: twice the LDS bytes per product;
+// cycles of softmax and 16 KiB of LDS reads (128 of the CU's LDS cycles), and the time is
+// what these do not overlap: by counters (2 x 509 tokens after 3500) the matrix cores are
+// busy 27% of the cycles, VALU 38%, both at once 12%, so half of them nothing issues, with
+// two wavefronts per SIMD between the barriers and 224 workgroups on 256 CUs; no LDS
+// conflicts, K/V read from HBM once.  The earlier kernel (16 vectors per wavefront: twice the LDS bytes per product;
 // V transposed by 2-byte LDS writes) was bound by LDS.  Measured (us, before -> now): 2 x
 // 509 tokens after 3500 (28/4 heads) 178 -> 84, 2048 after 6000 (32/8) 625 -> 271 (870
 // TFLOP/s), a 2048-token prompt 102 -> 57, 8 x 512 tokens 54 -> 41, 10 tokens after 5000

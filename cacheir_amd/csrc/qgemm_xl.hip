@@ -15,14 +15,19 @@
 //     together one every two, and the MFMAs of one run under the FMAs of the other.
 //   * Exact weights and per-block fp32 scales as in the m <= 32 kernel, the quads and blocks of
 //     a split in order, so a split's partials are the same bits at every m > 16.
-// What bounds it: without the loads the arithmetic alone takes 70-90% of the time, and its
-// parts (MFMA, scale FMAs, conversions) add up even where they overlap in the schedule: a loop
-// of MFMAs alone runs at 1.6 GHz and of MFMAs with FMAs at 1.4-2.0 GHz on this card, so the
-// power they draw sets the pace.  Measured (us, before -> now; before: the compiler's order, the
-// row formats' activation sums repeated by every wavefront, fixed 128-column groups): Q4_0
-// 28672 x 4096 + SwiGLU at m = 77 59.4 -> 39.2, 128 61.1 -> 47.5, 2048 533 -> 519 (927
-// TFLOP/s); Q8_0 37888 x 3584 at 77 66.7 -> 51.8, 128 65.7 -> 60.7, 2048 705 -> 674; int4 rows
-// 28672 x 4096 at 77 39.8 -> 32.9, 2048 741 -> 433; Q4_0 4096 x 14336 at 77 28.6 -> 20.8.
+// What bounds it, by the launches' counters: over many workgroups the issue of VALU and MFMA
+// instructions, which overlap too little (Q4_0 28672 x 4096 + SwiGLU at m = 2048: VALU 70% of
+// the cycles, matrix cores 40%, both at once 15%, so 95% busy; 6.9 VALU instructions an MFMA,
+// most of them the scale FMAs and conversions).  In one round at m <= 128 latency and an uneven
+// share: Q8_0 37888 x 3584 at 128 VALU 48%, matrix cores 22%, both 8%, neither 38%; the L1
+// refuses requests 31% of the cycles, HBM gives each byte once (152 MB in 62 us), and of ten
+// wavefronts two SIMDs hold three and two hold two.  Measured against the kernels before (us;
+// the compiler's order, the row formats' activation sums repeated by every wavefront, fixed
+// 128-column groups or runs on four wavefronts; the builds timed in turn): Q4_0 28672 x 4096 +
+// SwiGLU at m = 77 65.4 -> 40.5, 128 64.7 -> 48.6, 2048 540-548 -> 545-548 (882 TFLOP/s); Q8_0
+// 37888 x 3584 at 77 67.4 -> 49.7, 128 66.9 -> 58.1, 2048 715-729 -> 692-704; int4 rows
+// 28672 x 4096 at 77 40.1 -> 31.4, 2048 804 -> 459-469; Q4_0 4096 x 14336 and store at 77 32.7
+// -> 24.3.
 // EPI 0: fp32 split-k partials part[split][m][n]; EPI 1: SwiGLU over interleaved gate/up tiles
 // (one split), out[m][N/2] in type TO; EPI 2: greedy-head candidates (one split), the best
 // column of each pair and row: value in part, index in act (as int), at [m][run * W/H + pair].

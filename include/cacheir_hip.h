@@ -128,7 +128,10 @@ int cir_paged_decode_attention_qkv_parts(const float* qkv_partial, int splits, c
  * (b, s) attends to tokens t < seq_lens[b] - q_len + s + 1, where seq_lens[b] is the
  * length after the q_len new tokens were appended.  On the fp16 head_dim-128 path
  * (q_len > 1) the workspace is checked but not written: up to 128 query vectors of a
- * sequence share each K/V block read and the output is written directly. */
+ * sequence share each K/V block read and the output is written directly.  With tables of
+ * up to 1024 tokens (max_pages * page_size) a sequence's rows have the same bits in every
+ * batch; with wider ones the launch form depends on batch and max_pages, and rows may
+ * differ in their last bits between batches or table widths. */
 int cir_paged_prefill_attention(const void* q, const void* k_pool, const void* v_pool,
                                 const int32_t* page_table, const int32_t* seq_lens, void* out,
                                 void* workspace, size_t workspace_bytes,
@@ -141,7 +144,9 @@ int cir_paged_prefill_attention(const void* q, const void* k_pool, const void* v
  * cir_paged_prefill_split_bytes(...) bytes on the fp16 head_dim-128 path (q_len > 1; 0: no
  * splits at these sizes, and it may be NULL), elsewhere
  * cir_paged_attention_workspace_bytes(batch * q_len, ...), where split_bytes is 0.  At 5
- * tokens after 5000 (28 / 4 heads) 18 us against 59 unsplit. */
+ * tokens after 5000 (28 / 4 heads) 18 us against 59 unsplit; a table of more than 1024
+ * tokens whose sequences hold a few hundred pays the merge launch for nothing (5 tokens
+ * after 100, 32 / 8 heads: 10.5 against 7.7), so size the table to its sequences. */
 size_t cir_paged_prefill_split_bytes(int batch, int q_len, int num_heads, int num_kv_heads, int head_dim,
                                      int page_size, int max_pages, int kv_dtype);
 int cir_paged_prefill_attention_split(const void* q, const void* k_pool, const void* v_pool,
@@ -178,8 +183,9 @@ int cir_dequant(const void* weights, int tiled, int fmt, float* out, int n, int 
 
 /* The k-split cir_qgemm is tuned for at this shape: enough workgroups to fill the GPU,
  * no more partials than that needs (for m <= 8, the split under which the GEMV gives
- * every CU the same share of the weights; on the large-m GEMM, one round of workgroups
- * over the CUs, which need not divide k/128).
+ * every CU the same share of the weights; on the large-m GEMM up to 128 rows, as many as
+ * keep one round of workgroups over the CUs, past that the least estimate over 1 .. 16,
+ * of one or several rounds; these need not divide k/128).
  * 0 for an invalid shape.  (The reference has no k-split; this replaces its GEMM plan choice,
  * cacheir/runtime/cuda.py:956-974 _select_gemm_plan.) */
 int cir_qgemm_splits(int m, int n, int k);
