@@ -146,14 +146,15 @@ def paged_prefill_attention(q, k_pool, v_pool, page_table, seq_lens, q_len: int,
     if workspace is None:
         workspace = attention_workspace(rows, num_heads, head_dim, max_pages * psize, q.device)
         own_workspace = True
-    need = hip.size_call("cir_paged_prefill_split_bytes", batch, q_len, num_heads, kvh, head_dim, psize, max_pages, code)
-    name = "cir_paged_prefill_attention"
-    if need:
-        if not own_workspace:
+    name = "cir_paged_prefill_attention_split"  # (it takes any sizes, and the advertised workspace holds its partials)
+    if not own_workspace:
+        need = hip.size_call("cir_paged_prefill_split_bytes", batch, q_len, num_heads, kvh, head_dim, psize, max_pages, code)
+        if need:
             _req(workspace.numel() >= hip.size_call("cir_paged_attention_workspace_bytes", rows, num_heads, head_dim,
                                                     max_pages * psize), "attention: workspace too small", RuntimeError)
             workspace = torch.empty(need, dtype=torch.uint8, device=q.device)
-        name = "cir_paged_prefill_attention_split"
+        else:
+            name = "cir_paged_prefill_attention"
     scale = 1.0 / math.sqrt(head_dim) if scale is None else scale
     hip.call(name, q.data_ptr(), k_pool.data_ptr(), v_pool.data_ptr(), page_table.data_ptr(), seq_lens.data_ptr(),
              out.data_ptr(), workspace.data_ptr(), workspace.numel(), batch, q_len, num_heads, kvh, head_dim, psize,
