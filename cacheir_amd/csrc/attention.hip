@@ -1146,20 +1146,20 @@ int device_cus() {
 }
 
 // Prefill launch: wavefronts on query tiles x wavefronts sharing their context, tiles per (sequence, KV head) and
-// context splits.  All of it follows from the batch, the table's width and the CUs, so past kPfSplitTokens of table the
-// bits of a row may differ between batches and between table widths; up to there the sequence's own sizes decide, and a
-// batch gives the bits of its sequences launched one by one.  Measured on MI355X, us per launch (32/8 heads unless said):
+// context splits.  A sequence of more than 64 vectors has the same bits in every batch up to kPfSplitTokens of table; else
+// the batch, the table's width and the CUs decide too, and a row's last bits may differ between batches and widths.
+// Measured on MI355X, us per launch (32/8 heads unless said):
 //   * up to kPfSplitTokens of table a workgroup walks few stages and its start and merge dominate: four wavefronts, two
-//     workgroups per CU, in one context group (8 x 512 tokens 39.7 against 51.2 with 8 wavefronts, 5 x 301 at 28/4 15.1
-//     against 20.4), or in two groups on 64-vector tiles where a sequence has no more vectors (<2,2,1> against <2,4,1>,
-//     whose 128 KiB of LDS leave one workgroup per CU: 64 x 4 tokens after 100 7.8 / 13.8, after 500 24.2 / 31.2, 128 x 2
-//     after 900 82.7 / 99.3; in a grid of at most one workgroup per CU 1 x 2 after 500 11.6 / 11.2, after 900 18.0 / 16.4).
+//     workgroups per CU, no merge (8 x 512 tokens 39.7 against 51.2 with 8 wavefronts, 5 x 301 at 28/4 15.1 against 20.4).
 //   * longer contexts: 8 wavefronts in two context groups (2 x 509 tokens after 3500 at 28/4: 78.6 against 94.8 with
 //     four wavefronts in one group); four in one group again once the grid keeps every CU's two workgroups busy for more than one round
 //     (2 x 2048 tokens: 89.0 against 98.3); 64-vector tiles in four context groups where 128-vector tiles leave half
-//     of the CUs idle (4 x 400 tokens after 1000 at 8/8: 23.5 against 28.9, 100 after 3000: 24.3 against 28.5), in two
-//     where the splits share out the context or the grid exceeds the CUs (64 x 4 after 1500 66 / 72, after 4000 180 / 187;
-//     split 16 x 5 after 1500 22.9 / 24.4; unsplit 1 x 2 after 1500 25.9 / 21.9).
+//     of the CUs idle (4 x 400 tokens after 1000 at 8/8: 23.5 against 28.9, 100 after 3000: 24.3 against 28.5).
+//   * a sequence of up to 64 vectors, at any length: four context groups, or two once the grid exceeds the CUs, since the
+//     128 KiB of LDS of four leave one workgroup per CU (64 x 4 tokens after 100 7.8 / 13.8, after 500 24.2 / 31.2, after
+//     1500 66 / 72, 128 x 2 after 900 82.7 / 99.3; in smaller grids 1 x 2 after 900 18.0 / 16.4), or its splits fill
+//     three quarters of them (16 x 5 after 1050 19.3 / 20.7, 8 x 5 after 4500 29.2 / 31.4; on fewer workgroups 3 x 5
+//     after 1500 18.8 / 17.0; with more tiles 8 x 30 after 4500 54.3 / 46.4).
 //   * a grid below one workgroup per CU splits long contexts, by the table's capacity, into pieces of about
 //     kPfSplitTokens / 2 (of that capacity: a context that fills half its table is cut twice as fine), if the caller
 //     gave a workspace for the partials (may_split).  The host does not see the lengths, so a short context in a wide
@@ -1178,7 +1178,8 @@ PrefillPlan prefill_plan(int batch, int q_len, int Hkv, int G, int max_ctx, bool
   p.vec_waves = (nvec <= 2 * kPfVec || (longctx && 2 * groups4 <= cus)) ? 2 : 4;
   p.tiles = (nvec + kPfVec * p.vec_waves - 1) / (kPfVec * p.vec_waves);
   p.splits = longctx && may_split ? (int)max(1L, min(2L * max_ctx / kPfSplitTokens, cus / (p.tiles * seqs))) : 1;
-  if (p.vec_waves == 2) p.ctx_waves = longctx && p.splits == 1 && p.tiles * seqs <= cus ? 4 : 2;
+  const long wgs = p.tiles * seqs * p.splits;
+  if (p.vec_waves == 2) p.ctx_waves = (p.splits > 1 ? p.tiles == 1 && wgs >= 3 * cus / 4 : wgs > cus) ? 2 : 4;
   else p.ctx_waves = longctx && groups4 < 3 * cus ? 2 : 1;
   return p;
 }

@@ -129,9 +129,10 @@ int cir_paged_decode_attention_qkv_parts(const float* qkv_partial, int splits, c
  * length after the q_len new tokens were appended.  On the fp16 head_dim-128 path
  * (q_len > 1) the workspace is checked but not written: up to 128 query vectors of a
  * sequence share each K/V block read and the output is written directly.  With tables of
- * up to 1024 tokens (max_pages * page_size) a sequence's rows have the same bits in every
- * batch; with wider ones the launch form depends on batch and max_pages, and rows may
- * differ in their last bits between batches or table widths. */
+ * up to 1024 tokens (max_pages * page_size) and more than 64 query vectors a sequence
+ * (q_len * num_heads / num_kv_heads) its rows have the same bits in every batch; else the
+ * launch form depends on batch and max_pages, and rows may differ in their last bits
+ * between batches or table widths. */
 int cir_paged_prefill_attention(const void* q, const void* k_pool, const void* v_pool,
                                 const int32_t* page_table, const int32_t* seq_lens, void* out,
                                 void* workspace, size_t workspace_bytes,

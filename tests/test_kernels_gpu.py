@@ -210,6 +210,7 @@ def test_prefill_attention_fp16_random_shapes(device, seed):
     (1, 1, 1, 65, 0, 0.0),         # a zero scale: uniform weights over the visible tokens
     (70, 4, 4, 4, 20, None),       # 64-vector tiles in two context groups past one workgroup per CU
     (70, 4, 4, 4, 140, None),      # the same with a table of more than 1024 tokens
+    (8, 4, 8, 4, 1050, None),      # the same over context splits that fill three quarters of the CUs
     (20, 4, 8, 4, 800, None),      # in four context groups: unsplit, at most one workgroup per CU
 ])
 def test_prefill_attention_geometries(device, batch, g, hkv, q_len, past, scale):
@@ -237,23 +238,25 @@ def test_prefill_attention_geometries(device, batch, g, hkv, q_len, past, scale)
     (600, 14, 1, 300, 57, True),    # 128-vector tiles in one context group: 532 workgroups, 38 alone
     (590, 10, 1, 300, 56, True),    # a ragged last tile
     (512, 16, 1, 300, 64, True),    # a table of 1024 tokens, the widest that the batch does not decide about
-    (5, 80, 4, 700, 45, True),      # 64-vector tiles in two context groups: 320 workgroups, 4 alone
+    (9, 80, 4, 700, 45, True),      # 72 vectors: a mostly empty 128-vector tile
+    (5, 80, 4, 700, 45, False),     # 64-vector tiles: 320 workgroups in two context groups, 4 alone in four
     (5, 80, 4, 700, 65, False),     # a wider table: the batch unsplit, a sequence alone over context splits
+    (5, 60, 4, 700, 65, False),     # the batch unsplit in four context groups: 240 workgroups
     (140, 12, 2, 1100, 78, False),  # the batch in two context groups over 128-vector tiles, alone 64-vector tiles
 ])
 def test_prefill_attention_batch_agrees_with_sequences_alone(device, q_len, batch, hkv, past, pages, same):
     """A batch of prompts (8 query heads per KV head, ragged context before the new tokens) against the oracle and against
-    each sequence launched alone: bit for bit with a table of up to 1024 tokens, where the sequence's own sizes pick the
-    launch form, within the fp16 storage bound with a wider one, where the forms differ."""
+    each sequence launched alone: bit for bit with a table of up to 1024 tokens and more than 64 query vectors, where the
+    sequence's own sizes pick the launch form, within the fp16 storage bound elsewhere, where the forms differ."""
     from cacheir_amd import hip, kernels
 
     rng = np.random.default_rng(q_len)
     g = 8
     hq = g * hkv
-    assert same == (pages * 16 <= 1024)
+    assert same == (pages * 16 <= 1024 and q_len * g > 64)
     alone_bytes, batch_bytes = (hip.size_call("cir_paged_prefill_split_bytes", n, q_len, hq, hkv, 128, 16, pages,
                                               hip.CIR_F16) for n in (1, batch))
-    assert batch_bytes == 0 and (alone_bytes == 0) == same
+    assert batch_bytes == 0 and (alone_bytes == 0) == (pages * 16 <= 1024)
     total = rng.integers(0, past + 1, batch) + q_len
     kp, vp, pt, lens = paged.build_pool(rng, total, hkv, 128, 16)
     assert pt.shape[1] <= pages
